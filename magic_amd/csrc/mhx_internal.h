@@ -40,48 +40,43 @@ bool is_device_ptr(const void *ptr);
     } while (0)
 
 // ----------------------------------------------------- Legendre job model
-// A transform "job" runs one kind of Legendre contraction for a group of
-// radial levels.  B columns are complex coefficient vectors built on the fly
-// from up to two input arrays:
-//     col = i^ipow * m^mpow * (g(l, lev) * x0 + hcoef * x1)
-// with g = 1, l(l+1) or or2[lev] l(l+1).
+// A synthesis job runs one kind of Legendre contraction for a group of radial
+// levels.  Its fields (Q, S, T or x) are formed on the fly from one or two
+// coefficient arrays:
+//     f = (im ? i m : 1) * (g(l, lev) x0 - x1),  g = 1, l(l+1) or or2[lev] l(l+1)
 enum GKind { G_ONE = 0, G_LL = 1, G_OR2LL = 2 };
 
 struct ColOp {
-    int src0;     // index into the job's source list
-    int src1;     // -1 if unused
-    int gkind;
-    int ipow;     // power of i (0..3)
-    int mpow;     // power of m (0..2)
-    double hcoef; // coefficient of x1
-    double scale;
+    const double *x0, *x1;  // coefficient arrays (complex, level stride src_ld); x1 may be null
+    int gkind, im;
 };
 
-// synthesis kinds (see mhx_legendre.hip for the product tables)
+// synthesis kinds: fields and outputs
+//   SCAL x -> x;  GRAD x -> dx/dtheta, dx/dphi;  SG x -> x, dx/dtheta, dx/dphi;
+//   QST Q, S, T -> r, theta, phi components;  SPHTOR S, T -> theta, phi
 enum SynKind { SYN_SCAL = 0, SYN_GRAD = 1, SYN_SG = 2, SYN_QST = 3, SYN_SPHTOR = 4 };
 // analysis kinds
 enum AnaKind { ANA_SH = 0, ANA_SPHTOR = 1, ANA_QST = 2 };
 
-constexpr int MAX_SRC = 4;
-constexpr int MAX_COL = 5;
 constexpr int MAX_OUT = 3;
 constexpr int LEV_GROUP = 8;   // radial levels per MFMA column tile (re/im -> 16)
+constexpr int MAX_SYN_JOBS = 12;  // jobs of one synthesis launch
 
 struct SynJob {
     int kind;
+    ColOp col[3];          // fields in the kind's order
+    double *fout;          // Fourier arrays F[lev][comp][m][theta] complex
+    int out_comp[MAX_OUT]; // comp index of each output
+    int row_scale;         // 1: outputs times 1/sin^2(theta) (dphspat)
+};
+
+// what the jobs of one launch share
+struct SynBatch {
     int nlev;
-    // sources: coefficient arrays (complex, interleaved), level stride ld (complex)
-    const double *src[MAX_SRC];
-    size_t src_ld;
-    ColOp col[MAX_COL];
-    // outputs: Fourier arrays F[lev][comp][m][theta] complex; comp index and
-    // per-level stride (complex elements)
-    double *fout;
-    size_t fout_ld;      // complex elements per level
-    int out_comp[MAX_OUT];
-    int row_scale[MAX_OUT]; // 1: multiply by 1/sin^2(theta) (dphspat)
-    const int *lcut;     // device, per level
-    const double *or2;   // device, per level (may be null)
+    size_t src_ld;         // complex elements per level of the coefficients
+    size_t fout_ld;        // complex elements per level of the Fourier arrays
+    const int *lcut;       // device, per level
+    const double *or2;     // device, per level (may be null)
 };
 
 struct AnaJob {
@@ -245,6 +240,10 @@ struct Plan {
     double *d_syn_P = nullptr, *d_syn_dP = nullptr;   // FP64 MFMA-tiled
     double *d_ana_wP = nullptr, *d_ana_wdP = nullptr;
     size_t *d_syn_off = nullptr, *d_ana_off = nullptr;
+    // the FP64 Legendre kernels' tables: P_lm for l <= l_max + 1, two K quads
+    // per lane, and the factors c_l (ensure_p_tables)
+    double *d_synx = nullptr, *d_crec64 = nullptr;
+    size_t *d_synx_off = nullptr;
     double *d_osin2 = nullptr;      // n_theta (scrambled)
     double *d_theta = nullptr, *d_gauss = nullptr; // nh
     double *d_tw = nullptr;         // M complex: exp(-2 pi i k/M)
@@ -348,7 +347,8 @@ int launch_nsyn16(const Plan *p, int kind, const NSynArgs &args, hipStream_t s);
 int launch_get_td(const Plan *p, const TdArgs &args, hipStream_t s);
 int launch_e_kin(const Plan *p, const EkArgs &args, hipStream_t s);
 int launch_nana16(const Plan *p, int kind, const NAnaArgs &args, hipStream_t s);
-int launch_syn(const Plan *p, const SynJob &job, hipStream_t s);
+// the jobs of one launch (their outputs distinct comps)
+int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, hipStream_t s);
 int launch_ana(const Plan *p, const AnaJob &job, hipStream_t s);
 // Fourier data (complex, m < n_m): inverse side F[lev][comp][m][theta],
 // forward side F2[lev][comp][theta][m]; grids in the reference layout (theta
@@ -444,6 +444,9 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &a, hipStream_t s);
 // recurrence, without FP64 tables
 int table_layout(Plan *p);
 int ensure_fp64_tables(Plan *p);
+// the P-only tables of the FP64 Legendre kernels, built at plan creation for
+// FP64 plans, else by the first call that runs those kernels
+int ensure_p_tables(Plan *p);
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff);
 // the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768
 bool grid_tile_supported(const Plan *p);

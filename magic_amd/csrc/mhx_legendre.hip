@@ -7,19 +7,21 @@
 // coefficients.  With theta rows as GEMM rows, l as K and (8 radial levels x
 // re/im) as 16 GEMM columns this is a dense contraction per m.  The
 // equatorial symmetry of the reference (ES/EA sums, :172-189) is kept: K runs
-// over l of one parity at a time, and two accumulators per output gather
-//     Sym  = sum_{l-m even} P-terms + sum_{l-m odd} dP-terms
-//     Anti = sum_{l-m odd}  P-terms + sum_{l-m even} dP-terms
-// so that north = Sym + Anti and south = Sym - Anti (P is even and sin dP/dth
-// odd under theta -> pi - theta for l - m even).
+// over l of one parity at a time, and two accumulators per column gather
+//     Sym  = sum over l - m even,   Anti = sum over l - m odd
+// so that north = Sym + Anti and south = Sym - Anti (P is even under theta ->
+// pi - theta for l - m even).
+//
+// Only P_lm is contracted: sin(theta) dP_l/dtheta = l c_{l+1} P_{l+1} -
+// (l+1) c_l P_{l-1} (src/plms.f90:142-162) moves every dP product onto P,
+//     sum_l dP_l x_l = sum_l P_l x'_l,  x'_l = (l-1) c_l x_{l-1} - (l+2) c_{l+1} x_{l+1}
+// for l <= l_max + 1, so that a vector field takes three column products
+// (Q, S' + i m T, i m S - T') instead of five.
 //
 // Analysis (src/shtransforms.f90:648-872): rows are l of one parity, K is the
 // northern theta, columns as above; the ES/EA combinations of north/south
 // Fourier rows are formed while staging B, Gauss weights are folded into the
 // tables (wPlm, wdPlm).
-//
-// The factors i m of the vector transforms are folded into the B columns so
-// that every output is a plain sum of MFMA products held in the same lanes.
 #include "mhx_internal.h"
 
 namespace mhx {
@@ -32,28 +34,6 @@ constexpr int CHUNK = 4 * KQC;  // 32 rows of B per parity / per theta chunk
 
 struct Prod {
     int acc, tab, col;  // tab 0: P, 1: dP
-};
-
-template <int KIND> struct SynSpec;
-template <> struct SynSpec<SYN_SCAL> {
-    static constexpr int NOUT = 1, NCOL = 1, NPROD = 1;
-    static constexpr Prod prod[1] = {{0, 0, 0}};
-};
-template <> struct SynSpec<SYN_GRAD> {  // gt = dP.x ; gp = P.(i m x)
-    static constexpr int NOUT = 2, NCOL = 2, NPROD = 2;
-    static constexpr Prod prod[2] = {{0, 1, 0}, {1, 0, 1}};
-};
-template <> struct SynSpec<SYN_SG> {    // s = P.x ; gt = dP.x ; gp = P.(i m x)
-    static constexpr int NOUT = 3, NCOL = 2, NPROD = 3;
-    static constexpr Prod prod[3] = {{0, 0, 0}, {1, 1, 0}, {2, 0, 1}};
-};
-template <> struct SynSpec<SYN_QST> {   // cols: Q, S, i m T, i m S, -T
-    static constexpr int NOUT = 3, NCOL = 5, NPROD = 5;
-    static constexpr Prod prod[5] = {{0, 0, 0}, {1, 1, 1}, {1, 0, 2}, {2, 0, 3}, {2, 1, 4}};
-};
-template <> struct SynSpec<SYN_SPHTOR> {  // cols: S, i m T, i m S, -T
-    static constexpr int NOUT = 2, NCOL = 4, NPROD = 4;
-    static constexpr Prod prod[4] = {{0, 1, 0}, {0, 0, 1}, {1, 0, 2}, {1, 1, 3}};
 };
 
 template <int KIND> struct AnaSpec;
@@ -74,9 +54,14 @@ template <> struct AnaSpec<ANA_QST> {     // cols: f, vt, -i m vp, -vp, -i m vt
 };
 
 struct SynArgs {
-    SynJob job;
-    const double *sP, *sdP;
+    SynJob job[MAX_SYN_JOBS];
+    int njob, nlev, ng, gz;
+    size_t src_ld, fout_ld;
+    const int *lcut;
+    const double *or2;
+    const double *tab;     // P_lm, l <= l_max + 1 (layout: mhx_tables.hip)
     const size_t *off;
+    const double *crec;
     const int *lstart;
     const double *osin2;
     int l_max, minc, n_m, nh, n_theta, nt16;
@@ -126,197 +111,241 @@ __device__ inline void apply_factor(double &re, double &im, int ipow, int mpow, 
 }
 
 // ------------------------------------------------------------- synthesis
-template <int KIND>
-__global__ __launch_bounds__(WG) void k_syn(SynArgs a)
-{
-    using S = SynSpec<KIND>;
-    constexpr int NOUT = S::NOUT, NCOL = S::NCOL, NPROD = S::NPROD;
-    // B chunk: [col][parity][32 kk][16 cols]; reused by the epilogue
-    constexpr int BS_DOUBLES = NCOL * 2 * CHUNK * 16;
-    constexpr int EP_DOUBLES = 4 * LEV_GROUP * 32 * 2;  // per wave: 8 lev x 32 theta x re/im
-    __shared__ double smem[BS_DOUBLES > EP_DOUBLES ? BS_DOUBLES : EP_DOUBLES];
+__device__ inline double2 czero() { return make_double2(0.0, 0.0); }
+__device__ inline double2 cimul(double m, double2 z) { return make_double2(-m * z.y, m * z.x); }  // i m z
 
-    const SynJob &job = a.job;
-    const int lb = xcd_logical(blockIdx.x, gridDim.x);
-    const int mc = lb % a.n_m;
-    const int ng = (job.nlev + LEV_GROUP - 1) / LEV_GROUP;
-    const int gy = (lb / a.n_m) % ng, gz = lb / (a.n_m * ng);
-    const int m = mc * a.minc;
+// B chunk in LDS: 32 consecutive l, [column][parity][pair of quads] blocks of
+// 64 lanes x 2 quads; the blocks are padded so that the eight levels and the
+// chunk's parities and pairs of one store fall on different banks (block
+// strides 8, 16 modulo 32 doubles)
+constexpr int SB_PAIR = 136, SB_PAR = 2 * SB_PAIR, SB_COL = 2 * SB_PAR;
+
+template <int KIND> constexpr int syn_np() { return KIND == SYN_QST ? 3 : (KIND == SYN_SCAL ? 1 : 2); }
+
+// One workgroup: one job, one order m (index mc), 8 radial levels from lev0,
+// theta tiles of 16 rows dealt over the waves of gz workgroups, TPW per wave.
+// Per chunk of 32 degrees a thread owns one (level, l): its coefficients are
+// loaded a chunk ahead (consecutive l of a level by consecutive lanes), formed
+// into the columns with the l -/+ 1 neighbours taken from the adjacent lanes,
+// and written to the other half of the LDS buffer, so that one barrier per
+// chunk is enough; the table fragments (16 bytes per lane: two quads) are
+// loaded one step of 2 NP TPW products ahead.  Loads are unconditional at
+// clamped addresses, the values masked at their use.
+template <int TPW, int KIND>
+__device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, int mc, int lev0, int gz, double *sB)
+{
+    constexpr int NP = syn_np<KIND>();
+    constexpr bool QST = KIND == SYN_QST, TWO = KIND == SYN_QST || KIND == SYN_SPHTOR;
+    constexpr int CS = QST ? 1 : 0, CT = QST ? 2 : 1;  // fields S (or x) and T
+    const int m = mc * a.minc, L = a.l_max;
     const double dm = (double)m;
-    const int lev0 = gy * LEV_GROUP;
-    const int nlev_here = min(LEV_GROUP, job.nlev - lev0);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tt = gz * 4 + wave;
-    const bool active = tt < a.nt16;
-    const int K0 = (a.l_max - m) / 2 + 1, K1 = (a.l_max - m + 1) / 2;
-    const int Kq[2] = {(K0 + 3) / 4, (K1 + 3) / 4};
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int tt0 = gz * 4 + __builtin_amdgcn_readfirstlane(tid >> 6), tstep = 4 * a.gz;
     const int l0 = a.lstart[mc];
 
-    d4 acc[NOUT][2];
+    // the thread's (level, degree) of a chunk
+    const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
+    const int lc = lev < a.nlev ? min(a.lcut[lev], L) : -1;
+    int lcm = -1;  // largest cut-off of the level group
 #pragma unroll
-    for (int o = 0; o < NOUT; ++o)
-        for (int s = 0; s < 2; ++s) acc[o][s] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, min(a.lcut[min(lev0 + i, a.nlev - 1)], L));
+    const int nrow = max(lcm + 2 - m, 0);  // degrees m .. lcm + 1
+    const int nch = (nrow + 31) >> 5;
+    const int nquad[2] = {((nrow + 1) / 2 + 3) >> 2, (nrow / 2 + 3) >> 2};
+    const int levc = min(lev, a.nlev - 1);
+    const double or2 = a.or2 ? a.or2[levc] : 0.0;
+    const size_t src0 = ((size_t)levc * a.src_ld + (size_t)(l0 - m)) * 2;
 
-    // B staging is software-pipelined: the input coefficients of chunk c+1
-    // are loaded into registers while the MFMAs of chunk c run, then built
-    // into columns in LDS.  The table fragments of a chunk are all issued
-    // before its MFMAs.
-    constexpr int NE = (2 * CHUNK * LEV_GROUP) / WG;  // staging entries per thread
-    double pxr[NE][MAX_SRC], pxi[NE][MAX_SRC];
-    double pll[NE];
-    bool pval[NE];
-    auto load_B = [&](int c) {
-#pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            int idx = threadIdx.x + e * WG;
-            int levl = idx % LEV_GROUP;
-            int kkl = (idx / LEV_GROUP) % CHUNK;
-            int par = idx / (LEV_GROUP * CHUNK);
-            int l = m + par + 2 * (c * CHUNK + kkl);
-            int lev = lev0 + levl;
-            bool valid = (levl < nlev_here) && (l <= a.l_max);
-            if (valid) valid = l <= job.lcut[lev];
-            pval[e] = valid;
-            size_t o = ((size_t)lev * job.src_ld + (size_t)(l0 + l - m)) * 2;
-#pragma unroll
-            for (int sidx = 0; sidx < MAX_SRC; ++sidx) {
-                double2 v = make_double2(0.0, 0.0);
-                if (valid && job.src[sidx]) v = *reinterpret_cast<const double2 *>(job.src[sidx] + o);
-                pxr[e][sidx] = v.x;
-                pxi[e][sidx] = v.y;
+    const double *const q0 = job.col[0].x0, *const s0 = job.col[CS].x0;
+    const double *const t0 = job.col[CT].x0, *const t1 = job.col[CT].x1;
+    double2 xq, xs, xt0, xt1, hs, ht0, ht1;  // own degree; the chunk's outer neighbours (lanes 0, 31)
+    auto ld = [&](const double *p, int l) { return *reinterpret_cast<const double2 *>(p + src0 + 2 * (size_t)l); };
+    const int hd = j == 0 ? -1 : 1;
+    auto load = [&](int c) {
+        const int l = m + 32 * c + j;
+        const int li = min(l, L), lh = max(min(l + hd, L), m);
+        if constexpr (QST) xq = ld(q0, li);
+        xs = ld(s0, li);
+        if constexpr (KIND != SYN_SCAL) {
+            if (j == 0 || j == 31) hs = ld(s0, lh);
+        }
+        if constexpr (TWO) {
+            xt0 = ld(t0, li);
+            if (j == 0 || j == 31) ht0 = ld(t0, lh);
+            if (t1) {
+                xt1 = ld(t1, li);
+                if (j == 0 || j == 31) ht1 = ld(t1, lh);
             }
         }
     };
-    auto store_B = [&]() {
-#pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            int idx = threadIdx.x + e * WG;
-            int levl = idx % LEV_GROUP;
-            int kkl = (idx / LEV_GROUP) % CHUNK;
-            int par = idx / (LEV_GROUP * CHUNK);
-            int lev = lev0 + levl;
-#pragma unroll
-            for (int col = 0; col < NCOL; ++col) {
-                double re = 0.0, im = 0.0;
-                if (pval[e]) {
-                    const ColOp &op = job.col[col];
-                    double g = 1.0;
-                    if (op.gkind != G_ONE) {
-                        double ll = pll[e];
-                        g = (op.gkind == G_LL) ? ll : job.or2[lev] * ll;
-                    }
-                    double xr0 = 0.0, xi0 = 0.0, xr1 = 0.0, xi1 = 0.0;
-#pragma unroll
-                    for (int sidx = 0; sidx < MAX_SRC; ++sidx) {
-                        if (op.src0 == sidx) { xr0 = pxr[e][sidx]; xi0 = pxi[e][sidx]; }
-                        if (op.src1 == sidx) { xr1 = pxr[e][sidx]; xi1 = pxi[e][sidx]; }
-                    }
-                    re = g * xr0 + op.hcoef * xr1;
-                    im = g * xi0 + op.hcoef * xi1;
-                    apply_factor(re, im, op.ipow, op.mpow, dm, op.scale);
-                }
-                double *b = smem + (((col * 2 + par) * CHUNK + kkl) * 16 + levl * 2);
-                b[0] = re;
-                b[1] = im;
+    // the field at (level, l), zero outside m <= l <= lcut
+    auto field = [&](const ColOp &op, int l, double2 x0, double2 x1) {
+        const double ll = (double)l * (double)(l + 1);
+        const double g = op.gkind == G_ONE ? 1.0 : (op.gkind == G_LL ? ll : or2 * ll);
+        double2 v = make_double2(g * x0.x, g * x0.y);
+        if (op.x1) v = make_double2(v.x - x1.x, v.y - x1.y);
+        if (op.im) v = cimul(dm, v);
+        const bool ok = l >= m && l <= lc;
+        return make_double2(ok ? v.x : 0.0, ok ? v.y : 0.0);
+    };
+    auto put = [&](int buf, int col, double2 v) {
+        double *b = sB + buf * NP * SB_COL + col * SB_COL + (j & 1) * SB_PAR + (j >> 4) * SB_PAIR +
+                    (((j >> 1) & 3) * 16 + 2 * lv) * 2 + ((j >> 3) & 1);
+        b[0] = v.x;
+        b[2] = v.y;
+    };
+    auto build = [&](int c, int buf) {
+        const int l = m + 32 * c + j;
+        if constexpr (QST) put(buf, 0, field(job.col[0], l, xq, czero()));
+        const double2 s = field(job.col[CS], l, xs, czero());
+        if constexpr (KIND == SYN_SCAL) {
+            put(buf, 0, s);
+        } else {
+            const double *cr = a.crec + l0 + 2 * mc + min(l, L + 1) - m;
+            const double fm = (double)(l - 1) * cr[0], fp = (double)(l + 2) * cr[1];
+            // x' from the neighbours of x
+            auto prime = [&](double2 x, double2 h) {
+                double2 lo = make_double2(__shfl_up(x.x, 1, 32), __shfl_up(x.y, 1, 32));
+                double2 hi = make_double2(__shfl_down(x.x, 1, 32), __shfl_down(x.y, 1, 32));
+                if (j == 0) lo = h;
+                if (j == 31) hi = h;
+                return make_double2(fm * lo.x - fp * hi.x, fm * lo.y - fp * hi.y);
+            };
+            const double2 sp = prime(s, field(job.col[CS], l + hd, hs, czero()));
+            if constexpr (TWO) {
+                const double2 t = field(job.col[CT], l, xt0, xt1);
+                const double2 tp = prime(t, field(job.col[CT], l + hd, ht0, ht1));
+                put(buf, CS, make_double2(sp.x - dm * t.y, sp.y + dm * t.x));       // S' + i m T
+                put(buf, CS + 1, make_double2(-dm * s.y - tp.x, dm * s.x - tp.y));  // i m S - T'
+            } else {
+                put(buf, 0, s);
+                put(buf, 1, sp);
             }
         }
     };
 
-    const int nchunk = (Kq[0] + KQC - 1) / KQC;
-    auto set_ll = [&](int c) {
+    d4 acc[TPW][NP][2];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            int idx = threadIdx.x + e * WG;
-            int kkl = (idx / LEV_GROUP) % CHUNK;
-            int par = idx / (LEV_GROUP * CHUNK);
-            double l = (double)(m + par + 2 * (c * CHUNK + kkl));
-            pll[e] = l * (l + 1.0);
-        }
+    for (int s = 0; s < TPW; ++s)
+#pragma unroll
+        for (int pr = 0; pr < NP; ++pr) acc[s][pr][0] = acc[s][pr][1] = d4{0.0, 0.0, 0.0, 0.0};
+
+    // table fragments of (pair of quads kp, parity); past the last pair the
+    // last one is loaded and not used
+    const double2 *tab[2];
+#pragma unroll
+    for (int par = 0; par < 2; ++par)
+        tab[par] = reinterpret_cast<const double2 *>(a.tab + a.off[2 * mc + par]) + lane;
+    auto load_A = [&](double2 *f, int kp, int par) {
+        const double2 *t = tab[par] + (size_t)max(min(kp, (nquad[par] - 1) >> 1), 0) * (a.nt16 * 64);
+#pragma unroll
+        for (int s = 0; s < TPW; ++s) f[s] = t[min(tt0 + s * tstep, a.nt16 - 1) * 64];
     };
-    load_B(0);
-    set_ll(0);
-    store_B();
-    __syncthreads();
-    const double *tP[2], *tdP[2];
-#pragma unroll
-    for (int par = 0; par < 2; ++par) {
-        tP[par] = a.sP + a.off[2 * mc + par] + (size_t)tt * 64 + lane;
-        tdP[par] = a.sdP + a.off[2 * mc + par] + (size_t)tt * 64 + lane;
+    const bool act = tt0 < a.nt16;
+    double2 fa[2][TPW];
+
+    if (nch > 0) {
+        load(0);
+        if (nquad[0] > 0) load_A(fa[0], 0, 0);
+        build(0, 0);
     }
-    const size_t qstride = (size_t)a.nt16 * 64;
-    for (int c = 0; c < nchunk; ++c) {
-        double aP[2][KQC], adP[2][KQC];
-        int nq[2];
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        const int buf = c & 1;
+        if (c + 1 < nch) load(c + 1);
+        if (act) {
 #pragma unroll
-        for (int par = 0; par < 2; ++par) {
-            nq[par] = min(KQC, Kq[par] - c * KQC);
+            for (int k = 0; k < 4; ++k) {
+                const int par = k & 1, pair = k >> 1;
+                // the next step's fragments
+                if (nquad[1 - par] > 0) load_A(fa[1 - par], 2 * c + ((k + 1) >> 1), 1 - par);
+                const int qq = 4 * c + 2 * pair;  // first quad of this step
+                if (qq < nquad[par]) {
+                    double2 b[NP];
+                    const double *sb = sB + buf * NP * SB_COL + par * SB_PAR + pair * SB_PAIR + 2 * lane;
 #pragma unroll
-            for (int q = 0; q < KQC; ++q) {
-                bool ok = active && q < nq[par];
-                size_t kq = (size_t)(c * KQC + q);
-                aP[par][q] = ok ? tP[par][kq * qstride] : 0.0;
-                adP[par][q] = ok ? tdP[par][kq * qstride] : 0.0;
-            }
-        }
-        if (c + 1 < nchunk) load_B(c + 1);
-        if (active) {
+                    for (int pr = 0; pr < NP; ++pr) b[pr] = *reinterpret_cast<const double2 *>(sb + pr * SB_COL);
 #pragma unroll
-            for (int par = 0; par < 2; ++par)
+                    for (int pr = 0; pr < NP; ++pr)
 #pragma unroll
-                for (int q = 0; q < KQC; ++q) {
-                    if (q >= nq[par]) break;
+                        for (int s = 0; s < TPW; ++s) acc[s][pr][par] = mfma64(fa[par][s].x, b[pr].x, acc[s][pr][par]);
+                    if (qq + 1 < nquad[par]) {
 #pragma unroll
-                    for (int pr = 0; pr < NPROD; ++pr) {
-                        const Prod P = S::prod[pr];
-                        double b = smem[((P.col * 2 + par) * CHUNK + q * 4 + (lane >> 4)) * 16 + (lane & 15)];
-                        // P-table: even parity -> Sym (0); dP-table: even -> Anti (1)
-                        int tgt = (P.tab == 0) ? par : (1 - par);
-                        acc[P.acc][tgt] = mfma64(P.tab == 0 ? aP[par][q] : adP[par][q], b, acc[P.acc][tgt]);
+                        for (int pr = 0; pr < NP; ++pr)
+#pragma unroll
+                            for (int s = 0; s < TPW; ++s)
+                                acc[s][pr][par] = mfma64(fa[par][s].y, b[pr].y, acc[s][pr][par]);
                     }
                 }
+            }
         }
-        __syncthreads();
-        if (c + 1 < nchunk) {
-            set_ll(c + 1);
-            store_B();
-        }
+        if (c + 1 < nch) build(c + 1, buf ^ 1);
         __syncthreads();
     }
 
-    // epilogue: north = Sym + Anti, south = Sym - Anti; transposed through
-    // LDS into contiguous runs of 32 theta rows of F[lev][comp][m][theta]
-    __syncthreads();
-    double *ep = smem + wave * (LEV_GROUP * 32 * 2);
-    const int col = lane & 15, levl_c = col >> 1, ri = col & 1;
+    // epilogue: north = Sym + Anti, south = Sym - Anti; adjacent lanes (re, im)
+    // exchange, so that the even lane stores the northern complex value and
+    // the odd lane the southern one: 128-byte runs of F[lev][comp][m][theta]
+    const int col = lane & 15, elev = lev0 + (col >> 1), odd = col & 1;
+    if (elev >= a.nlev) return;
+    const size_t cstride = (size_t)a.n_m * a.n_theta;
+    double2 *fo = reinterpret_cast<double2 *>(job.fout) + (size_t)elev * a.fout_ld + (size_t)mc * a.n_theta + odd;
 #pragma unroll
-    for (int o = 0; o < NOUT; ++o) {
-        if (active) {
+    for (int s = 0; s < TPW; ++s) {
+        const int tt = tt0 + s * tstep;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                int row = (lane >> 4) + 4 * j;
-                int th = tt * 16 + row;
-                double sc = 1.0;
-                if (job.row_scale[o] && th < a.nh) sc = a.osin2[2 * th];
-                ep[(levl_c * 32 + 2 * row) * 2 + ri] = (acc[o][0][j] + acc[o][1][j]) * sc;
-                ep[(levl_c * 32 + 2 * row + 1) * 2 + ri] = (acc[o][0][j] - acc[o][1][j]) * sc;
-            }
-        }
-        __syncthreads();
-        if (active) {
+        for (int jj = 0; jj < 4; ++jj) {
+            const int th = tt * 16 + (lane >> 4) + 4 * jj;
+            const bool ok = th < a.nh;
+            const double sc = job.row_scale ? a.osin2[2 * min(th, a.nh - 1)] : 1.0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int e = r * 64 + lane;
-                int levl = e >> 5, thl = e & 31;
-                int theta = tt * 32 + thl;
-                if (levl < nlev_here && theta < a.n_theta) {
-                    size_t o2 = ((size_t)(lev0 + levl) * job.fout_ld +
-                                 ((size_t)job.out_comp[o] * a.n_m + mc) * a.n_theta + theta) * 2;
-                    *reinterpret_cast<double2 *>(job.fout + o2) =
-                        make_double2(ep[(levl * 32 + thl) * 2], ep[(levl * 32 + thl) * 2 + 1]);
+            for (int pr = 0; pr < NP; ++pr) {
+                const double n = acc[s][pr][0][jj] + acc[s][pr][1][jj];
+                const double so = acc[s][pr][0][jj] - acc[s][pr][1][jj];
+                const double other = __shfl_xor(odd ? n : so, 1, 64);
+                double2 v = odd ? make_double2(other, so) : make_double2(n, other);
+                if (job.row_scale) v = make_double2(sc * v.x, sc * v.y);
+                auto store = [&](int o, double2 w) {
+                    if (ok) fo[job.out_comp[o] * cstride + 2 * th] = w;
+                };
+                // columns: QST (Q, C1, C2), SPHTOR (C1, C2), SCAL x;
+                // SG, GRAD: x, x' with d/dphi = i m (P x)
+                if constexpr (KIND == SYN_SG) {
+                    store(pr, v);
+                    if (pr == 0) store(2, cimul(dm, v));
+                } else if constexpr (KIND == SYN_GRAD) {
+                    store(1 - pr, pr == 0 ? cimul(dm, v) : v);
+                } else {
+                    store(pr, v);
                 }
             }
         }
-        __syncthreads();
+    }
+}
+
+// the jobs of one launch: kinds of at most NP columns
+template <int TPW, int NP>
+__global__ __launch_bounds__(WG, 2) void k_syn(SynArgs a)
+{
+    __shared__ double sB[2 * NP * SB_COL];
+    // block -> (order, level group, theta group, job): orders dealt to the 8
+    // XCDs (blocks go round-robin over them) from the longest on, all blocks
+    // of one order on one XCD, whose L2 then holds its table slice once, and
+    // the jobs of a level group together, which share coefficients
+    const int inner = a.njob * a.gz * a.ng;
+    const int mc = (int)(blockIdx.x >> 3) / inner * 8 + (int)(blockIdx.x & 7);
+    if (mc >= a.n_m) return;
+    int r = (int)(blockIdx.x >> 3) % inner;
+    const SynJob &job = a.job[r % a.njob];
+    r /= a.njob;
+    const int gz = r % a.gz, lev0 = r / a.gz * LEV_GROUP;
+    switch (job.kind) {
+    case SYN_SCAL: syn_body<TPW, SYN_SCAL>(a, job, mc, lev0, gz, sB); break;
+    case SYN_GRAD: if constexpr (NP > 1) syn_body<TPW, SYN_GRAD>(a, job, mc, lev0, gz, sB); break;
+    case SYN_SG: if constexpr (NP > 1) syn_body<TPW, SYN_SG>(a, job, mc, lev0, gz, sB); break;
+    case SYN_SPHTOR: if constexpr (NP > 1) syn_body<TPW, SYN_SPHTOR>(a, job, mc, lev0, gz, sB); break;
+    case SYN_QST: if constexpr (NP > 2) syn_body<TPW, SYN_QST>(a, job, mc, lev0, gz, sB); break;
+    default: break;
     }
 }
 
@@ -473,17 +502,47 @@ __global__ __launch_bounds__(WG) void k_ana(AnaArgs a)
     }
 }
 
+// theta tiles per wave and theta groups: 12 tiles per workgroup at most
+// (three per wave: 144 accumulator registers of the 256 at two waves per SIMD)
+template <int NP>
+int launch_syn_np(const SynArgs &a, int tpw, unsigned grid, hipStream_t s)
+{
+    switch (tpw) {
+    case 1: k_syn<1, NP><<<grid, WG, 0, s>>>(a); break;
+    case 2: k_syn<2, NP><<<grid, WG, 0, s>>>(a); break;
+    default: k_syn<3, NP><<<grid, WG, 0, s>>>(a); break;
+    }
+    MHX_HIP_CHECK(hipGetLastError());
+    return MHX_OK;
+}
+
 }  // namespace
 
-int launch_syn(const Plan *p, const SynJob &job, hipStream_t s)
+int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, hipStream_t s)
 {
-    if (int rc = ensure_fp64_tables(const_cast<Plan *>(p))) return rc;
-    if (job.nlev <= 0) return MHX_OK;
+    if (b.nlev <= 0 || njob <= 0) return MHX_OK;
+    if (njob > MAX_SYN_JOBS) return fail(MHX_E_INVALID, "too many synthesis jobs in one launch");
+    if (int rc = ensure_p_tables(const_cast<Plan *>(p))) return rc;
     SynArgs a;
-    a.job = job;
-    a.sP = p->d_syn_P;
-    a.sdP = p->d_syn_dP;
-    a.off = p->d_syn_off;
+    int np = 0;
+    for (int i = 0; i < njob; ++i) {
+        a.job[i] = jobs[i];
+        switch (jobs[i].kind) {
+        case SYN_SCAL: np = np < 1 ? 1 : np; break;
+        case SYN_GRAD: case SYN_SG: case SYN_SPHTOR: np = np < 2 ? 2 : np; break;
+        case SYN_QST: np = 3; break;
+        default: return fail(MHX_E_INVALID, "unknown synthesis kind");
+        }
+    }
+    a.njob = njob;
+    a.nlev = b.nlev;
+    a.src_ld = b.src_ld;
+    a.fout_ld = b.fout_ld;
+    a.lcut = b.lcut;
+    a.or2 = b.or2;
+    a.tab = p->d_synx;
+    a.off = p->d_synx_off;
+    a.crec = p->d_crec64;
     a.lstart = p->d_lstart;
     a.osin2 = p->d_osin2;
     a.l_max = p->l_max;
@@ -492,17 +551,15 @@ int launch_syn(const Plan *p, const SynJob &job, hipStream_t s)
     a.nh = p->nh;
     a.n_theta = p->n_theta;
     a.nt16 = p->nt16;
-    dim3 grid((unsigned)(p->n_m * ((job.nlev + LEV_GROUP - 1) / LEV_GROUP) * ((p->nt16 + 3) / 4)));
-    switch (job.kind) {
-    case SYN_SCAL: k_syn<SYN_SCAL><<<grid, WG, 0, s>>>(a); break;
-    case SYN_GRAD: k_syn<SYN_GRAD><<<grid, WG, 0, s>>>(a); break;
-    case SYN_SG: k_syn<SYN_SG><<<grid, WG, 0, s>>>(a); break;
-    case SYN_QST: k_syn<SYN_QST><<<grid, WG, 0, s>>>(a); break;
-    case SYN_SPHTOR: k_syn<SYN_SPHTOR><<<grid, WG, 0, s>>>(a); break;
-    default: return fail(MHX_E_INVALID, "unknown synthesis kind");
+    a.ng = (b.nlev + LEV_GROUP - 1) / LEV_GROUP;
+    a.gz = (p->nt16 + 11) / 12;
+    const int tpw = (p->nt16 + 4 * a.gz - 1) / (4 * a.gz);
+    const unsigned grid = (unsigned)((p->n_m + 7) / 8 * 8 * njob * a.ng * a.gz);
+    switch (np) {
+    case 1: return launch_syn_np<1>(a, tpw, grid, s);
+    case 2: return launch_syn_np<2>(a, tpw, grid, s);
+    default: return launch_syn_np<3>(a, tpw, grid, s);
     }
-    MHX_HIP_CHECK(hipGetLastError());
-    return MHX_OK;
 }
 
 int launch_ana(const Plan *p, const AnaJob &job, hipStream_t s)

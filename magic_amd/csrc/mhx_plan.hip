@@ -147,33 +147,29 @@ const double *stage_in(Plan *p, const double *src, int slot, size_t count_double
     return dst;
 }
 
-ColOp op(int s0, int g = G_ONE, int ipow = 0, int mpow = 0, double scale = 1.0, int s1 = -1,
-         double h = 0.0)
+ColOp op(const double *x0, int g = G_ONE, const double *x1 = nullptr, int im = 0)
 {
-    ColOp c;
-    c.src0 = s0;
-    c.src1 = s1;
-    c.gkind = g;
-    c.ipow = ipow;
-    c.mpow = mpow;
-    c.hcoef = h;
-    c.scale = scale;
-    return c;
+    return ColOp{x0, x1, g, im};
 }
 
-SynJob syn_job(Plan *p, int kind, int nlev, size_t src_ld)
+// a synthesis job into comps comp0, comp0 + 1, ... of ws_F
+SynJob syn_job(Plan *p, int kind, ColOp c0, ColOp c1 = ColOp(), ColOp c2 = ColOp(), int comp0 = 0)
 {
     SynJob j;
     std::memset(&j, 0, sizeof(j));
     j.kind = kind;
-    j.nlev = nlev;
-    j.src_ld = src_ld;
+    j.col[0] = c0;
+    j.col[1] = c1;
+    j.col[2] = c2;
     j.fout = p->ws_F;
-    j.fout_ld = (size_t)18 * p->n_m * p->n_theta;
-    j.lcut = p->d_lcut;
-    j.or2 = p->d_rad;
-    for (int i = 0; i < MAX_OUT; ++i) j.out_comp[i] = i;
+    for (int i = 0; i < MAX_OUT; ++i) j.out_comp[i] = comp0 + i;
     return j;
+}
+
+// levels of the synthesis launches into ws_F (18 comps per level)
+SynBatch syn_batch(Plan *p, int nlev, size_t src_ld)
+{
+    return SynBatch{nlev, src_ld, (size_t)18 * p->n_m * p->n_theta, p->d_lcut, p->d_rad};
 }
 
 // Fourier -> grid for ncomp comps starting at comp0 of ws_F into separate
@@ -238,13 +234,13 @@ int finish_coefs(Plan *p, int n, double *const *out)
 }
 
 // run a one-level synthesis job then inverse FFT of its ncomp outputs into ws_G
-int synth_call(Plan *p, SynJob &j, int ncomp, int lcut, double or2, double *const *out)
+int synth_call(Plan *p, const SynJob &j, int ncomp, int lcut, double or2, double *const *out)
 {
     int rc = check_lcut(p, lcut);
     if (rc) return rc;
     MHX_HIP_CHECK(hipMemcpyAsync(p->d_lcut, &lcut, sizeof(int), hipMemcpyHostToDevice, p->stream));
     MHX_HIP_CHECK(hipMemcpyAsync(p->d_rad, &or2, sizeof(double), hipMemcpyHostToDevice, p->stream));
-    if ((rc = launch_syn(p, j, p->stream))) return rc;
+    if ((rc = launch_syn(p, &j, 1, syn_batch(p, 1, 0), p->stream))) return rc;
     double *dst[3] = {p->ws_G, p->ws_G + (size_t)p->n_phi * p->n_theta,
                       p->ws_G + (size_t)2 * p->n_phi * p->n_theta};
     if ((rc = ifft_to(p, 0, ncomp, 1, dst, 0))) return rc;
@@ -448,6 +444,7 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
     // split kernels generate the tables in-kernel, and the per-call entries
     // that read FP64 tables build them on first use (ensure_fp64_tables)
     if ((rc = (rec && l_max > 255) ? table_layout(p) : build_tables(p)) ||
+        (precision == MHX_PREC_FP64 && (rc = ensure_p_tables(p))) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
         (rc = ensure_ws(p, std::max(1, max_levels)))) {
         mhx_plan_destroy(h);
@@ -482,6 +479,9 @@ int mhx_plan_destroy(mhx_plan *h)
     free_dev(p->d_ana_wP);
     free_dev(p->d_ana_wdP);
     free_dev(p->d_syn_off);
+    free_dev(p->d_synx);
+    free_dev(p->d_synx_off);
+    free_dev(p->d_crec64);
     free_dev(p->d_ana_off);
     free_dev(p->d_osin2);
     free_dev(p->d_theta);
@@ -588,9 +588,7 @@ int mhx_plan_tables(const mhx_plan *h, double *theta_ord, double *gauss, double 
 int mhx_scal_to_spat(mhx_plan *h, const double *Slm, double *fieldc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_SCAL, 1, 0);
-    j.src[0] = stage_in(P, Slm, 0, 2 * P->lm_max);
-    j.col[0] = op(0);
+    SynJob j = syn_job(P, SYN_SCAL, op(stage_in(P, Slm, 0, 2 * P->lm_max)));
     double *out[1] = {fieldc};
     return synth_call(P, j, 1, lcut, 0.0, out);
 }
@@ -598,10 +596,7 @@ int mhx_scal_to_spat(mhx_plan *h, const double *Slm, double *fieldc, int lcut)
 int mhx_scal_to_grad_spat(mhx_plan *h, const double *Slm, double *gradtc, double *gradpc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_GRAD, 1, 0);
-    j.src[0] = stage_in(P, Slm, 0, 2 * P->lm_max);
-    j.col[0] = op(0);
-    j.col[1] = op(0, G_ONE, 1, 1);
+    SynJob j = syn_job(P, SYN_GRAD, op(stage_in(P, Slm, 0, 2 * P->lm_max)));
     double *out[2] = {gradtc, gradpc};
     return synth_call(P, j, 2, lcut, 0.0, out);
 }
@@ -609,58 +604,18 @@ int mhx_scal_to_grad_spat(mhx_plan *h, const double *Slm, double *gradtc, double
 int mhx_pol_to_grad_spat(mhx_plan *h, const double *Slm, double *gradtc, double *gradpc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_GRAD, 1, 0);
-    j.src[0] = stage_in(P, Slm, 0, 2 * P->lm_max);
-    j.col[0] = op(0, G_LL);
-    j.col[1] = op(0, G_LL, 1, 1);
+    SynJob j = syn_job(P, SYN_GRAD, op(stage_in(P, Slm, 0, 2 * P->lm_max), G_LL));
     double *out[2] = {gradtc, gradpc};
     return synth_call(P, j, 2, lcut, 0.0, out);
-}
-
-static void qst_cols(SynJob &j, ColOp Q, ColOp S, ColOp T)
-{
-    // columns Q, S, i m T, i m S, -T (T and S may be built from two sources)
-    j.col[0] = Q;
-    j.col[1] = S;
-    ColOp miT = T;
-    miT.ipow = (miT.ipow + 1) & 3;
-    miT.mpow += 1;
-    ColOp miS = S;
-    miS.ipow = (miS.ipow + 1) & 3;
-    miS.mpow += 1;
-    ColOp mT = T;
-    mT.scale = -mT.scale;
-    j.col[2] = miT;
-    j.col[3] = miS;
-    j.col[4] = mT;
-}
-
-static void sphtor_cols(SynJob &j, ColOp S, ColOp T)
-{
-    // columns S, i m T, i m S, -T
-    ColOp miT = T;
-    miT.ipow = (miT.ipow + 1) & 3;
-    miT.mpow += 1;
-    ColOp miS = S;
-    miS.ipow = (miS.ipow + 1) & 3;
-    miS.mpow += 1;
-    ColOp mT = T;
-    mT.scale = -mT.scale;
-    j.col[0] = S;
-    j.col[1] = miT;
-    j.col[2] = miS;
-    j.col[3] = mT;
 }
 
 int mhx_torpol_to_spat(mhx_plan *h, const double *Wlm, const double *dWlm, const double *Zlm,
                        double *vrc, double *vtc, double *vpc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_QST, 1, 0);
-    j.src[0] = stage_in(P, Wlm, 0, 2 * P->lm_max);
-    j.src[1] = stage_in(P, dWlm, 1, 2 * P->lm_max);
-    j.src[2] = stage_in(P, Zlm, 2, 2 * P->lm_max);
-    qst_cols(j, op(0, G_LL), op(1), op(2));
+    const size_t n = 2 * P->lm_max;
+    SynJob j = syn_job(P, SYN_QST, op(stage_in(P, Wlm, 0, n), G_LL), op(stage_in(P, dWlm, 1, n)),
+                       op(stage_in(P, Zlm, 2, n)));
     double *out[3] = {vrc, vtc, vpc};
     return synth_call(P, j, 3, lcut, 0.0, out);
 }
@@ -669,10 +624,8 @@ int mhx_sphtor_to_spat(mhx_plan *h, const double *dWlm, const double *Zlm, doubl
                        double *vpc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_SPHTOR, 1, 0);
-    j.src[0] = stage_in(P, dWlm, 0, 2 * P->lm_max);
-    j.src[1] = stage_in(P, Zlm, 1, 2 * P->lm_max);
-    sphtor_cols(j, op(0), op(1));
+    const size_t n = 2 * P->lm_max;
+    SynJob j = syn_job(P, SYN_SPHTOR, op(stage_in(P, dWlm, 0, n)), op(stage_in(P, Zlm, 1, n)));
     double *out[2] = {vtc, vpc};
     return synth_call(P, j, 2, lcut, 0.0, out);
 }
@@ -691,11 +644,7 @@ static int ic_call(Plan *P, double r, double r_ICB, int curl, const double *a0, 
     k_ic_preop<<<(P->lm_max + 127) / 128, 128, 0, P->stream>>>(P->lm_max, P->d_lm2l, r / r_ICB, r_ICB,
                                                                r, curl, s0, s1, s2, s3, Q, S, T);
     MHX_HIP_CHECK(hipGetLastError());
-    SynJob j = syn_job(P, SYN_QST, 1, 0);
-    j.src[0] = Q;
-    j.src[1] = S;
-    j.src[2] = T;
-    qst_cols(j, op(0), op(1), op(2));
+    SynJob j = syn_job(P, SYN_QST, op(Q), op(S), op(T));
     double *out[3] = {o0, o1, o2};
     return synth_call(P, j, 3, P->l_max, 0.0, out);
 }
@@ -719,13 +668,12 @@ int mhx_torpol_to_dphspat(mhx_plan *h, const double *dWlm, const double *Zlm, do
                           double *dvpdp, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_SPHTOR, 1, 0);
-    j.src[0] = stage_in(P, dWlm, 0, 2 * P->lm_max);
-    j.src[1] = stage_in(P, Zlm, 1, 2 * P->lm_max);
     // S = i m dW, T = i m Z (src/sht_native.f90:249-262); outputs times
     // 1/sin^2(theta) (:266-270)
-    sphtor_cols(j, op(0, G_ONE, 1, 1), op(1, G_ONE, 1, 1));
-    j.row_scale[0] = j.row_scale[1] = 1;
+    const size_t n = 2 * P->lm_max;
+    SynJob j = syn_job(P, SYN_SPHTOR, op(stage_in(P, dWlm, 0, n), G_ONE, nullptr, 1),
+                       op(stage_in(P, Zlm, 1, n), G_ONE, nullptr, 1));
+    j.row_scale = 1;
     double *out[2] = {dvtdp, dvpdp};
     return synth_call(P, j, 2, lcut, 0.0, out);
 }
@@ -733,9 +681,7 @@ int mhx_torpol_to_dphspat(mhx_plan *h, const double *dWlm, const double *Zlm, do
 int mhx_pol_to_curlr_spat(mhx_plan *h, const double *Qlm, double *cvrc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_SCAL, 1, 0);
-    j.src[0] = stage_in(P, Qlm, 0, 2 * P->lm_max);
-    j.col[0] = op(0, G_LL);
+    SynJob j = syn_job(P, SYN_SCAL, op(stage_in(P, Qlm, 0, 2 * P->lm_max), G_LL));
     double *out[1] = {cvrc};
     return synth_call(P, j, 1, lcut, 0.0, out);
 }
@@ -745,13 +691,11 @@ int mhx_torpol_to_curl_spat(mhx_plan *h, double or2, const double *Blm, const do
                             double *cvpc, int lcut)
 {
     PLAN_OR_FAIL(h);
-    SynJob j = syn_job(P, SYN_QST, 1, 0);
-    j.src[0] = stage_in(P, Blm, 0, 2 * P->lm_max);
-    j.src[1] = stage_in(P, ddBlm, 1, 2 * P->lm_max);
-    j.src[2] = stage_in(P, Jlm, 2, 2 * P->lm_max);
-    j.src[3] = stage_in(P, dJlm, 3, 2 * P->lm_max);
+    const size_t n = 2 * P->lm_max;
+    const double *B = stage_in(P, Blm, 0, n), *ddB = stage_in(P, ddBlm, 1, n);
     // Q = l(l+1) J, S = dJ, T = or2 l(l+1) B - ddB (src/sht_native.f90:320-330)
-    qst_cols(j, op(2, G_LL), op(3), op(0, G_OR2LL, 0, 0, 1.0, 1, -1.0));
+    SynJob j = syn_job(P, SYN_QST, op(stage_in(P, Jlm, 2, n), G_LL), op(stage_in(P, dJlm, 3, n)),
+                       op(B, G_OR2LL, ddB));
     double *out[3] = {cvrc, cvtc, cvpc};
     return synth_call(P, j, 3, lcut, or2, out);
 }
@@ -904,12 +848,8 @@ int mhx_torpol_to_spat_batch(mhx_plan *h, int nlev, const double *W, const doubl
     if ((rc = order_after(P, stream)) || (rc = ensure_ws(P, nlev)) ||
         (rc = upload_lcut(P, lcut, nlev)))
         return rc;
-    SynJob j = syn_job(P, SYN_QST, nlev, ld_lm);
-    j.src[0] = W;
-    j.src[1] = dW;
-    j.src[2] = Z;
-    qst_cols(j, op(0, G_LL), op(1), op(2));
-    if ((rc = launch_syn(P, j, P->stream))) return rc;
+    SynJob j = syn_job(P, SYN_QST, op(W, G_LL), op(dW), op(Z));
+    if ((rc = launch_syn(P, &j, 1, syn_batch(P, nlev, ld_lm), P->stream))) return rc;
     double *dst[3] = {vr, vt, vp};
     if ((rc = ifft_to(P, 0, 3, nlev, dst, ld_grid))) return rc;
     MHX_HIP_CHECK(hipStreamSynchronize(P->stream));
@@ -1185,39 +1125,31 @@ static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t l
         };
         auto launch_fp64 = [&]() -> int {
             int rc2;
-            {
-                SynJob j = syn_job(P, SYN_SG, nlev, ld_lm);
-                j.src[0] = din[S];
-                j.col[0] = op(0);
-                j.col[1] = op(0, G_ONE, 1, 1);
-                j.out_comp[0] = 15; j.out_comp[1] = 16; j.out_comp[2] = 17;
-                if ((rc2 = fork())) return rc2;
-                if ((rc2 = launch_syn(P, j, on(5))) || (rc2 = mark())) return rc2;
-            }
-            struct QSpec { int q, sidx, t0, t1; bool curl; int comp0; };
             // torpol_to_spat(a, b, c): Q = l(l+1) a, S = b, T = c
             // torpol_to_curl_spat(or2, B, ddB, J, dJ): Q = l(l+1) J, S = dJ, T = or2 l(l+1) B - ddB
-            const QSpec qs[5] = {
-                {W, DW, Z, -1, false, 0},     // u
-                {Z, DZ, W, DDW, true, 3},     // curl u
-                {DW, DDW, DZ, -1, false, 6},  // du/dr
-                {B, DB, AJ, -1, false, 9},    // B
-                {AJ, DJ, B, DDB, true, 12},   // curl B
+            auto torpol = [&](int a, int b, int c, int comp0) {
+                return syn_job(P, SYN_QST, op(din[a], G_LL), op(din[b]), op(din[c]), comp0);
             };
-            for (int v = 0; v < 5; ++v) {
-                if (v == 2 && !dudr) continue;
-                const QSpec &q = qs[v];
-                SynJob j = syn_job(P, SYN_QST, nlev, ld_lm);
-                j.src[0] = din[q.q];
-                j.src[1] = din[q.sidx];
-                j.src[2] = din[q.t0];
-                j.src[3] = q.t1 >= 0 ? din[q.t1] : nullptr;
-                ColOp T = q.curl ? op(2, G_OR2LL, 0, 0, 1.0, 3, -1.0) : op(2);
-                qst_cols(j, op(0, G_LL), op(1), T);
-                j.out_comp[0] = q.comp0; j.out_comp[1] = q.comp0 + 1; j.out_comp[2] = q.comp0 + 2;
-                if ((rc2 = launch_syn(P, j, on(v))) || (rc2 = mark())) return rc2;
+            auto curl = [&](int b, int ddb, int j, int dj, int comp0) {
+                return syn_job(P, SYN_QST, op(din[j], G_LL), op(din[dj]), op(din[b], G_OR2LL, din[ddb]), comp0);
+            };
+            SynJob jobs[6];
+            int nj = 0;
+            jobs[nj++] = syn_job(P, SYN_SG, op(din[S]), ColOp(), ColOp(), 15);
+            jobs[nj++] = torpol(W, DW, Z, 0);
+            jobs[nj++] = curl(W, DDW, Z, DZ, 3);
+            if (dudr) jobs[nj++] = torpol(DW, DDW, DZ, 6);
+            jobs[nj++] = torpol(B, DB, AJ, 9);
+            jobs[nj++] = curl(B, DDB, AJ, DJ, 12);
+            // all in one launch (one by one when timed); the scalar's short
+            // blocks last
+            const SynBatch sb = syn_batch(P, nlev, ld_lm);
+            if (P->timing) {
+                for (int v = 0; v < nj; ++v)
+                    if ((rc2 = launch_syn(P, jobs + v, 1, sb, s)) || (rc2 = mark())) return rc2;
+            } else {
+                if ((rc2 = launch_syn(P, jobs, nj, sb, s))) return rc2;
             }
-            if ((rc2 = join())) return rc2;
             // fused: inverse FFTs, grid products, forward FFTs; du/dr grids to ws_G
             if (((rc2 = launch_nl_fused(P, nlev, P->ws_F, P->ws_F2, P->d_rad, LFfac, dudr ? P->ws_G : nullptr,
                                                  grids, s)) ||

@@ -233,38 +233,9 @@ int grow(double *&buf, size_t &have, size_t need_doubles)
     return MHX_OK;
 }
 
-ColOp rop(int s0, int g = G_ONE, int ipow = 0, int mpow = 0, double scale = 1.0, int s1 = -1,
-          double h = 0.0)
+ColOp rop(const double *x0, int g = G_ONE, const double *x1 = nullptr, int im = 0)
 {
-    ColOp c;
-    c.src0 = s0;
-    c.src1 = s1;
-    c.gkind = g;
-    c.ipow = ipow;
-    c.mpow = mpow;
-    c.hcoef = h;
-    c.scale = scale;
-    return c;
-}
-
-// columns Q, S, i m T, i m S, -T of a QST synthesis; S, i m T, i m S, -T of a
-// sph-tor synthesis (the forms of the per-call entries)
-void rl_qst_cols(SynJob &j, ColOp Q, ColOp S, ColOp T, bool with_q)
-{
-    ColOp miT = T;
-    miT.ipow = (miT.ipow + 1) & 3;
-    miT.mpow += 1;
-    ColOp miS = S;
-    miS.ipow = (miS.ipow + 1) & 3;
-    miS.mpow += 1;
-    ColOp mT = T;
-    mT.scale = -mT.scale;
-    int k = 0;
-    if (with_q) j.col[k++] = Q;
-    j.col[k++] = S;
-    j.col[k++] = miT;
-    j.col[k++] = miS;
-    j.col[k++] = mT;
+    return ColOp{x0, x1, g, im};
 }
 
 }  // namespace
@@ -567,25 +538,24 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
 
     // ---- synthesis ----
     enum { W = 0, DW, DDW, Z, DZ, S_, XI, PHI, BB, DB, DDB, AJ, DJ };
-    auto syn = [&](int kind, std::initializer_list<int> srcs, int c0, int c1, int c2) -> SynJob {
-        SynJob j;
+    const SynBatch sb{nlev, ld_lm, (size_t)nin * P->n_m * P->n_theta, B->lcut, d_or2};
+    SynJob jobs[MAX_SYN_JOBS];
+    int njob = 0;
+    auto add = [&](int kind, ColOp a, ColOp b, ColOp c, int c0, int c1, int c2) -> SynJob & {
+        SynJob &j = jobs[njob++];
         std::memset(&j, 0, sizeof(j));
         j.kind = kind;
-        j.nlev = nlev;
-        j.src_ld = ld_lm;
-        int k = 0;
-        for (int sidx : srcs) j.src[k++] = din[sidx];
+        j.col[0] = a;
+        j.col[1] = b;
+        j.col[2] = c;
         j.fout = B->F;
-        j.fout_ld = (size_t)nin * P->n_m * P->n_theta;
         j.out_comp[0] = c0;
         j.out_comp[1] = c1;
         j.out_comp[2] = c2;
-        j.lcut = B->lcut;
-        j.or2 = d_or2;
         return j;
     };
-    // independent launches (the syntheses, then the analyses) dealt over
-    // the plan's branch streams, forked from and joined back into s
+    // independent launches (the analyses) dealt over the plan's branch
+    // streams, forked from and joined back into s
     int nl_launch = 0;
     auto on = [&]() -> hipStream_t {
         const int i = nl_launch++ % P->nbranch;
@@ -605,60 +575,38 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
         }
         return MHX_OK;
     };
-    if ((rc = fork())) return rc;
-    if (conv) {
-        // torpol_to_spat(w, dw, z): Q = l(l+1) w, S = dw, T = z
-        SynJob j = syn(SYN_QST, {W, DW, Z}, in_of[RI_VR], in_of[RI_VT], in_of[RI_VP]);
-        rl_qst_cols(j, rop(0, G_LL), rop(1), rop(2), true);
-        if ((rc = launch_syn(P, j, on()))) return rc;
-        if (curl) {
-            // torpol_to_curl_spat(or2, w, ddw, z, dz): Q = l(l+1) z, S = dz,
-            // T = or2 l(l+1) w - ddw
-            SynJob c = syn(SYN_QST, {W, DDW, Z, DZ}, in_of[RI_CVR], in_of[RI_CVT], in_of[RI_CVP]);
-            rl_qst_cols(c, rop(2, G_LL), rop(3), rop(0, G_OR2LL, 0, 0, 1.0, 1, -1.0), true);
-            if ((rc = launch_syn(P, c, on()))) return rc;
-        }
-        if (need_grad) {
-            if (!curl) {
-                // pol_to_curlr_spat(z): l(l+1) z
-                SynJob c = syn(SYN_SCAL, {Z}, in_of[RI_CVR], 0, 0);
-                c.col[0] = rop(0, G_LL);
-                if ((rc = launch_syn(P, c, on()))) return rc;
-            }
-            // torpol_to_spat(dw, ddw, dz)
-            SynJob d = syn(SYN_QST, {DW, DDW, DZ}, in_of[RI_DVRDR], in_of[RI_DVTDR], in_of[RI_DVPDR]);
-            rl_qst_cols(d, rop(0, G_LL), rop(1), rop(2), true);
-            if ((rc = launch_syn(P, d, on()))) return rc;
-            // pol_to_grad_spat(w): gradient of l(l+1) w
-            SynJob g = syn(SYN_GRAD, {W}, in_of[RI_DVRDT], in_of[RI_DVRDP], 0);
-            g.col[0] = rop(0, G_LL);
-            g.col[1] = rop(0, G_LL, 1, 1);
-            if ((rc = launch_syn(P, g, on()))) return rc;
-            // torpol_to_dphspat(dw, z): S = i m dw, T = i m z, times 1/sin^2
-            SynJob q = syn(SYN_SPHTOR, {DW, Z}, in_of[RI_DVTDP], in_of[RI_DVPDP], 0);
-            rl_qst_cols(q, ColOp(), rop(0, G_ONE, 1, 1), rop(1, G_ONE, 1, 1), false);
-            q.row_scale[0] = q.row_scale[1] = 1;
-            if ((rc = launch_syn(P, q, on()))) return rc;
-        }
-    }
-    auto scalar = [&](int src, int comp) -> int {
-        SynJob j = syn(SYN_SCAL, {src}, comp, 0, 0);
-        j.col[0] = rop(0);
-        return launch_syn(P, j, on());
+    const ColOp none = ColOp();
+    auto torpol = [&](int a, int b, int c, int comp) {
+        add(SYN_QST, rop(din[a], G_LL), rop(din[b]), rop(din[c]), in_of[comp], in_of[comp + 1], in_of[comp + 2]);
     };
-    if (heat && (rc = scalar(S_, in_of[RI_S]))) return rc;
-    if (chem && (rc = scalar(XI, in_of[RI_XI]))) return rc;
-    if (phase && (rc = scalar(PHI, in_of[RI_PHI]))) return rc;
-    if (mag) {
-        SynJob b = syn(SYN_QST, {BB, DB, AJ}, in_of[RI_BR], in_of[RI_BT], in_of[RI_BP]);
-        rl_qst_cols(b, rop(0, G_LL), rop(1), rop(2), true);
-        if ((rc = launch_syn(P, b, on()))) return rc;
-        SynJob c = syn(SYN_QST, {BB, DDB, AJ, DJ}, in_of[RI_CBR], in_of[RI_CBT], in_of[RI_CBP]);
-        rl_qst_cols(c, rop(2, G_LL), rop(3), rop(0, G_OR2LL, 0, 0, 1.0, 1, -1.0), true);
-        if ((rc = launch_syn(P, c, on()))) return rc;
+    // torpol_to_curl_spat(or2, B, ddB, J, dJ): Q = l(l+1) J, S = dJ, T = or2 l(l+1) B - ddB
+    auto tocurl = [&](int b, int ddb, int j, int dj, int comp) {
+        add(SYN_QST, rop(din[j], G_LL), rop(din[dj]), rop(din[b], G_OR2LL, din[ddb]), in_of[comp], in_of[comp + 1],
+            in_of[comp + 2]);
+    };
+    auto scalar = [&](int src, int g, int comp) { add(SYN_SCAL, rop(din[src], g), none, none, in_of[comp], 0, 0); };
+    if (conv) {
+        torpol(W, DW, Z, RI_VR);
+        if (curl) tocurl(W, DDW, Z, DZ, RI_CVR);
+        if (need_grad) {
+            if (!curl) scalar(Z, G_LL, RI_CVR);  // pol_to_curlr_spat(z): l(l+1) z
+            torpol(DW, DDW, DZ, RI_DVRDR);
+            // pol_to_grad_spat(w): gradient of l(l+1) w
+            add(SYN_GRAD, rop(din[W], G_LL), none, none, in_of[RI_DVRDT], in_of[RI_DVRDP], 0);
+            // torpol_to_dphspat(dw, z): S = i m dw, T = i m z, times 1/sin^2
+            add(SYN_SPHTOR, rop(din[DW], G_ONE, nullptr, 1), rop(din[Z], G_ONE, nullptr, 1), none,
+                in_of[RI_DVTDP], in_of[RI_DVPDP], 0)
+                .row_scale = 1;
+        }
     }
-
-    if ((rc = join())) return rc;
+    if (heat) scalar(S_, G_ONE, RI_S);
+    if (chem) scalar(XI, G_ONE, RI_XI);
+    if (phase) scalar(PHI, G_ONE, RI_PHI);
+    if (mag) {
+        torpol(BB, DB, AJ, RI_BR);
+        tocurl(BB, DDB, AJ, DJ, RI_CBR);
+    }
+    if ((rc = launch_syn(P, jobs, njob, sb, s))) return rc;
 
     // ---- grid stage ----
     RlGridArgs g;

@@ -12,6 +12,9 @@
 //   analysis   (MFMA A operand 16 l x 4 theta):
 //     ana[ana_off[2mc+p] + ((kk/16) * nq4 + th/4) * 64 + (kk%16) + 16*(th%4)]
 // where th is the northern-hemisphere theta index.  Padding entries are 0.
+//   FP64 kernels' synthesis table, l <= l_max + 1 (two K quads per lane, so
+//   that a fragment load is 16 bytes per lane):
+//     synx[synx_off[2mc+p] + ((kk/8) * nt16 + th/16) * 128 + ((th%16) + 16*(kk%4)) * 2 + (kk/4)%2]
 #include "mhx_internal.h"
 
 #include <cmath>
@@ -98,6 +101,33 @@ __global__ void k_plm_tables(int l_max, int minc, int n_m, int nh, int nt16, int
         aP[ao] = w * Pl;
         adP[ao] = w * dPl;
     });
+}
+
+// the FP64 kernels' tables: the same recurrence up to l_max + 1, P only
+__global__ void k_p_tables(int l_max, int minc, int n_m, int nh, int nt16,
+                           const double *__restrict__ theta, const size_t *__restrict__ synx_off,
+                           double *__restrict__ synx)
+{
+    int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= n_m * nh) return;
+    int mc = idx / nh, th = idx - mc * nh;
+    int m = mc * minc;
+    double t = theta[th];
+    plm_sweep(l_max + 1, m, sin(t), cos(t), [&](int l, double Pl, double) {
+        int par = (l - m) & 1, kk = (l - m) >> 1;
+        synx[synx_off[2 * mc + par] + ((size_t)(kk >> 3) * nt16 + (th >> 4)) * 128 +
+             ((th & 15) + 16 * (kk & 3)) * 2 + ((kk >> 2) & 1)] = Pl;
+    });
+}
+
+// c_l = sqrt((l^2 - m^2) / (4 l^2 - 1)) for l = m .. l_max + 2 at lstart[mc] +
+// 2 mc; one thread per (mc, l - m)
+__global__ void k_crec64(int l_max, int minc, const int *__restrict__ lstart, double *__restrict__ c)
+{
+    const int mc = blockIdx.y, m = mc * minc, d = blockIdx.x * blockDim.x + threadIdx.x;
+    if (d > l_max + 2 - m) return;
+    const double dl = (double)(m + d), dm = (double)m;
+    c[lstart[mc] + 2 * mc + d] = d > 0 ? sqrt((dl - dm) * (dl + dm) / ((2.0 * dl - 1.0) * (2.0 * dl + 1.0))) : 0.0;
 }
 
 // Row factors of the split tables straight from the recurrence (plans whose
@@ -217,6 +247,37 @@ int build_tables(Plan *p)
     k_plm_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, nh, p->nt16, p->nq4,
                                            p->d_theta, p->d_gauss, p->d_syn_off, p->d_ana_off,
                                            p->d_syn_P, p->d_syn_dP, p->d_ana_wP, p->d_ana_wdP);
+    MHX_HIP_CHECK(hipGetLastError());
+    MHX_HIP_CHECK(hipDeviceSynchronize());
+    return MHX_OK;
+}
+
+int ensure_p_tables(Plan *p)
+{
+    if (p->d_synx) return MHX_OK;
+    if (int rc = ensure_fp64_tables(p)) return rc;
+    std::vector<size_t> so(2 * (size_t)p->n_m);
+    size_t ns = 0, nc = 0;
+    for (int mc = 0; mc < p->n_m; ++mc) {
+        const int nrow = p->l_max + 2 - mc * p->minc;
+        const int K[2] = {(nrow + 1) / 2, nrow / 2};
+        for (int par = 0; par < 2; ++par) {
+            so[2 * mc + par] = ns;
+            ns += (size_t)((K[par] + 7) / 8) * p->nt16 * 128;
+        }
+        nc = (size_t)p->lstart[mc] + 2 * mc + nrow + 1;
+    }
+    double *synx = nullptr;
+    if (!p->d_synx_off) MHX_HIP_CHECK(hipMalloc(&p->d_synx_off, so.size() * sizeof(size_t)));
+    if (!p->d_crec64) MHX_HIP_CHECK(hipMalloc(&p->d_crec64, nc * sizeof(double)));
+    MHX_HIP_CHECK(hipMemcpy(p->d_synx_off, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMalloc(&synx, ns * sizeof(double)));
+    p->d_synx = synx;
+    MHX_HIP_CHECK(hipMemset(synx, 0, ns * sizeof(double)));
+    const int n = p->n_m * p->nh;
+    k_p_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, p->nh, p->nt16, p->d_theta, p->d_synx_off, synx);
+    k_crec64<<<dim3((unsigned)((p->l_max + 3 + 127) / 128), (unsigned)p->n_m), 128>>>(p->l_max, p->minc, p->d_lstart,
+                                                                                      p->d_crec64);
     MHX_HIP_CHECK(hipGetLastError());
     MHX_HIP_CHECK(hipDeviceSynchronize());
     return MHX_OK;
