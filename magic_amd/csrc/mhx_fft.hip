@@ -10,14 +10,27 @@
 // and N/2 (src/fft.f90:386-398).
 //
 // Fourier layouts: the inverse side F[lev][comp][m][theta] (written in
-// contiguous theta runs by the synthesis), the forward side
-// F2[lev][comp][theta][m] (written in contiguous rows by the FFT kernels);
-// m < n_m, modes up to N/2 beyond n_m are zero (src/shtransforms.f90:224-232).
+// contiguous theta runs by the synthesis), the forward side theta-blocked,
+// F2[lev][comp][theta/TH][m][theta%TH] with TH = 8 in FP64 and 16 in FP32: the
+// analysis reads one 128-byte line per (comp, m, block); m < n_m, modes up to N/2 beyond n_m are zero (src/shtransforms.f90:224-232).
 #include "mhx_fftcore.h"
 
 namespace mhx {
 
 namespace {
+
+// forward side: theta rows per block of F2, complex elements per comp, and the
+// index of (comp, theta, m)
+template <typename T> constexpr int f2_th() { return sizeof(T) == 4 ? 16 : 8; }
+template <typename T> __device__ __forceinline__ size_t f2_size(int n_theta, int n_m)
+{
+    return (size_t)((n_theta + f2_th<T>() - 1) / f2_th<T>()) * n_m * f2_th<T>();
+}
+template <typename T> __device__ __forceinline__ size_t f2_index(int comp, int th, int k, int n_theta, int n_m)
+{
+    constexpr int TH = f2_th<T>();
+    return comp * f2_size<T>(n_theta, n_m) + ((size_t)(th / TH) * n_m + k) * TH + th % TH;
+}
 
 // ---------------------------------------------------------------------------
 // API path: Fourier rows <-> theta-fastest grids (Fortran f(n_theta, n_phi))
@@ -69,8 +82,7 @@ __global__ void k_ifft_rows(FFTArgs f, const T *__restrict__ F, size_t F_ld, int
 template <typename T>
 __global__ void k_fft_rows(FFTArgs f, const T *__restrict__ g, size_t g_ld_lev, size_t g_ld_comp,
                            int n_m, int n_theta, int ncomp, int TB, int ntb, unsigned osin2_mask,
-                           const double *__restrict__ osin2, T *__restrict__ F, size_t F_ld,
-                           int blk)
+                           const double *__restrict__ osin2, T *__restrict__ F, size_t F_ld)
 {
     typedef cpx<T> C;
     extern __shared__ char smem_raw[];
@@ -96,19 +108,13 @@ __global__ void k_fft_rows(FFTArgs f, const T *__restrict__ g, size_t g_ld_lev, 
     __syncthreads();
     C *res = fft_pp(A, B, TB, f, s_tw, -1);
     const bool os = (osin2_mask >> comp) & 1u;
-    // F[lev][comp][theta][m], or theta-blocked F[lev][comp][theta/16][m][theta%16]
-    // (blk; the split analysis reads 16 rows of one m as one line)
     C *Fl = reinterpret_cast<C *>(F) + (size_t)lev * F_ld;
-    const int nt16 = (n_theta + 15) / 16;
     for (int idx = threadIdx.x; idx < n_m * TB; idx += blockDim.x) {
-        int k = idx % n_m, r = idx / n_m;
+        const int r = idx % TB, k = idx / TB;
         if (r >= nrows) continue;
         T sc = T(1.0 / (double)N);
         if (os) sc *= T(osin2[th0 + r]);
-        const int th = th0 + r;
-        const size_t o = blk ? (((size_t)comp * nt16 + (th >> 4)) * n_m + k) * 16 + (th & 15)
-                             : ((size_t)comp * n_theta + th) * n_m + k;
-        Fl[o] = rfft_post(res + r * M, k, M, s_twr, sc);
+        Fl[f2_index<T>(comp, th0 + r, k, n_theta, n_m)] = rfft_post(res + r * M, k, M, s_twr, sc);
     }
 }
 
@@ -123,7 +129,7 @@ __global__ void k_fft_rows(FFTArgs f, const T *__restrict__ g, size_t g_ld_lev, 
 // Fin comps (layout [lev][comp][m][theta]):
 //             vr vt vp | cvr cvt cvp | dvr dvt dvp | br bt bp | cbr cbt cbp |
 //             s dsdt dsdp
-// Fout (layout [lev][comp][theta][m]):
+// Fout (theta-blocked F2):
 //             Advr Advt Advp | VSr VSt VSp | VxBr VxBt VxBp | uGs
 // du/dr grids (not consumed by the products) are written to dgrid
 // [lev][3][theta][phi]; with full_grids != nullptr all 18 inverse grids are
@@ -136,8 +142,6 @@ __global__ void k_nl_fused(FFTArgs f, const T *__restrict__ Fin, T *__restrict__
                            const double *__restrict__ rad, double LFfac_d,
                            T *__restrict__ dgrid, T *__restrict__ full_grids, CourArgs cour)
 {
-    // split form (T = float): theta-blocked forward side
-    constexpr bool BLK = sizeof(T) == 4;
     typedef cpx<T> C;
     extern __shared__ char smem_raw[];
     const int M = f.M, N = f.N;
@@ -162,9 +166,8 @@ __global__ void k_nl_fused(FFTArgs f, const T *__restrict__ Fin, T *__restrict__
     __syncthreads();
 
     const size_t rowsz = (size_t)n_m;                   // complex per forward row
-    const int ntb = (n_theta + 15) / 16;
     const C *Fi = reinterpret_cast<const C *>(Fin) + (size_t)lev * 18 * n_theta * rowsz + th;
-    C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * (BLK ? ntb * 16 : n_theta) * rowsz;
+    C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * f2_size<T>(n_theta, n_m);
 
     T u[3][PMAX], adv[3][PMAX], bb[3][PMAX], vxb[3][PMAX], vs[3][PMAX], ugs[PMAX];
     T val[3][PMAX];
@@ -224,11 +227,7 @@ __global__ void k_nl_fused(FFTArgs f, const T *__restrict__ Fin, T *__restrict__
             const T invN = T(1.0 / (double)N);
             for (int idx = tid; idx < gn * n_m; idx += nthr) {
                 int r2 = idx / n_m, k = idx - r2 * n_m;
-                C v = rfft_post(res + r2 * M, k, M, s_twr, invN);
-                if constexpr (BLK)
-                    Fo[(((size_t)(c0 + g0 + r2) * ntb + (th >> 4)) * rowsz + k) * 16 + (th & 15)] = v;
-                else
-                    Fo[((size_t)(c0 + g0 + r2) * n_theta + th) * rowsz + k] = v;
+                Fo[f2_index<T>(c0 + g0 + r2, th, k, n_theta, n_m)] = rfft_post(res + r2 * M, k, M, s_twr, invN);
             }
             __syncthreads();
         }
@@ -356,7 +355,6 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
                                                   CourArgs cour)
 {
     typedef cpx<T> C;
-    constexpr bool BLK = sizeof(T) == 4;  // split form: theta-blocked F2
     extern __shared__ char smem_raw[];
     typedef SlotFFT<A, B> FFT;
     constexpr int M = FFT::M, N = 2 * M, Q = FFT::Q;
@@ -385,9 +383,8 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
     }
     __syncthreads();
 
-    const int ntb = (n_theta + 15) / 16;
     const C *Fi = reinterpret_cast<const C *>(Fin) + (size_t)lev * 18 * n_theta * n_m + th;
-    C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * (BLK ? ntb * 16 : n_theta) * n_m;
+    C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * f2_size<T>(n_theta, n_m);
 
     T u[3][NPT], adv[3][NPT], vxb[3][NPT];
     T val[6][NPT];
@@ -501,10 +498,9 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
             FFT::run(z, t, s_tw, -1);
             const int comp = round == 0 ? (slot < 3 ? slot : slot + 3) : (slot < 3 ? slot + 3 : 9);
             const T invN = T(1.0 / (double)N);
-            // F2 theta-blocked (split form): consecutive k are 16 apart
-            constexpr int FS = BLK ? 16 : 1;
-            C *fo = BLK ? Fo + (((size_t)comp * ntb + (th >> 4)) * n_m + t) * 16 + (th & 15)
-                        : Fo + ((size_t)comp * n_theta + th) * n_m + t;
+            // F2 theta-blocked: consecutive k are FS apart
+            constexpr int FS = f2_th<T>();
+            C *fo = Fo + f2_index<T>(comp, th, t, n_theta, n_m);
             for (int k = t; k < n_m; k += Q, fo += Q * FS) *fo = rfft_post_padded<FFT::P>(z, k, M, s_twr, invN);
         }
         __syncthreads();
@@ -807,15 +803,15 @@ __global__ __launch_bounds__(512) void k_rl_grid(FFTArgs f, RlGridArgs a)
     rl_points(a, reinterpret_cast<double *>(rows), [&](int c, int j) { return (size_t)c * N + j; }, N, lev, th);
     __syncthreads();
 
-    // forward FFTs of rows[0, nout) into F2[lev][comp][theta][m]
-    C *Fo = reinterpret_cast<C *>(a.Fout) + (size_t)lev * a.nout * n_theta * n_m;
+    // forward FFTs of rows[0, nout) into F2
+    C *Fo = reinterpret_cast<C *>(a.Fout) + (size_t)lev * a.nout * f2_size<double>(n_theta, n_m);
     const double invN = 1.0 / (double)N;
     for (int g0 = 0; g0 < a.nout; g0 += a.G) {
         const int gn = min(a.G, a.nout - g0);
         C *res = fft_pp(rows + (size_t)g0 * M, B, gn, f, s_tw, -1);
         for (int idx = tid; idx < gn * n_m; idx += nthr) {
             const int r2 = idx / n_m, k = idx - r2 * n_m;
-            Fo[((size_t)(g0 + r2) * n_theta + th) * n_m + k] = rfft_post(res + (size_t)r2 * M, k, M, s_twr, invN);
+            Fo[f2_index<double>(g0 + r2, th, k, n_theta, n_m)] = rfft_post(res + (size_t)r2 * M, k, M, s_twr, invN);
         }
         __syncthreads();
     }
@@ -885,15 +881,15 @@ __global__ __launch_bounds__(512) void k_rl_grid_s(FFTArgs f, RlGridArgs a)
               [&](int c, int j) { return (size_t)c * 2 * MP + 2 * pidx<P>(j >> 1) + (j & 1); }, N, lev, th);
     __syncthreads();
 
-    // forward FFTs of rows [0, nout) in place, then F2[lev][comp][theta][m]
+    // forward FFTs of rows [0, nout) in place, then F2
     if (act)
         for (int c = slot; c < a.nout; c += nslot) FFT::run(rows + (size_t)c * MP, t, s_tw, -1);
     __syncthreads();
-    C *Fo = reinterpret_cast<C *>(a.Fout) + (size_t)lev * a.nout * n_theta * n_m;
+    C *Fo = reinterpret_cast<C *>(a.Fout) + (size_t)lev * a.nout * f2_size<double>(n_theta, n_m);
     const double invN = 1.0 / (double)N;
     for (int idx = tid; idx < a.nout * n_m; idx += nthr) {
         const int r2 = idx / n_m, k = idx - r2 * n_m;
-        Fo[((size_t)r2 * n_theta + th) * n_m + k] = rfft_post_padded<P>(rows + (size_t)r2 * MP, k, M, s_twr, invN);
+        Fo[f2_index<double>(r2, th, k, n_theta, n_m)] = rfft_post_padded<P>(rows + (size_t)r2 * MP, k, M, s_twr, invN);
     }
 }
 
@@ -951,7 +947,7 @@ int launch_fft(const Plan *p, const double *grid, size_t grid_ld_lev, size_t gri
     size_t shm = api_shm(p, TB);
     k_fft_rows<double><<<dim3((unsigned)(ntb * ncomp * nlev)), 256, shm, s>>>(
         f, grid, grid_ld_lev, grid_ld_comp, p->n_m, p->n_theta, ncomp, TB, ntb, osin2_mask,
-        p->d_osin2, F, F_ld_lev, 0);
+        p->d_osin2, F, F_ld_lev);
     MHX_HIP_CHECK(hipGetLastError());
     return MHX_OK;
 }
@@ -987,7 +983,7 @@ int launch_fft_f32(const Plan *p, const float *grid, size_t g_ld_row, size_t g_l
     if (shm > 64 * 1024 || 256 % TB) return fail(MHX_E_UNSUPPORTED, "rows per block too large");
     k_fft_rows<float><<<dim3((unsigned)(ntb * ncomp * nrow)), 256, shm, s>>>(
         f, grid, g_ld_row, g_ld_comp, p->n_m, p->n_theta, ncomp, TB, ntb, osin2_mask, p->d_osin2,
-        F2, F2_ld, 1);
+        F2, F2_ld);
     MHX_HIP_CHECK(hipGetLastError());
     return MHX_OK;
 }

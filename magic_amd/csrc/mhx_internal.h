@@ -79,18 +79,25 @@ struct SynBatch {
     const double *or2;     // device, per level (may be null)
 };
 
+constexpr int MAX_ANA_JOBS = 8;   // jobs of one analysis launch
+
 struct AnaJob {
     int kind;
-    int nlev;
-    // inputs: Fourier arrays F[lev][comp][m][theta]
-    const double *fin;
-    size_t fin_ld;       // complex elements per level
-    int in_comp[3];      // f (SH/QST), vt, vp
-    // outputs: coefficient arrays
-    double *out[MAX_OUT];
-    size_t out_ld;       // complex elements per level
-    const int *lcut;     // device
+    const double *fin;     // Fourier arrays F2[lev][comp][theta/8][m][theta%8] complex
+    int in_comp[3];        // SH: f; SPHTOR: vt, vp; QST: f, vt, vp
+    double *out[MAX_OUT];  // coefficient arrays
 };
+
+// what the jobs of one launch share
+struct AnaBatch {
+    int nlev;
+    size_t fin_ld;         // complex elements per level of the Fourier arrays
+    size_t out_ld;         // complex elements per level of the outputs
+    const int *lcut;       // device, per level
+};
+
+// complex elements of one comp of the FP64 forward side F2 (theta in blocks of 8)
+inline size_t f2_comp(int n_m, int n_theta) { return (size_t)((n_theta + 7) / 8) * n_m * 8; }
 
 // Legendre kernels of the nonlinear step in the split form (mhx_nlsplit.hip)
 // NS_S: the scalar alone (no gradient), split whole-K form only
@@ -191,7 +198,7 @@ struct RlPhys {
 
 struct RlGridArgs {
     const double *Fin;   // F[lev][nin][m][theta] complex
-    double *Fout;        // F2[lev][nout][theta][m] complex
+    double *Fout;        // F2[lev][nout][theta/8][m][theta%8] complex
     int nin, nout;
     int in_of[RI_N];     // row (compact comp index) of each grid component, -1 absent
     int out_of[RO_N];    // row of each product, -1 absent
@@ -242,8 +249,8 @@ struct Plan {
     size_t *d_syn_off = nullptr, *d_ana_off = nullptr;
     // the FP64 Legendre kernels' tables: P_lm for l <= l_max + 1, two K quads
     // per lane, and the factors c_l (ensure_p_tables)
-    double *d_synx = nullptr, *d_crec64 = nullptr;
-    size_t *d_synx_off = nullptr;
+    double *d_synx = nullptr, *d_anax = nullptr, *d_crec64 = nullptr;
+    size_t *d_synx_off = nullptr, *d_anax_off = nullptr;
     double *d_osin2 = nullptr;      // n_theta (scrambled)
     double *d_theta = nullptr, *d_gauss = nullptr; // nh
     double *d_tw = nullptr;         // M complex: exp(-2 pi i k/M)
@@ -349,10 +356,10 @@ int launch_e_kin(const Plan *p, const EkArgs &args, hipStream_t s);
 int launch_nana16(const Plan *p, int kind, const NAnaArgs &args, hipStream_t s);
 // the jobs of one launch (their outputs distinct comps)
 int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, hipStream_t s);
-int launch_ana(const Plan *p, const AnaJob &job, hipStream_t s);
+int launch_ana(const Plan *p, const AnaJob *jobs, int njob, const AnaBatch &b, hipStream_t s);
 // Fourier data (complex, m < n_m): inverse side F[lev][comp][m][theta],
-// forward side F2[lev][comp][theta][m]; grids in the reference layout (theta
-// fastest).  F points at the first comp; F_ld_lev is the level stride in
+// forward side F2[lev][comp][theta/8][m][theta%8]; grids in the reference layout
+// (theta fastest).  F points at the first comp; F_ld_lev is the level stride in
 // complex elements; grid comp c of level l starts at
 // grid + l*grid_ld_lev + c*grid_ld_comp (doubles).
 int launch_ifft(const Plan *p, const double *F, size_t F_ld_lev, int F_ncomp, int ncomp,

@@ -21,38 +21,18 @@
 // Analysis (src/shtransforms.f90:648-872): rows are l of one parity, K is the
 // northern theta, columns as above; the ES/EA combinations of north/south
 // Fourier rows are formed while staging B, Gauss weights are folded into the
-// tables (wPlm, wdPlm).
+// table.  Again only wP is contracted, G_l = sum_theta wP_l v for l <= l_max +
+// 1 and v = f, vt, vp; the dP products follow from the same identity,
+//     sum_theta wdP_l v = l c_{l+1} G_{l+1} - (l+1) c_l G_{l-1}.
 #include "mhx_internal.h"
+
+#include <algorithm>
 
 namespace mhx {
 
 namespace {
 
 constexpr int WG = 256;
-constexpr int KQC = 8;          // quads (of 4 l or 4 theta) per staged chunk
-constexpr int CHUNK = 4 * KQC;  // 32 rows of B per parity / per theta chunk
-
-struct Prod {
-    int acc, tab, col;  // tab 0: P, 1: dP
-};
-
-template <int KIND> struct AnaSpec;
-template <> struct AnaSpec<ANA_SH> {      // cols: f
-    static constexpr int NOUT = 1, NCOL = 1, NPROD = 1;
-    static constexpr Prod prod[1] = {{0, 0, 0}};
-    static constexpr bool divll[1] = {false};
-};
-template <> struct AnaSpec<ANA_SPHTOR> {  // cols: vt, -i m vp, -vp, -i m vt
-    static constexpr int NOUT = 2, NCOL = 4, NPROD = 4;
-    static constexpr Prod prod[4] = {{0, 1, 0}, {0, 0, 1}, {1, 1, 2}, {1, 0, 3}};
-    static constexpr bool divll[2] = {true, true};
-};
-template <> struct AnaSpec<ANA_QST> {     // cols: f, vt, -i m vp, -vp, -i m vt
-    static constexpr int NOUT = 3, NCOL = 5, NPROD = 5;
-    static constexpr Prod prod[5] = {{0, 0, 0}, {1, 1, 1}, {1, 0, 2}, {2, 1, 3}, {2, 0, 4}};
-    static constexpr bool divll[3] = {false, true, true};
-};
-
 struct SynArgs {
     SynJob job[MAX_SYN_JOBS];
     int njob, nlev, ng, gz;
@@ -68,11 +48,16 @@ struct SynArgs {
 };
 
 struct AnaArgs {
-    AnaJob job;
-    const double *aP, *adP;
+    AnaJob job[MAX_ANA_JOBS];
+    int njob, nlev, ng, gz;
+    size_t fin_ld, out_ld;
+    const int *lcut;
+    const double *tab;     // 2 pi w P_lm, l <= l_max + 1 (layout: mhx_tables.hip)
     const size_t *off;
+    const double *crec;
     const int *lstart;
-    int l_max, m_max, minc, n_m, nh, n_theta, nq4;
+    int l_max, m_max, minc, n_m, nh, n_theta, nq8;
+    int erows;             // rows of one epilogue area in LDS
 };
 
 // v_mfma_f64_16x16x4f64 operands: A lane l holds A[l % 16][l / 16], B lane l
@@ -80,34 +65,6 @@ struct AnaArgs {
 __device__ inline d4 mfma64(double a, double b, d4 c)
 {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// Blocks are dispatched round-robin over the 8 XCDs (each with its own L2).
-// Remap the linear block id so that each XCD works through a contiguous range
-// of logical blocks; with the order index m fastest, the blocks resident on
-// one XCD at a time cover neighbouring m, whose values share cache lines of
-// the row-contiguous forward-side layout F2[lev][comp][theta][m].
-__device__ inline int xcd_logical(int b, int nb)
-{
-    const int nx = 8;
-    int per = nb / nx, rem = nb % nx;
-    int x = b % nx, i = b / nx;
-    return (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + i;
-}
-
-// i^ipow * m^mpow * scale applied to (re, im)
-__device__ inline void apply_factor(double &re, double &im, int ipow, int mpow, double m,
-                                    double scale)
-{
-    double f = scale;
-    for (int k = 0; k < mpow; ++k) f *= m;
-    re *= f;
-    im *= f;
-    for (int k = 0; k < (ipow & 3); ++k) {
-        double t = re;
-        re = -im;
-        im = t;
-    }
 }
 
 // ------------------------------------------------------------- synthesis
@@ -350,155 +307,230 @@ __global__ __launch_bounds__(WG, 2) void k_syn(SynArgs a)
 }
 
 // -------------------------------------------------------------- analysis
-template <int KIND>
-__global__ __launch_bounds__(WG) void k_ana(AnaArgs a)
-{
-    using S = AnaSpec<KIND>;
-    constexpr int NOUT = S::NOUT, NCOL = S::NCOL, NPROD = S::NPROD;
-    constexpr int BS_DOUBLES = NCOL * 2 * CHUNK * 16;     // [col][sym/anti][32 th][16]
-    constexpr int EP_DOUBLES = 4 * LEV_GROUP * 32 * 2;
-    __shared__ double smem[BS_DOUBLES > EP_DOUBLES ? BS_DOUBLES : EP_DOUBLES];
+template <int KIND> constexpr int ana_np() { return KIND == ANA_QST ? 3 : (KIND == ANA_SH ? 1 : 2); }
 
-    const AnaJob &job = a.job;
-    const int lb = xcd_logical(blockIdx.x, gridDim.x);
-    const int mc = lb % a.n_m;
-    const int ng = (job.nlev + LEV_GROUP - 1) / LEV_GROUP;
-    const int gy = (lb / a.n_m) % ng, gz = lb / (a.n_m * ng);
-    const int m = mc * a.minc;
+// B chunk in LDS: 32 northern theta, [column][Sym/Anti][pair of quads] blocks
+// of 64 lanes x 2 quads, padded as the synthesis' blocks
+constexpr int AB_PAIR = 132, AB_SA = 4 * AB_PAIR, AB_COL = 2 * AB_SA;
+// epilogue rows [l][8 levels x re/im], padded against the column reads
+constexpr int AE_ROW = 18;
+
+// One workgroup: one job, one order m (index mc), 8 radial levels from lev0,
+// and up to 2 TPW pairs of l tiles (32 consecutive l: 16 of each parity);
+// waves 0 and 1 take the even-parity tiles, 2 and 3 the odd ones.  Per chunk
+// of 32 northern theta a thread owns one (level, theta): it loads the north
+// and south rows (32 consecutive bytes of the theta-blocked F2) a chunk
+// ahead, forms Sym and Anti and writes them to the other half of the LDS
+// buffer; table fragments are loaded a step (8 theta) ahead.  Where the
+// order's tiles need more than one workgroup they overlap by one tile pair,
+// whose rows each workgroup's edge needs as neighbours.
+template <int TPW, int KIND>
+__device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, int mc, int lev0, int gz, double *sB)
+{
+    constexpr int NP = ana_np<KIND>();
+    constexpr int BUF = NP * AB_COL;
+    const int m = mc * a.minc, L = a.l_max;
     const double dm = (double)m;
-    const int lev0 = gy * LEV_GROUP;
-    const int nlev_here = min(LEV_GROUP, job.nlev - lev0);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int t = gz * 4 + wave;  // pair tile: l = m + 32 t + 0..31
-    const int K0 = (a.l_max - m) / 2 + 1;
-    const int ntile = (K0 + 15) / 16;
-    const bool active = t < ntile;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int nt = (L + 2 - m + 31) >> 5;                // tile pairs of this order (l <= l_max + 1)
+    const int zb = gz * (2 * TPW - 1);                   // first tile pair of this workgroup
+    if (gz > 0 && zb + 1 >= nt) return;                  // covered by the workgroup before
+    const int par = wave >> 1, t0 = zb + (wave & 1);     // this wave's tiles: t0 + 2 s
     const int l0 = a.lstart[mc];
 
-    // column definitions: source comp slot, i-power, m-power, scale
-    // SH: f | SPHTOR: vt, -i m vp, -vp, -i m vt | QST: f + SPHTOR's
-    int csrc[NCOL], cip[NCOL], cmp[NCOL];
-    double csc[NCOL];
-    if constexpr (KIND == ANA_SH) {
-        csrc[0] = 0; cip[0] = 0; cmp[0] = 0; csc[0] = 1.0;
-    } else {
-        const int b = (KIND == ANA_QST) ? 1 : 0;
-        if constexpr (KIND == ANA_QST) { csrc[0] = 0; cip[0] = 0; cmp[0] = 0; csc[0] = 1.0; }
-        csrc[b + 0] = 1; cip[b + 0] = 0; cmp[b + 0] = 0; csc[b + 0] = 1.0;
-        csrc[b + 1] = 2; cip[b + 1] = 1; cmp[b + 1] = 1; csc[b + 1] = -1.0;
-        csrc[b + 2] = 2; cip[b + 2] = 0; cmp[b + 2] = 0; csc[b + 2] = -1.0;
-        csrc[b + 3] = 1; cip[b + 3] = 1; cmp[b + 3] = 1; csc[b + 3] = -1.0;
-    }
+    const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
+    const int lc = lev < a.nlev ? a.lcut[lev] : -1;
+    const bool lev_on = lev < a.nlev && m <= min(lc, a.m_max);
+    int lcm = -1;
+#pragma unroll
+    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, a.lcut[min(lev0 + i, a.nlev - 1)]);
+    const int nch = m <= min(lcm, a.m_max) ? (a.nh + 31) >> 5 : 0;
 
-    d4 acc[NOUT][2];
+    // F2[lev][comp][theta/8][m][theta%8]
+    const int levc = min(lev, a.nlev - 1);
+    const double2 *fin = reinterpret_cast<const double2 *>(job.fin) + (size_t)levc * a.fin_ld;
+    const size_t cstride = (size_t)((a.n_theta + 7) / 8) * a.n_m * 8;
+    double2 xn[NP], xs[NP];
+    auto load = [&](int c) {
+        const int th = min(32 * c + j, a.nh - 1);
+        const double2 *f = fin + ((size_t)(th >> 2) * a.n_m + mc) * 8 + (2 * th & 7);
 #pragma unroll
-    for (int o = 0; o < NOUT; ++o)
-        for (int s = 0; s < 2; ++s) acc[o][s] = d4{0.0, 0.0, 0.0, 0.0};
-
-    const int nchunk = (a.nq4 + KQC - 1) / KQC;
-    for (int c = 0; c < nchunk; ++c) {
-        __syncthreads();
-        for (int idx = threadIdx.x; idx < CHUNK * LEV_GROUP; idx += WG) {
-            int levl = idx % LEV_GROUP;
-            int thl = idx / LEV_GROUP;
-            int th = c * CHUNK + thl;
-            int lev = lev0 + levl;
-            bool valid = (levl < nlev_here) && (th < a.nh);
-            if (valid) {
-                int lc = job.lcut[lev];
-                int mlim = lc < a.m_max ? lc : a.m_max;
-                valid = m <= mlim;
-            }
-            double nr[3], ni[3], sr[3], si[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) { nr[k] = ni[k] = sr[k] = si[k] = 0.0; }
-            if (valid) {
-                int nsrc = (KIND == ANA_SH) ? 1 : 3;
-                for (int k = 0; k < nsrc; ++k) {
-                    int comp = job.in_comp[k];
-                    if (comp < 0) continue;
-                    size_t o = ((size_t)lev * job.fin_ld + ((size_t)comp * a.n_theta + 2 * th) * a.n_m + mc) * 2;
-                    size_t o2 = o + (size_t)a.n_m * 2;
-                    nr[k] = job.fin[o];
-                    ni[k] = job.fin[o + 1];
-                    sr[k] = job.fin[o2];
-                    si[k] = job.fin[o2 + 1];
-                }
-            }
-#pragma unroll
-            for (int col = 0; col < NCOL; ++col) {
-                int k = csrc[col];
-                double syr = nr[k] + sr[k], syi = ni[k] + si[k];
-                double anr = nr[k] - sr[k], ani = ni[k] - si[k];
-                apply_factor(syr, syi, cip[col], cmp[col], dm, csc[col]);
-                apply_factor(anr, ani, cip[col], cmp[col], dm, csc[col]);
-                double *b0 = smem + (((col * 2 + 0) * CHUNK + thl) * 16 + levl * 2);
-                double *b1 = smem + (((col * 2 + 1) * CHUNK + thl) * 16 + levl * 2);
-                b0[0] = syr; b0[1] = syi;
-                b1[0] = anr; b1[1] = ani;
-            }
+        for (int k = 0; k < NP; ++k) {
+            xn[k] = f[(size_t)job.in_comp[k] * cstride];
+            xs[k] = f[(size_t)job.in_comp[k] * cstride + 1];
         }
-        __syncthreads();
-        if (active) {
-            int nq = min(KQC, a.nq4 - c * KQC);
-            for (int q = 0; q < nq; ++q) {
-                size_t tq = (size_t)(c * KQC + q);
+    };
+    auto build = [&](int c, int buf) {
+        const bool ok = lev_on && 32 * c + j < a.nh;
+        double *b = sB + buf * BUF + (j >> 3) * AB_PAIR + ((j & 3) * 16 + 2 * lv) * 2 + ((j >> 2) & 1);
 #pragma unroll
-                for (int par = 0; par < 2; ++par) {
-                    size_t o = a.off[2 * mc + par] + ((size_t)t * a.nq4 + tq) * 64 + lane;
-                    double aP = a.aP[o];
-                    double adP = a.adP[o];
+        for (int k = 0; k < NP; ++k) {
+            const double2 n = ok ? xn[k] : make_double2(0.0, 0.0), so = ok ? xs[k] : make_double2(0.0, 0.0);
+            double *b0 = b + k * AB_COL, *b1 = b0 + AB_SA;
+            b0[0] = n.x + so.x;
+            b0[2] = n.y + so.y;
+            b1[0] = n.x - so.x;
+            b1[2] = n.y - so.y;
+        }
+    };
+
+    d4 acc[TPW][NP];
 #pragma unroll
-                    for (int pr = 0; pr < NPROD; ++pr) {
-                        const Prod P = S::prod[pr];
-                        // even rows: P uses the symmetric combination, dP the antisymmetric
-                        int use = (P.tab == 0) ? par : (1 - par);
-                        double b = smem[((P.col * 2 + use) * CHUNK + q * 4 + (lane >> 4)) * 16 + (lane & 15)];
-                        acc[P.acc][par] = mfma64(P.tab == 0 ? aP : adP, b, acc[P.acc][par]);
+    for (int s = 0; s < TPW; ++s)
+#pragma unroll
+        for (int k = 0; k < NP; ++k) acc[s][k] = d4{0.0, 0.0, 0.0, 0.0};
+    const double2 *tab = reinterpret_cast<const double2 *>(a.tab + a.off[2 * mc + par]) + lane;
+    const int nmine = t0 < nt ? min(TPW, (nt - t0 + 1) >> 1) : 0;  // tiles of this wave
+    const int npair = a.nq8;
+    auto load_A = [&](double2 *f, int p) {
+        const double2 *t = tab + (size_t)min(p, npair - 1) * 64;
+#pragma unroll
+        for (int s = 0; s < TPW; ++s)
+            if (s < nmine) f[s] = t[(size_t)(t0 + 2 * s) * (npair * 64)];
+    };
+    double2 fa[2][TPW];
+
+    if (nch > 0) {
+        load(0);
+        load_A(fa[0], 0);
+        build(0, 0);
+    }
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        const int buf = c & 1;
+        if (c + 1 < nch) load(c + 1);
+        if (nmine > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int p = 4 * c + k;
+                load_A(fa[(k + 1) & 1], p + 1);
+                if (p < npair) {
+                    double2 b[NP];
+                    const double *sb = sB + buf * BUF + par * AB_SA + k * AB_PAIR + 2 * lane;
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) b[q] = *reinterpret_cast<const double2 *>(sb + q * AB_COL);
+#pragma unroll
+                    for (int s = 0; s < TPW; ++s) {
+                        if (s >= nmine) break;
+#pragma unroll
+                        for (int q = 0; q < NP; ++q) acc[s][q] = mfma64(fa[k & 1][s].x, b[q].x, acc[s][q]);
+#pragma unroll
+                        for (int q = 0; q < NP; ++q) acc[s][q] = mfma64(fa[k & 1][s].y, b[q].y, acc[s][q]);
                     }
                 }
             }
         }
+        if (c + 1 < nch) build(c + 1, buf ^ 1);
+        __syncthreads();
     }
 
-    // epilogue: rows r -> l = m + par + 2 (16 t + r); transpose to 32
-    // consecutive l per level
-    __syncthreads();
-    double *ep = smem + wave * (LEV_GROUP * 32 * 2);
-    const int col = lane & 15, levl_c = col >> 1, ri = col & 1;
+    // epilogue through LDS: rows of consecutive l (both parities), then one
+    // (level, l) per thread and round, consecutive l by consecutive lanes
+    const int nrow = min(32 * 2 * TPW, L + 2 - m - 32 * zb);  // rows held: l = m + 32 zb + row
+    auto stage = [&](int area, int k) {
+        const int col = lane & 15;
 #pragma unroll
-    for (int o = 0; o < NOUT; ++o) {
-        if (active) {
+        for (int s = 0; s < TPW; ++s) {
+            if (s >= nmine) break;
 #pragma unroll
-            for (int par = 0; par < 2; ++par)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    int r = (lane >> 4) + 4 * j;
-                    int l = m + par + 2 * (16 * t + r);
-                    double v = acc[o][par][j];
-                    if (S::divll[o] && l > 0) v /= (double)l * (double)(l + 1);
-                    ep[(levl_c * 32 + 2 * r + par) * 2 + ri] = v;
-                }
+            for (int jj = 0; jj < 4; ++jj) {
+                const int row = 32 * (t0 + 2 * s - zb) + par + 2 * ((lane >> 4) + 4 * jj);
+                if (row < nrow) sB[area * a.erows * AE_ROW + row * AE_ROW + col] = acc[s][k][jj];
+            }
         }
+    };
+    auto at = [&](int area, int row) {
+        return *reinterpret_cast<const double2 *>(sB + area * a.erows * AE_ROW + row * AE_ROW + 2 * lv);
+    };
+    const int lo = gz > 0 ? 31 : 0;  // rows written: the one before the edge belongs to the workgroup before
+    const int zn = zb + 2 * TPW - 1;
+    const int hi = nt > zn + 1 ? 32 * (zn + 1 - zb) - 1 : L + 1 - m - 32 * zb;
+    double2 *const *outs = reinterpret_cast<double2 *const *>(job.out);
+    const size_t o0 = (size_t)lev * a.out_ld + (size_t)(l0 + 32 * zb);
+    auto kept = [&](int l) { return lev_on && l <= lc; };
+    if constexpr (KIND != ANA_SH) {
+        stage(0, NP - 2);  // G of vt
+        stage(1, NP - 1);  // G of vp
         __syncthreads();
-        if (active) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                int e = rr * 64 + lane;
-                int levl = e >> 5, ll = e & 31;
-                int l = m + 32 * t + ll;
-                if (levl < nlev_here && l <= a.l_max) {
-                    int lev = lev0 + levl;
-                    int lc = job.lcut[lev];
-                    bool keep = (l <= lc) && (m <= (lc < a.m_max ? lc : a.m_max));
-                    double2 v = keep ? make_double2(ep[(levl * 32 + ll) * 2], ep[(levl * 32 + ll) * 2 + 1])
-                                     : make_double2(0.0, 0.0);
-                    size_t o2 = ((size_t)lev * job.out_ld + (size_t)(l0 + l - m)) * 2;
-                    *reinterpret_cast<double2 *>(job.out[o] + o2) = v;
-                }
+        double2 *oS = outs[NP - 2], *oT = outs[NP - 1];
+        for (int row = lo + ((j - lo) & 31); row < hi; row += 32) {
+            const int l = m + 32 * zb + row;
+            const double dl = (double)l;
+            const double *cr = a.crec + l0 + 2 * mc + l - m;
+            const double fp = dl * cr[1], fm = (dl + 1.0) * cr[0];
+            const double2 z = make_double2(0.0, 0.0);
+            const double2 tm = row > 0 ? at(0, row - 1) : z, tp = at(0, row + 1), tc = at(0, row);
+            const double2 pm = row > 0 ? at(1, row - 1) : z, pp = at(1, row + 1), pc = at(1, row);
+            const double rl = dl * (dl + 1.0);
+            // S = (dP vt - i m P vp) / l(l+1), T = (-dP vp - i m P vt) / l(l+1)
+            double2 S = make_double2(fp * tp.x - fm * tm.x + dm * pc.y, fp * tp.y - fm * tm.y - dm * pc.x);
+            double2 T = make_double2(fm * pm.x - fp * pp.x + dm * tc.y, fm * pm.y - fp * pp.y - dm * tc.x);
+            if (l > 0) {
+                S = make_double2(S.x / rl, S.y / rl);
+                T = make_double2(T.x / rl, T.y / rl);
+            }
+            if (lev < a.nlev) {
+                oS[o0 + row] = kept(l) ? S : z;
+                oT[o0 + row] = kept(l) ? T : z;
             }
         }
         __syncthreads();
+    }
+    if constexpr (KIND != ANA_SPHTOR) {
+        stage(0, 0);
+        __syncthreads();
+        for (int row = lo + ((j - lo) & 31); row < hi; row += 32)
+            if (lev < a.nlev) outs[0][o0 + row] = kept(m + 32 * zb + row) ? at(0, row) : make_double2(0.0, 0.0);
+    }
+}
+
+// the jobs of one launch: kinds of at most NP columns; blocks ordered as the
+// synthesis'
+template <int TPW, int NP>
+__global__ __launch_bounds__(WG, 2) void k_ana(AnaArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) double sB[];
+    const int inner = a.njob * a.gz * a.ng;
+    const int mc = (int)(blockIdx.x >> 3) / inner * 8 + (int)(blockIdx.x & 7);
+    if (mc >= a.n_m) return;
+    int r = (int)(blockIdx.x >> 3) % inner;
+    const AnaJob &job = a.job[r % a.njob];
+    r /= a.njob;
+    const int gz = r % a.gz, lev0 = r / a.gz * LEV_GROUP;
+    switch (job.kind) {
+    case ANA_SH: ana_body<TPW, ANA_SH>(a, job, mc, lev0, gz, sB); break;
+    case ANA_SPHTOR: if constexpr (NP > 1) ana_body<TPW, ANA_SPHTOR>(a, job, mc, lev0, gz, sB); break;
+    case ANA_QST: if constexpr (NP > 2) ana_body<TPW, ANA_QST>(a, job, mc, lev0, gz, sB); break;
+    default: break;
+    }
+}
+
+template <int TPW, int NP>
+int launch_ana_t(const AnaArgs &a, unsigned grid, hipStream_t s)
+{
+    // the two B buffers, reused by the epilogue's areas (vt and vp; f alone
+    // in a scalar launch)
+    const size_t shm = std::max((size_t)2 * NP * AB_COL, (size_t)(NP > 1 ? 2 : 1) * a.erows * AE_ROW) * sizeof(double);
+    // set once per kernel and raised only, so that a call under graph capture
+    // makes no attribute call
+    static int shm_set = 0;
+    if (shm > 64 * 1024 && (int)shm > shm_set) {
+        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_ana<TPW, NP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)shm));
+        shm_set = (int)shm;
+    }
+    k_ana<TPW, NP><<<grid, WG, shm, s>>>(a);
+    MHX_HIP_CHECK(hipGetLastError());
+    return MHX_OK;
+}
+
+template <int NP>
+int launch_ana_np(const AnaArgs &a, int tpw, unsigned grid, hipStream_t s)
+{
+    switch (tpw) {
+    case 1: return launch_ana_t<1, NP>(a, grid, s);
+    case 3: return launch_ana_t<3, NP>(a, grid, s);
+    default: return launch_ana_t<5, NP>(a, grid, s);
     }
 }
 
@@ -562,15 +594,30 @@ int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, h
     }
 }
 
-int launch_ana(const Plan *p, const AnaJob &job, hipStream_t s)
+int launch_ana(const Plan *p, const AnaJob *jobs, int njob, const AnaBatch &b, hipStream_t s)
 {
-    if (int rc = ensure_fp64_tables(const_cast<Plan *>(p))) return rc;
-    if (job.nlev <= 0) return MHX_OK;
+    if (b.nlev <= 0 || njob <= 0) return MHX_OK;
+    if (njob > MAX_ANA_JOBS) return fail(MHX_E_INVALID, "too many analysis jobs in one launch");
+    if (int rc = ensure_p_tables(const_cast<Plan *>(p))) return rc;
     AnaArgs a;
-    a.job = job;
-    a.aP = p->d_ana_wP;
-    a.adP = p->d_ana_wdP;
-    a.off = p->d_ana_off;
+    int np = 0;
+    for (int i = 0; i < njob; ++i) {
+        a.job[i] = jobs[i];
+        switch (jobs[i].kind) {
+        case ANA_SH: np = np < 1 ? 1 : np; break;
+        case ANA_SPHTOR: np = np < 2 ? 2 : np; break;
+        case ANA_QST: np = 3; break;
+        default: return fail(MHX_E_INVALID, "unknown analysis kind");
+        }
+    }
+    a.njob = njob;
+    a.nlev = b.nlev;
+    a.fin_ld = b.fin_ld;
+    a.out_ld = b.out_ld;
+    a.lcut = b.lcut;
+    a.tab = p->d_anax;
+    a.off = p->d_anax_off;
+    a.crec = p->d_crec64;
     a.lstart = p->d_lstart;
     a.l_max = p->l_max;
     a.m_max = p->m_max;
@@ -578,17 +625,20 @@ int launch_ana(const Plan *p, const AnaJob &job, hipStream_t s)
     a.n_m = p->n_m;
     a.nh = p->nh;
     a.n_theta = p->n_theta;
-    a.nq4 = p->nq4;
-    int ntile0 = ((p->l_max) / 2 + 1 + 15) / 16;  // pair tiles at m = 0
-    dim3 grid((unsigned)(p->n_m * ((job.nlev + LEV_GROUP - 1) / LEV_GROUP) * ((ntile0 + 3) / 4)));
-    switch (job.kind) {
-    case ANA_SH: k_ana<ANA_SH><<<grid, WG, 0, s>>>(a); break;
-    case ANA_SPHTOR: k_ana<ANA_SPHTOR><<<grid, WG, 0, s>>>(a); break;
-    case ANA_QST: k_ana<ANA_QST><<<grid, WG, 0, s>>>(a); break;
-    default: return fail(MHX_E_INVALID, "unknown analysis kind");
+    a.nq8 = (p->nh + 7) / 8;
+    a.ng = (b.nlev + LEV_GROUP - 1) / LEV_GROUP;
+    // tiles per wave: all of m = 0's tile pairs in one workgroup where five
+    // per wave hold them (120 accumulator registers), else groups of ten
+    const int nt = (p->l_max + 2 + 31) / 32;
+    const int tpw = nt <= 2 ? 1 : (nt <= 6 ? 3 : 5);
+    a.erows = std::min(64 * tpw, p->l_max + 2);
+    a.gz = nt <= 2 * tpw ? 1 : (nt - 1 + 2 * tpw - 2) / (2 * tpw - 1);
+    const unsigned grid = (unsigned)((p->n_m + 7) / 8 * 8 * njob * a.ng * a.gz);
+    switch (np) {
+    case 1: return launch_ana_np<1>(a, tpw, grid, s);
+    case 2: return launch_ana_np<2>(a, tpw, grid, s);
+    default: return launch_ana_np<3>(a, tpw, grid, s);
     }
-    MHX_HIP_CHECK(hipGetLastError());
-    return MHX_OK;
 }
 
 }  // namespace mhx

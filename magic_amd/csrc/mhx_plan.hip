@@ -189,27 +189,32 @@ int ifft_to(Plan *p, int comp0, int ncomp, int nlev, double *const *dst, size_t 
 int fft_from(Plan *p, int ncomp, int nlev, const double *const *src, size_t ld_grid,
              const bool *osin2)
 {
-    size_t Fld = (size_t)10 * p->n_m * p->n_theta;
+    const size_t comp = f2_comp(p->n_m, p->n_theta);
     for (int c = 0; c < ncomp; ++c) {
-        double *F = p->ws_F2 + (size_t)c * p->n_m * p->n_theta * 2;
-        int rc = launch_fft(p, src[c], ld_grid, 0, 1, nlev, osin2[c] ? 1u : 0u, F, Fld, p->stream);
+        double *F = p->ws_F2 + c * comp * 2;
+        int rc = launch_fft(p, src[c], ld_grid, 0, 1, nlev, osin2[c] ? 1u : 0u, F, 10 * comp, p->stream);
         if (rc) return rc;
     }
     return MHX_OK;
 }
 
-AnaJob ana_job(Plan *p, int kind, int nlev, size_t out_ld)
+// an analysis job of comps comp0, comp0 + 1, ... of ws_F2
+AnaJob ana_job(Plan *p, int kind, double *o0, double *o1 = nullptr, double *o2 = nullptr, int comp0 = 0)
 {
     AnaJob j;
-    std::memset(&j, 0, sizeof(j));
     j.kind = kind;
-    j.nlev = nlev;
     j.fin = p->ws_F2;
-    j.fin_ld = (size_t)10 * p->n_m * p->n_theta;
-    j.in_comp[0] = j.in_comp[1] = j.in_comp[2] = -1;
-    j.out_ld = out_ld;
-    j.lcut = p->d_lcut;
+    for (int i = 0; i < 3; ++i) j.in_comp[i] = comp0 + i;
+    j.out[0] = o0;
+    j.out[1] = o1;
+    j.out[2] = o2;
     return j;
+}
+
+// levels of the analysis launches from ws_F2 (10 comps per level)
+AnaBatch ana_batch(Plan *p, int nlev, size_t out_ld)
+{
+    return AnaBatch{nlev, 10 * f2_comp(p->n_m, p->n_theta), out_ld, p->d_lcut};
 }
 
 // ---- per-call helpers: grids staged through ws_G, coefficients through ws_C
@@ -265,19 +270,10 @@ int analysis_call(Plan *p, int kind, int ngrid, const double *const *grids, cons
         }
     }
     if ((rc = fft_from(p, ngrid, 1, src, 0, os))) return rc;
-    AnaJob j = ana_job(p, kind, 1, 0);
-    if (kind == ANA_SH) {
-        j.in_comp[0] = 0;
-    } else if (kind == ANA_SPHTOR) {
-        j.in_comp[1] = 0;
-        j.in_comp[2] = 1;
-    } else {
-        j.in_comp[0] = 0;
-        j.in_comp[1] = 1;
-        j.in_comp[2] = 2;
-    }
-    for (int c = 0; c < nout; ++c) j.out[c] = p->ws_C + (size_t)(4 + c) * p->lm_max * 2;
-    if ((rc = launch_ana(p, j, p->stream))) return rc;
+    double *o[3] = {};
+    for (int c = 0; c < nout; ++c) o[c] = p->ws_C + (size_t)(4 + c) * p->lm_max * 2;
+    const AnaJob j = ana_job(p, kind, o[0], o[1], o[2]);
+    if ((rc = launch_ana(p, &j, 1, ana_batch(p, 1, 0), p->stream))) return rc;
     return finish_coefs(p, nout, out);
 }
 
@@ -481,6 +477,8 @@ int mhx_plan_destroy(mhx_plan *h)
     free_dev(p->d_syn_off);
     free_dev(p->d_synx);
     free_dev(p->d_synx_off);
+    free_dev(p->d_anax);
+    free_dev(p->d_anax_off);
     free_dev(p->d_crec64);
     free_dev(p->d_ana_off);
     free_dev(p->d_osin2);
@@ -871,14 +869,8 @@ int mhx_spat_to_qst_batch(mhx_plan *h, int nlev, const double *f, const double *
     const double *src[3] = {f, g, hh};
     bool os[3] = {false, true, true};
     if ((rc = fft_from(P, 3, nlev, src, ld_grid, os))) return rc;
-    AnaJob j = ana_job(P, ANA_QST, nlev, ld_lm);
-    j.in_comp[0] = 0;
-    j.in_comp[1] = 1;
-    j.in_comp[2] = 2;
-    j.out[0] = q;
-    j.out[1] = s;
-    j.out[2] = t;
-    if ((rc = launch_ana(P, j, P->stream))) return rc;
+    const AnaJob j = ana_job(P, ANA_QST, q, s, t);
+    if ((rc = launch_ana(P, &j, 1, ana_batch(P, nlev, ld_lm), P->stream))) return rc;
     MHX_HIP_CHECK(hipStreamSynchronize(P->stream));
     return MHX_OK;
 }
@@ -1155,24 +1147,14 @@ static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t l
                                                  grids, s)) ||
                            (rc2 = mark())))
                 return rc2;
-            if ((rc2 = fork())) return rc2;
-            for (int v = 0; v < 3; ++v) {
-                AnaJob j = ana_job(P, ANA_QST, nlev, ld_lm);
-                j.in_comp[0] = 3 * v;
-                j.in_comp[1] = 3 * v + 1;
-                j.in_comp[2] = 3 * v + 2;
-                j.out[0] = dout[3 * v];
-                j.out[1] = dout[3 * v + 1];
-                j.out[2] = dout[3 * v + 2];
-                if ((rc2 = launch_ana(P, j, on(v))) || (rc2 = mark())) return rc2;
-            }
-            {
-                AnaJob j = ana_job(P, ANA_SH, nlev, ld_lm);
-                j.in_comp[0] = 9;
-                j.out[0] = dout[9];
-                if ((rc2 = launch_ana(P, j, on(3))) || (rc2 = mark())) return rc2;
-            }
-            return join();
+            AnaJob anas[4];
+            for (int v = 0; v < 3; ++v) anas[v] = ana_job(P, ANA_QST, dout[3 * v], dout[3 * v + 1], dout[3 * v + 2], 3 * v);
+            anas[3] = ana_job(P, ANA_SH, dout[9], nullptr, nullptr, 9);
+            const AnaBatch ab = ana_batch(P, nlev, ld_lm);
+            if (!P->timing) return launch_ana(P, anas, 4, ab, s);
+            for (int v = 0; v < 4; ++v)
+                if ((rc2 = launch_ana(P, anas + v, 1, ab, s)) || (rc2 = mark())) return rc2;
+            return MHX_OK;
         };
         auto launch_all = [&]() -> int {
             if (P->cour.max) {

@@ -425,7 +425,7 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
     const size_t four = (size_t)P->n_m * P->n_theta * 2;  // doubles per Fourier comp
     const size_t lmd = (size_t)nlev * ld_lm * 2;           // doubles per nl array
     if ((rc = grow(B->F, B->nF, (size_t)nlev * nin * four)) ||
-        (rc = grow(B->F2, B->nF2, (size_t)nlev * nout * four)) ||
+        (rc = grow(B->F2, B->nF2, (size_t)nlev * nout * 2 * f2_comp(P->n_m, P->n_theta))) ||
         (rc = grow(B->nl, B->nnl, (size_t)NL_N * lmd)) ||
         (rc = grow(B->rad, B->nrad, (size_t)(RL_NRAD + TR_NRAD + 2) * nlev)))
         return rc;
@@ -554,27 +554,6 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
         j.out_comp[2] = c2;
         return j;
     };
-    // independent launches (the analyses) dealt over the plan's branch
-    // streams, forked from and joined back into s
-    int nl_launch = 0;
-    auto on = [&]() -> hipStream_t {
-        const int i = nl_launch++ % P->nbranch;
-        return i == 0 ? s : P->br[i - 1];
-    };
-    auto fork = [&]() -> int {
-        nl_launch = 0;
-        if (P->nbranch < 2) return MHX_OK;
-        MHX_HIP_CHECK(hipEventRecord(P->ev_fork, s));
-        for (int i = 0; i + 1 < P->nbranch; ++i) MHX_HIP_CHECK(hipStreamWaitEvent(P->br[i], P->ev_fork, 0));
-        return MHX_OK;
-    };
-    auto join = [&]() -> int {
-        for (int i = 0; i + 1 < P->nbranch; ++i) {
-            MHX_HIP_CHECK(hipEventRecord(P->ev_join[i], P->br[i]));
-            MHX_HIP_CHECK(hipStreamWaitEvent(s, P->ev_join[i], 0));
-        }
-        return MHX_OK;
-    };
     const ColOp none = ColOp();
     auto torpol = [&](int a, int b, int c, int comp) {
         add(SYN_QST, rop(din[a], G_LL), rop(din[b]), rop(din[c]), in_of[comp], in_of[comp + 1], in_of[comp + 2]);
@@ -661,40 +640,28 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
     // ---- analysis ----
     double *nl[NL_N];
     for (int k = 0; k < NL_N; ++k) nl[k] = B->nl + (size_t)k * lmd;
-    auto ana = [&](int kind, int c0, double *o0, double *o1, double *o2, size_t ld) -> int {
-        AnaJob j;
-        std::memset(&j, 0, sizeof(j));
+    AnaJob anas[MAX_ANA_JOBS];
+    int nana = 0;
+    auto ana = [&](int kind, int c0, double *o0, double *o1 = nullptr, double *o2 = nullptr) {
+        AnaJob &j = anas[nana++];
         j.kind = kind;
-        j.nlev = nlev;
         j.fin = B->F2;
-        j.fin_ld = (size_t)nout * P->n_m * P->n_theta;
-        if (kind == ANA_SH) {
-            j.in_comp[0] = c0;
-            j.in_comp[1] = j.in_comp[2] = -1;
-        } else {
-            j.in_comp[0] = c0;
-            j.in_comp[1] = c0 + 1;
-            j.in_comp[2] = c0 + 2;
-        }
+        for (int i = 0; i < 3; ++i) j.in_comp[i] = c0 + i;
         j.out[0] = o0;
         j.out[1] = o1;
         j.out[2] = o2;
-        j.out_ld = ld;
-        j.lcut = B->lcut;
-        return launch_ana(P, j, on());
     };
-    if ((rc = fork())) return rc;
     // the nonlinear_lm_t arrays live in nl[] with the caller's level stride
     // ld_lm, so that the outputs the reference writes straight from the
     // analysis (dVSrLM, dVXirLM, dphidt) share a launch with them
-    if (adv && (rc = ana(ANA_QST, out_of[RO_ADVR], nl[NL_ADVR], nl[NL_ADVT], nl[NL_ADVP], ld_lm))) return rc;
-    if (heat && (rc = ana(ANA_QST, out_of[RO_VSR], dout[4], nl[NL_VST], nl[NL_VSP], ld_lm))) return rc;
-    if (chem && (rc = ana(ANA_QST, out_of[RO_VXIR], dout[6], nl[NL_VXIT], nl[NL_VXIP], ld_lm))) return rc;
-    if (ph->l_mag_nl && (rc = ana(ANA_QST, out_of[RO_VXBR], nl[NL_VXBR], nl[NL_VXBT], nl[NL_VXBP], ld_lm)))
-        return rc;
-    if (anel && (rc = ana(ANA_SH, out_of[RO_HEAT], nl[NL_HEAT], nullptr, nullptr, ld_lm))) return rc;
-    if (phase && (rc = ana(ANA_SH, out_of[RO_PHI], dout[7], nullptr, nullptr, ld_lm))) return rc;
-    if ((rc = join())) return rc;
+    if (adv) ana(ANA_QST, out_of[RO_ADVR], nl[NL_ADVR], nl[NL_ADVT], nl[NL_ADVP]);
+    if (heat) ana(ANA_QST, out_of[RO_VSR], dout[4], nl[NL_VST], nl[NL_VSP]);
+    if (chem) ana(ANA_QST, out_of[RO_VXIR], dout[6], nl[NL_VXIT], nl[NL_VXIP]);
+    if (ph->l_mag_nl) ana(ANA_QST, out_of[RO_VXBR], nl[NL_VXBR], nl[NL_VXBT], nl[NL_VXBP]);
+    if (anel) ana(ANA_SH, out_of[RO_HEAT], nl[NL_HEAT]);
+    if (phase) ana(ANA_SH, out_of[RO_PHI], dout[7]);
+    const AnaBatch ab{nlev, (size_t)nout * f2_comp(P->n_m, P->n_theta), ld_lm, B->lcut};
+    if ((rc = launch_ana(P, anas, nana, ab, s))) return rc;
 
     // ---- lm-space assembly ----
     RlTdArgs t;

@@ -12,9 +12,10 @@
 //   analysis   (MFMA A operand 16 l x 4 theta):
 //     ana[ana_off[2mc+p] + ((kk/16) * nq4 + th/4) * 64 + (kk%16) + 16*(th%4)]
 // where th is the northern-hemisphere theta index.  Padding entries are 0.
-//   FP64 kernels' synthesis table, l <= l_max + 1 (two K quads per lane, so
-//   that a fragment load is 16 bytes per lane):
+//   FP64 kernels' tables, l <= l_max + 1 (two K quads per lane, so that a
+//   fragment load is 16 bytes per lane; P, and 2 pi w P):
 //     synx[synx_off[2mc+p] + ((kk/8) * nt16 + th/16) * 128 + ((th%16) + 16*(kk%4)) * 2 + (kk/4)%2]
+//     anax[anax_off[2mc+p] + ((kk/16) * nq8 + th/8) * 128 + ((kk%16) + 16*(th%4)) * 2 + (th/4)%2]
 #include "mhx_internal.h"
 
 #include <cmath>
@@ -98,25 +99,31 @@ __global__ void k_plm_tables(int l_max, int minc, int n_m, int nh, int nt16, int
         size_t ao = ana_off[2 * mc + par] + ((size_t)(kk >> 4) * nq4 + (th >> 2)) * 64 + (kk & 15) + 16 * (th & 3);
         sP[so] = Pl;
         sdP[so] = dPl;
-        aP[ao] = w * Pl;
-        adP[ao] = w * dPl;
+        if (aP) {
+            aP[ao] = w * Pl;
+            adP[ao] = w * dPl;
+        }
     });
 }
 
 // the FP64 kernels' tables: the same recurrence up to l_max + 1, P only
-__global__ void k_p_tables(int l_max, int minc, int n_m, int nh, int nt16,
-                           const double *__restrict__ theta, const size_t *__restrict__ synx_off,
-                           double *__restrict__ synx)
+__global__ void k_p_tables(int l_max, int minc, int n_m, int nh, int nt16, int nq8,
+                           const double *__restrict__ theta, const double *__restrict__ gauss,
+                           const size_t *__restrict__ synx_off, const size_t *__restrict__ anax_off,
+                           double *__restrict__ synx, double *__restrict__ anax)
 {
     int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= n_m * nh) return;
     int mc = idx / nh, th = idx - mc * nh;
     int m = mc * minc;
     double t = theta[th];
+    const double w = 6.283185307179586 * gauss[th];
     plm_sweep(l_max + 1, m, sin(t), cos(t), [&](int l, double Pl, double) {
         int par = (l - m) & 1, kk = (l - m) >> 1;
         synx[synx_off[2 * mc + par] + ((size_t)(kk >> 3) * nt16 + (th >> 4)) * 128 +
              ((th & 15) + 16 * (kk & 3)) * 2 + ((kk >> 2) & 1)] = Pl;
+        anax[anax_off[2 * mc + par] + ((size_t)(kk >> 4) * nq8 + (th >> 3)) * 128 +
+             ((kk & 15) + 16 * (th & 3)) * 2 + ((th >> 2) & 1)] = w * Pl;
     });
 }
 
@@ -237,12 +244,16 @@ int build_tables(Plan *p)
     const size_t so = p->syn_size, ao = p->ana_size;
     MHX_HIP_CHECK(hipMalloc(&p->d_syn_P, so * sizeof(double)));
     MHX_HIP_CHECK(hipMalloc(&p->d_syn_dP, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMalloc(&p->d_ana_wP, ao * sizeof(double)));
-    MHX_HIP_CHECK(hipMalloc(&p->d_ana_wdP, ao * sizeof(double)));
     MHX_HIP_CHECK(hipMemset(p->d_syn_P, 0, so * sizeof(double)));
     MHX_HIP_CHECK(hipMemset(p->d_syn_dP, 0, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(p->d_ana_wP, 0, ao * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(p->d_ana_wdP, 0, ao * sizeof(double)));
+    // the analysis pair feeds the split tables only (the FP64 kernels read
+    // the P-only tables)
+    if (p->precision == MHX_PREC_SPLIT16 && !p->rec) {
+        MHX_HIP_CHECK(hipMalloc(&p->d_ana_wP, ao * sizeof(double)));
+        MHX_HIP_CHECK(hipMalloc(&p->d_ana_wdP, ao * sizeof(double)));
+        MHX_HIP_CHECK(hipMemset(p->d_ana_wP, 0, ao * sizeof(double)));
+        MHX_HIP_CHECK(hipMemset(p->d_ana_wdP, 0, ao * sizeof(double)));
+    }
     int n = p->n_m * nh;
     k_plm_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, nh, p->nt16, p->nq4,
                                            p->d_theta, p->d_gauss, p->d_syn_off, p->d_ana_off,
@@ -256,26 +267,37 @@ int ensure_p_tables(Plan *p)
 {
     if (p->d_synx) return MHX_OK;
     if (int rc = ensure_fp64_tables(p)) return rc;
-    std::vector<size_t> so(2 * (size_t)p->n_m);
-    size_t ns = 0, nc = 0;
+    const int nq8 = (p->nh + 7) / 8;
+    std::vector<size_t> so(2 * (size_t)p->n_m), ao(2 * (size_t)p->n_m);
+    size_t ns = 0, na = 0, nc = 0;
     for (int mc = 0; mc < p->n_m; ++mc) {
         const int nrow = p->l_max + 2 - mc * p->minc;
         const int K[2] = {(nrow + 1) / 2, nrow / 2};
         for (int par = 0; par < 2; ++par) {
             so[2 * mc + par] = ns;
             ns += (size_t)((K[par] + 7) / 8) * p->nt16 * 128;
+            ao[2 * mc + par] = na;
+            na += (size_t)((K[0] + 15) / 16) * nq8 * 128;  // pair tiles: both parities use K[0]'s count
         }
         nc = (size_t)p->lstart[mc] + 2 * mc + nrow + 1;
     }
+    auto alloc = [&](auto *&dst, size_t n) -> int {
+        if (!dst) MHX_HIP_CHECK(hipMalloc(&dst, n * sizeof(*dst)));
+        return MHX_OK;
+    };
     double *synx = nullptr;
-    if (!p->d_synx_off) MHX_HIP_CHECK(hipMalloc(&p->d_synx_off, so.size() * sizeof(size_t)));
-    if (!p->d_crec64) MHX_HIP_CHECK(hipMalloc(&p->d_crec64, nc * sizeof(double)));
-    MHX_HIP_CHECK(hipMemcpy(p->d_synx_off, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
-    MHX_HIP_CHECK(hipMalloc(&synx, ns * sizeof(double)));
+    int rc;
+    if ((rc = alloc(p->d_synx_off, so.size())) || (rc = alloc(p->d_anax_off, ao.size())) ||
+        (rc = alloc(p->d_crec64, nc)) || (rc = alloc(p->d_anax, na)) || (rc = alloc(synx, ns)))
+        return rc;
     p->d_synx = synx;
-    MHX_HIP_CHECK(hipMemset(synx, 0, ns * sizeof(double)));
+    MHX_HIP_CHECK(hipMemcpy(p->d_synx_off, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMemcpy(p->d_anax_off, ao.data(), ao.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMemset(p->d_synx, 0, ns * sizeof(double)));
+    MHX_HIP_CHECK(hipMemset(p->d_anax, 0, na * sizeof(double)));
     const int n = p->n_m * p->nh;
-    k_p_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, p->nh, p->nt16, p->d_theta, p->d_synx_off, synx);
+    k_p_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, p->nh, p->nt16, nq8, p->d_theta, p->d_gauss,
+                                         p->d_synx_off, p->d_anax_off, p->d_synx, p->d_anax);
     k_crec64<<<dim3((unsigned)((p->l_max + 3 + 127) / 128), (unsigned)p->n_m), 128>>>(p->l_max, p->minc, p->d_lstart,
                                                                                       p->d_crec64);
     MHX_HIP_CHECK(hipGetLastError());
