@@ -97,7 +97,7 @@ struct AnaBatch {
 };
 
 // complex elements of one comp of the FP64 forward side F2 (theta in blocks of 8)
-inline size_t f2_comp(int n_m, int n_theta) { return (size_t)((n_theta + 7) / 8) * n_m * 8; }
+__host__ __device__ inline size_t f2_comp(int n_m, int n_theta) { return (size_t)((n_theta + 7) / 8) * n_m * 8; }
 
 // Legendre kernels of the nonlinear step in the split form (mhx_nlsplit.hip)
 // NS_S: the scalar alone (no gradient), split whole-K form only
@@ -256,6 +256,9 @@ struct Plan {
     double *d_tw = nullptr;         // M complex: exp(-2 pi i k/M)
     double *d_twr = nullptr;        // (M+1) complex: exp(-2 pi i k/n_phi)
     float *d_tw32 = nullptr, *d_twr32 = nullptr;  // the same in FP32
+    // factors of the wave FFTs (mhx_wavefft.h), where n_phi is a multiple of 64:
+    // exp(2 pi i a r / 64) [8][8], and exp(2 pi i j k / n_phi) [n_phi/64][64]
+    double *d_w64 = nullptr, *d_wn = nullptr;
     float *d_twn32 = nullptr;       // n_phi complex: exp(-2 pi i k/n_phi), FP32
     int grid_form = 0;              // grid stage of the split step: 0 tiles where supported, 1 slots
     // the nonlinear step's du/dr grids (synthesis of dw, ddw, dz and their
@@ -369,6 +372,24 @@ int launch_ifft(const Plan *p, const double *F, size_t F_ld_lev, int F_ncomp, in
 int launch_fft(const Plan *p, const double *grid, size_t grid_ld_lev, size_t grid_ld_comp,
                int ncomp, int nlev, unsigned osin2_mask, double *F, size_t F_ld_lev,
                hipStream_t s);
+// the same for up to three comps with a grid each in one launch
+// (mhx_rowfft.hip), where row_fft_supported
+struct RowFFT {
+    const double *F;        // inverse: F[lev][comp][m][theta]
+    double *F2;             // forward: F2[lev][comp][theta/8][m][theta%8]
+    size_t F_ld;            // complex elements per level
+    double *grid[3];        // inverse: grids
+    const double *src[3];   // forward: grids
+    size_t grid_ld;         // doubles per level
+    int ncomp;
+    unsigned osin2_mask;
+    // filled by the launcher
+    const double2 *w64, *wn;
+    const double *osin2;
+    int n_m, n_theta;
+};
+bool row_fft_supported(const Plan *p);
+int launch_row_fft(const Plan *p, const RowFFT &args, int nlev, bool inverse, hipStream_t s);
 // fused grid stage of the nonlinear step: Fin (18 comps per level) -> Fout
 // (10 comps per level); du/dr grids to dgrid [lev][3][theta][phi]; all 18
 // inverse grids in the reference layout to full_grids when not null

@@ -172,14 +172,23 @@ SynBatch syn_batch(Plan *p, int nlev, size_t src_ld)
     return SynBatch{nlev, src_ld, (size_t)18 * p->n_m * p->n_theta, p->d_lcut, p->d_rad};
 }
 
-// Fourier -> grid for ncomp comps starting at comp0 of ws_F into separate
-// destinations (level stride ld_grid doubles)
-int ifft_to(Plan *p, int comp0, int ncomp, int nlev, double *const *dst, size_t ld_grid)
+// Fourier comps [0, ncomp) of ws_F -> grids at separate destinations (level
+// stride ld_grid doubles)
+int ifft_to(Plan *p, int ncomp, int nlev, double *const *dst, size_t ld_grid)
 {
-    size_t Fld = (size_t)18 * p->n_m * p->n_theta;
+    const size_t comp = (size_t)p->n_m * p->n_theta;
+    if (row_fft_supported(p)) {
+        RowFFT a;
+        std::memset(&a, 0, sizeof(a));
+        a.F = p->ws_F;
+        a.F_ld = 18 * comp;
+        for (int c = 0; c < ncomp; ++c) a.grid[c] = dst[c];
+        a.grid_ld = ld_grid;
+        a.ncomp = ncomp;
+        return launch_row_fft(p, a, nlev, true, p->stream);
+    }
     for (int c = 0; c < ncomp; ++c) {
-        const double *F = p->ws_F + (size_t)(comp0 + c) * p->n_m * p->n_theta * 2;
-        int rc = launch_ifft(p, F, Fld, 1, 1, nlev, dst[c], ld_grid, 0, p->stream);
+        int rc = launch_ifft(p, p->ws_F + c * comp * 2, 18 * comp, 1, 1, nlev, dst[c], ld_grid, 0, p->stream);
         if (rc) return rc;
     }
     return MHX_OK;
@@ -190,6 +199,19 @@ int fft_from(Plan *p, int ncomp, int nlev, const double *const *src, size_t ld_g
              const bool *osin2)
 {
     const size_t comp = f2_comp(p->n_m, p->n_theta);
+    if (row_fft_supported(p)) {
+        RowFFT a;
+        std::memset(&a, 0, sizeof(a));
+        a.F2 = p->ws_F2;
+        a.F_ld = 10 * comp;
+        for (int c = 0; c < ncomp; ++c) {
+            a.src[c] = src[c];
+            a.osin2_mask |= osin2[c] ? 1u << c : 0u;
+        }
+        a.grid_ld = ld_grid;
+        a.ncomp = ncomp;
+        return launch_row_fft(p, a, nlev, false, p->stream);
+    }
     for (int c = 0; c < ncomp; ++c) {
         double *F = p->ws_F2 + c * comp * 2;
         int rc = launch_fft(p, src[c], ld_grid, 0, 1, nlev, osin2[c] ? 1u : 0u, F, 10 * comp, p->stream);
@@ -248,7 +270,7 @@ int synth_call(Plan *p, const SynJob &j, int ncomp, int lcut, double or2, double
     if ((rc = launch_syn(p, &j, 1, syn_batch(p, 1, 0), p->stream))) return rc;
     double *dst[3] = {p->ws_G, p->ws_G + (size_t)p->n_phi * p->n_theta,
                       p->ws_G + (size_t)2 * p->n_phi * p->n_theta};
-    if ((rc = ifft_to(p, 0, ncomp, 1, dst, 0))) return rc;
+    if ((rc = ifft_to(p, ncomp, 1, dst, 0))) return rc;
     return finish_grids(p, ncomp, out);
 }
 
@@ -413,6 +435,15 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         twn32[2 * k] = (float)std::cos(2.0 * pi * k / n_phi);
         twn32[2 * k + 1] = (float)-std::sin(2.0 * pi * k / n_phi);
     }
+    std::vector<double> w64, wn;
+    if (n_phi % 64 == 0) {
+        auto root = [&](std::vector<double> &v, int k, int n) {
+            v.push_back(std::cos(2.0 * pi * k / n));
+            v.push_back(std::sin(2.0 * pi * k / n));
+        };
+        for (int k = 0; k < 64; ++k) root(w64, k / 8 * (k % 8), 64);
+        for (int k = 0; k < n_phi; ++k) root(wn, k / 64 * (k % 64), n_phi);
+    }
     {
         const char *gf = std::getenv("MHX_GRID_FORM");
         p->grid_form = (gf && std::strcmp(gf, "slots") == 0) ? 1 : 0;
@@ -423,7 +454,7 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         (rc = up(p->d_gauss, p->gauss)) || (rc = up(p->d_osin2, osin2)) ||
         (rc = up(p->d_tw, tw)) || (rc = up(p->d_twr, twr)) || (rc = up(d_lm2l, lm2l)) ||
         (rc = up(p->d_tw32, tw32)) || (rc = up(p->d_twr32, twr32)) || (rc = up(p->d_lm2m, lm2m)) ||
-        (rc = up(p->d_twn32, twn32))) {
+        (rc = up(p->d_twn32, twn32)) || (!wn.empty() && ((rc = up(p->d_w64, w64)) || (rc = up(p->d_wn, wn))))) {
         mhx_plan_destroy(h);
         return rc;
     }
@@ -491,6 +522,8 @@ int mhx_plan_destroy(mhx_plan *h)
     free_dev(p->d_tw32);
     free_dev(p->d_twr32);
     free_dev(p->d_twn32);
+    free_dev(p->d_w64);
+    free_dev(p->d_wn);
     free_dev(p->d_syn16_P);
     free_dev(p->d_syn16_dP);
     free_dev(p->d_ana16_P);
@@ -849,7 +882,7 @@ int mhx_torpol_to_spat_batch(mhx_plan *h, int nlev, const double *W, const doubl
     SynJob j = syn_job(P, SYN_QST, op(W, G_LL), op(dW), op(Z));
     if ((rc = launch_syn(P, &j, 1, syn_batch(P, nlev, ld_lm), P->stream))) return rc;
     double *dst[3] = {vr, vt, vp};
-    if ((rc = ifft_to(P, 0, 3, nlev, dst, ld_grid))) return rc;
+    if ((rc = ifft_to(P, 3, nlev, dst, ld_grid))) return rc;
     MHX_HIP_CHECK(hipStreamSynchronize(P->stream));
     return MHX_OK;
 }
