@@ -9,8 +9,9 @@
 // the unnormalised Hermitian synthesis using only the real parts of modes 0
 // and N/2 (src/fft.f90:386-398).
 //
-// Fourier layouts: the inverse side F[lev][comp][m][theta] (written in
-// contiguous theta runs by the synthesis), the forward side theta-blocked,
+// Fourier layouts: the inverse side F[lev][comp][m][theta] in FP32 and
+// theta-blocked, F[lev][comp][theta/8][m][theta%8], in FP64 (whole 128-byte
+// lines of the synthesis either way); the forward side theta-blocked,
 // F2[lev][comp][theta/TH][m][theta%TH] with TH = 8 in FP64 and 16 in FP32: the
 // analysis reads one 128-byte line per (comp, m, block); m < n_m, modes up to N/2 beyond n_m are zero (src/shtransforms.f90:224-232).
 #include "mhx_fftcore.h"
@@ -19,6 +20,20 @@ namespace mhx {
 
 namespace {
 
+// inverse side: F[lev][comp][theta/8][m][theta%8] in FP64, whose row gathers
+// along m then run through consecutive lines (with m the outer index they are
+// a multiple of 4 KB apart on common grids and fall on two of an XCD's 16 L2
+// channels), F[lev][comp][m][theta] in FP32; complex elements per comp, offset
+// of a row within it, and the distance of consecutive m
+template <typename T> __device__ __forceinline__ size_t f1_size(int n_theta, int n_m)
+{
+    return sizeof(T) == 8 ? f2_comp(n_m, n_theta) : (size_t)n_m * n_theta;
+}
+template <typename T> __device__ __forceinline__ size_t f1_row(int th, int n_m)
+{
+    return sizeof(T) == 8 ? (size_t)(th / 8) * n_m * 8 + th % 8 : (size_t)th;
+}
+template <typename T> __device__ __forceinline__ size_t f1_step(int n_theta) { return sizeof(T) == 8 ? 8 : n_theta; }
 // forward side: theta rows per block of F2, complex elements per comp, and the
 // index of (comp, theta, m)
 template <typename T> constexpr int f2_th() { return sizeof(T) == 4 ? 16 : 8; }
@@ -55,14 +70,13 @@ __global__ void k_ifft_rows(FFTArgs f, const T *__restrict__ F, size_t F_ld, int
     int nrows = min(TB, n_theta - th0);
     load_twiddles(s_tw, s_twr, f);
     __syncthreads();
-    // inverse-side Fourier layout F[lev][comp][m][theta]; one thread team
-    // per theta row for the pre-step
-    const C *F0 = reinterpret_cast<const C *>(F) + (size_t)lev * F_ld + (size_t)comp * n_m * n_theta + th0;
+    // one thread team per theta row for the pre-step
+    const C *F0 = reinterpret_cast<const C *>(F) + (size_t)lev * F_ld + comp * f1_size<T>(n_theta, n_m);
     {
         int per = blockDim.x / TB;  // threads per row
         int r = threadIdx.x / per, t = threadIdx.x % per;
         if (r < TB) {
-            if (r < nrows) irfft_pre(F0 + r, (size_t)n_theta, n_m, A + r * M, M, s_twr, t, per);
+            if (r < nrows) irfft_pre(F0 + f1_row<T>(th0 + r, n_m), f1_step<T>(n_theta), n_m, A + r * M, M, s_twr, t, per);
             else
                 for (int k = t; k < M; k += per) A[r * M + k] = mk<C>(T(0), T(0));
         }
@@ -165,8 +179,7 @@ __global__ void k_nl_fused(FFTArgs f, const T *__restrict__ Fin, T *__restrict__
     load_twiddles(s_tw, s_twr, f);
     __syncthreads();
 
-    const size_t rowsz = (size_t)n_m;                   // complex per forward row
-    const C *Fi = reinterpret_cast<const C *>(Fin) + (size_t)lev * 18 * n_theta * rowsz + th;
+    const C *Fi = reinterpret_cast<const C *>(Fin) + lev * 18 * f1_size<T>(n_theta, n_m) + f1_row<T>(th, n_m);
     C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * f2_size<T>(n_theta, n_m);
 
     T u[3][PMAX], adv[3][PMAX], bb[3][PMAX], vxb[3][PMAX], vs[3][PMAX], ugs[PMAX];
@@ -180,7 +193,7 @@ __global__ void k_nl_fused(FFTArgs f, const T *__restrict__ Fin, T *__restrict__
             int per = nthr / gn;
             int r = tid / per, t = tid % per;
             if (r < gn)
-                irfft_pre(Fi + (size_t)(c0 + g0 + r) * n_m * n_theta, (size_t)n_theta, n_m,
+                irfft_pre(Fi + (c0 + g0 + r) * f1_size<T>(n_theta, n_m), f1_step<T>(n_theta), n_m,
                           A + r * M, M, s_twr, t, per);
             __syncthreads();
             C *res = fft_pp(A, B, gn, f, s_tw, +1);
@@ -383,7 +396,8 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
     }
     __syncthreads();
 
-    const C *Fi = reinterpret_cast<const C *>(Fin) + (size_t)lev * 18 * n_theta * n_m + th;
+    const C *Fi = reinterpret_cast<const C *>(Fin) + lev * 18 * f1_size<T>(n_theta, n_m) + f1_row<T>(th, n_m);
+    const size_t fstep = f1_step<T>(n_theta);
     C *Fo = reinterpret_cast<C *>(Fout) + (size_t)lev * 10 * f2_size<T>(n_theta, n_m);
 
     T u[3][NPT], adv[3][NPT], vxb[3][NPT];
@@ -397,7 +411,7 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
         if (slot < 6 && (round != 2 || slot >= 3 || dgrid)) {
             C *z = rows + slot * MP;
             const int comp = round == 0 ? slot : (round == 1 ? 9 + slot : (slot < 3 ? 6 + slot : 12 + slot));
-            const C *X = Fi + (size_t)comp * n_m * n_theta;
+            const C *X = Fi + comp * f1_size<T>(n_theta, n_m);
             // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/N} (X_k - conj X_{M-k})
             if constexpr (FFT::P == 24) {
                 // M = 1536: the lane's k = t + i Q <= M/2 take NK = 13 steps;
@@ -410,8 +424,8 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
 #pragma unroll
                 for (int i = 0; i < NK; ++i) {
                     const int k = t + i * Q;
-                    xa[i] = X[(size_t)min(k, n_m - 1) * n_theta];
-                    xc[i] = X[(size_t)min(M - k, n_m - 1) * n_theta];
+                    xa[i] = X[min(k, n_m - 1) * fstep];
+                    xc[i] = X[min(M - k, n_m - 1) * fstep];
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -430,8 +444,8 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
                 }
             } else {
                 // pointers stepped by Q rows (no index products per step)
-                const size_t step = (size_t)Q * n_theta;
-                const C *xa = X + (size_t)t * n_theta, *xc = X + (size_t)(M - t) * n_theta;
+                const size_t step = Q * fstep;
+                const C *xa = X + t * fstep, *xc = X + (M - t) * fstep;
                 for (int k = t; k <= M / 2; k += Q, xa += step, xc -= step) {
                     const int k2 = M - k;
                     C a = (k < n_m) ? *xa : mk<C>(T(0), T(0));
@@ -783,14 +797,14 @@ __global__ __launch_bounds__(512) void k_rl_grid(FFTArgs f, RlGridArgs a)
     __syncthreads();
 
     // inverse FFTs, G rows at a time, into rows[0, nin)
-    const C *Fi = reinterpret_cast<const C *>(a.Fin) + (size_t)lev * a.nin * n_theta * n_m + th;
+    const C *Fi = reinterpret_cast<const C *>(a.Fin) + lev * a.nin * f1_size<double>(n_theta, n_m) + f1_row<double>(th, n_m);
     for (int g0 = 0; g0 < a.nin; g0 += a.G) {
         const int gn = min(a.G, a.nin - g0);
         const int per = nthr / gn;
         const int r = tid / per, t = tid - r * per;
         if (r < gn)
-            irfft_pre(Fi + (size_t)(g0 + r) * n_m * n_theta, (size_t)n_theta, n_m, rows + (size_t)(g0 + r) * M,
-                      M, s_twr, t, per);
+            irfft_pre(Fi + (g0 + r) * f1_size<double>(n_theta, n_m), f1_step<double>(n_theta), n_m,
+                      rows + (size_t)(g0 + r) * M, M, s_twr, t, per);
         __syncthreads();
         C *res = fft_pp(rows + (size_t)g0 * M, B, gn, f, s_tw, +1);
         if (res != rows + (size_t)g0 * M) {
@@ -853,16 +867,16 @@ __global__ __launch_bounds__(512) void k_rl_grid_s(FFTArgs f, RlGridArgs a)
     __syncthreads();
 
     // inverse FFTs of rows [0, nin), one slot per row
-    const C *Fi = reinterpret_cast<const C *>(a.Fin) + (size_t)lev * a.nin * n_theta * n_m + th;
+    const C *Fi = reinterpret_cast<const C *>(a.Fin) + lev * a.nin * f1_size<double>(n_theta, n_m) + f1_row<double>(th, n_m);
     if (act)
         for (int c = slot; c < a.nin; c += nslot) {
             C *z = rows + (size_t)c * MP;
-            const C *X = Fi + (size_t)c * n_m * n_theta;
+            const C *X = Fi + c * f1_size<double>(n_theta, n_m);
             // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/N} (X_k - conj X_{M-k})
             for (int k = t; k <= M / 2; k += Q) {
                 const int k2 = M - k;
-                C xa = k < n_m ? X[(size_t)k * n_theta] : mk<C>(0.0, 0.0);
-                C xc = k2 < n_m ? X[(size_t)k2 * n_theta] : mk<C>(0.0, 0.0);
+                C xa = k < n_m ? X[(size_t)k * 8] : mk<C>(0.0, 0.0);
+                C xc = k2 < n_m ? X[(size_t)k2 * 8] : mk<C>(0.0, 0.0);
                 if (k == 0) {
                     xa.y = 0.0;
                     xc.y = 0.0;
@@ -1101,6 +1115,7 @@ int launch_nl_fused(const Plan *p, int nlev, const void *Fin, void *Fout, const 
             return launch_grid_tile(p, nlev, Fin, Fout, rad, LFfac, dgrid, full_grids, s);
         return launch_fused_t<float>(p, nlev, Fin, Fout, rad, LFfac, dgrid, full_grids, s);
     }
+    if (grid_wave_supported(p)) return launch_grid_wave(p, nlev, Fin, Fout, rad, LFfac, dgrid, full_grids, s);
     return launch_fused_t<double>(p, nlev, Fin, Fout, rad, LFfac, dgrid, full_grids, s);
 }
 

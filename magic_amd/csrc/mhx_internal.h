@@ -65,7 +65,7 @@ constexpr int MAX_SYN_JOBS = 12;  // jobs of one synthesis launch
 struct SynJob {
     int kind;
     ColOp col[3];          // fields in the kind's order
-    double *fout;          // Fourier arrays F[lev][comp][m][theta] complex
+    double *fout;          // Fourier arrays F[lev][comp][theta/8][m][theta%8] complex
     int out_comp[MAX_OUT]; // comp index of each output
     int row_scale;         // 1: outputs times 1/sin^2(theta) (dphspat)
 };
@@ -96,7 +96,7 @@ struct AnaBatch {
     const int *lcut;       // device, per level
 };
 
-// complex elements of one comp of the FP64 forward side F2 (theta in blocks of 8)
+// complex elements of one comp of the FP64 Fourier arrays (theta in blocks of 8)
 __host__ __device__ inline size_t f2_comp(int n_m, int n_theta) { return (size_t)((n_theta + 7) / 8) * n_m * 8; }
 
 // Legendre kernels of the nonlinear step in the split form (mhx_nlsplit.hip)
@@ -197,7 +197,7 @@ struct RlPhys {
 };
 
 struct RlGridArgs {
-    const double *Fin;   // F[lev][nin][m][theta] complex
+    const double *Fin;   // F[lev][nin][theta/8][m][theta%8] complex
     double *Fout;        // F2[lev][nout][theta/8][m][theta%8] complex
     int nin, nout;
     int in_of[RI_N];     // row (compact comp index) of each grid component, -1 absent
@@ -258,7 +258,8 @@ struct Plan {
     float *d_tw32 = nullptr, *d_twr32 = nullptr;  // the same in FP32
     // factors of the wave FFTs (mhx_wavefft.h), where n_phi is a multiple of 64:
     // exp(2 pi i a r / 64) [8][8], and exp(2 pi i j k / n_phi) [n_phi/64][64]
-    double *d_w64 = nullptr, *d_wn = nullptr;
+    // (row pairs) and, where it is one of 128, exp(2 pi i j k / M) [M/64][64] (single rows)
+    double *d_w64 = nullptr, *d_wn = nullptr, *d_wm = nullptr;
     float *d_twn32 = nullptr;       // n_phi complex: exp(-2 pi i k/n_phi), FP32
     int grid_form = 0;              // grid stage of the split step: 0 tiles where supported, 1 slots
     // the nonlinear step's du/dr grids (synthesis of dw, ddw, dz and their
@@ -360,8 +361,8 @@ int launch_nana16(const Plan *p, int kind, const NAnaArgs &args, hipStream_t s);
 // the jobs of one launch (their outputs distinct comps)
 int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, hipStream_t s);
 int launch_ana(const Plan *p, const AnaJob *jobs, int njob, const AnaBatch &b, hipStream_t s);
-// Fourier data (complex, m < n_m): inverse side F[lev][comp][m][theta],
-// forward side F2[lev][comp][theta/8][m][theta%8]; grids in the reference layout
+// Fourier data (complex, m < n_m): inverse side F and forward side F2 both
+// [lev][comp][theta/8][m][theta%8]; grids in the reference layout
 // (theta fastest).  F points at the first comp; F_ld_lev is the level stride in
 // complex elements; grid comp c of level l starts at
 // grid + l*grid_ld_lev + c*grid_ld_comp (doubles).
@@ -375,7 +376,7 @@ int launch_fft(const Plan *p, const double *grid, size_t grid_ld_lev, size_t gri
 // the same for up to three comps with a grid each in one launch
 // (mhx_rowfft.hip), where row_fft_supported
 struct RowFFT {
-    const double *F;        // inverse: F[lev][comp][m][theta]
+    const double *F;        // inverse: F[lev][comp][theta/8][m][theta%8]
     double *F2;             // forward: F2[lev][comp][theta/8][m][theta%8]
     size_t F_ld;            // complex elements per level
     double *grid[3];        // inverse: grids
@@ -477,6 +478,10 @@ int ensure_fp64_tables(Plan *p);
 int ensure_p_tables(Plan *p);
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff);
 // the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768
+// the FP64 step's grid stage on wave FFTs (mhx_gridwave.hip): n_phi = 128 P, P <= 10
+bool grid_wave_supported(const Plan *p);
+int launch_grid_wave(const Plan *p, int nlev, const void *Fin, void *Fout, const double *rad,
+                     double LFfac, void *dgrid, void *full_grids, hipStream_t s);
 bool grid_tile_supported(const Plan *p);
 int launch_grid_tile(const Plan *p, int nlev, const void *Fin, void *Fout, const double *rad,
                      double LFfac, void *dgrid, void *full_grids, hipStream_t s);

@@ -242,11 +242,11 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
 
     // epilogue: north = Sym + Anti, south = Sym - Anti; adjacent lanes (re, im)
     // exchange, so that the even lane stores the northern complex value and
-    // the odd lane the southern one: 128-byte runs of F[lev][comp][m][theta]
+    // the odd lane the southern one: 128-byte lines of the theta-blocked F
     const int col = lane & 15, elev = lev0 + (col >> 1), odd = col & 1;
     if (elev >= a.nlev) return;
-    const size_t cstride = (size_t)a.n_m * a.n_theta;
-    double2 *fo = reinterpret_cast<double2 *>(job.fout) + (size_t)elev * a.fout_ld + (size_t)mc * a.n_theta + odd;
+    const size_t cstride = f2_comp(a.n_m, a.n_theta);
+    double2 *fo = reinterpret_cast<double2 *>(job.fout) + (size_t)elev * a.fout_ld + (size_t)mc * 8 + odd;
 #pragma unroll
     for (int s = 0; s < TPW; ++s) {
         const int tt = tt0 + s * tstep;
@@ -263,7 +263,7 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
                 double2 v = odd ? make_double2(other, so) : make_double2(n, other);
                 if (job.row_scale) v = make_double2(sc * v.x, sc * v.y);
                 auto store = [&](int o, double2 w) {
-                    if (ok) fo[job.out_comp[o] * cstride + 2 * th] = w;
+                    if (ok) fo[job.out_comp[o] * cstride + (size_t)(th >> 2) * (a.n_m * 8) + (2 * th & 7)] = w;
                 };
                 // columns: QST (Q, C1, C2), SPHTOR (C1, C2), SCAL x;
                 // SG, GRAD: x, x' with d/dphi = i m (P x)

@@ -169,14 +169,14 @@ SynJob syn_job(Plan *p, int kind, ColOp c0, ColOp c1 = ColOp(), ColOp c2 = ColOp
 // levels of the synthesis launches into ws_F (18 comps per level)
 SynBatch syn_batch(Plan *p, int nlev, size_t src_ld)
 {
-    return SynBatch{nlev, src_ld, (size_t)18 * p->n_m * p->n_theta, p->d_lcut, p->d_rad};
+    return SynBatch{nlev, src_ld, 18 * f2_comp(p->n_m, p->n_theta), p->d_lcut, p->d_rad};
 }
 
 // Fourier comps [0, ncomp) of ws_F -> grids at separate destinations (level
 // stride ld_grid doubles)
 int ifft_to(Plan *p, int ncomp, int nlev, double *const *dst, size_t ld_grid)
 {
-    const size_t comp = (size_t)p->n_m * p->n_theta;
+    const size_t comp = f2_comp(p->n_m, p->n_theta);
     if (row_fft_supported(p)) {
         RowFFT a;
         std::memset(&a, 0, sizeof(a));
@@ -435,7 +435,7 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         twn32[2 * k] = (float)std::cos(2.0 * pi * k / n_phi);
         twn32[2 * k + 1] = (float)-std::sin(2.0 * pi * k / n_phi);
     }
-    std::vector<double> w64, wn;
+    std::vector<double> w64, wn, wm;
     if (n_phi % 64 == 0) {
         auto root = [&](std::vector<double> &v, int k, int n) {
             v.push_back(std::cos(2.0 * pi * k / n));
@@ -443,6 +443,7 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         };
         for (int k = 0; k < 64; ++k) root(w64, k / 8 * (k % 8), 64);
         for (int k = 0; k < n_phi; ++k) root(wn, k / 64 * (k % 64), n_phi);
+        for (int k = 0; n_phi % 128 == 0 && k < n_phi / 2; ++k) root(wm, k / 64 * (k % 64), n_phi / 2);
     }
     {
         const char *gf = std::getenv("MHX_GRID_FORM");
@@ -454,7 +455,8 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         (rc = up(p->d_gauss, p->gauss)) || (rc = up(p->d_osin2, osin2)) ||
         (rc = up(p->d_tw, tw)) || (rc = up(p->d_twr, twr)) || (rc = up(d_lm2l, lm2l)) ||
         (rc = up(p->d_tw32, tw32)) || (rc = up(p->d_twr32, twr32)) || (rc = up(p->d_lm2m, lm2m)) ||
-        (rc = up(p->d_twn32, twn32)) || (!wn.empty() && ((rc = up(p->d_w64, w64)) || (rc = up(p->d_wn, wn))))) {
+        (rc = up(p->d_twn32, twn32)) || (!wn.empty() && ((rc = up(p->d_w64, w64)) || (rc = up(p->d_wn, wn)))) ||
+        (!wm.empty() && (rc = up(p->d_wm, wm)))) {
         mhx_plan_destroy(h);
         return rc;
     }
@@ -524,6 +526,7 @@ int mhx_plan_destroy(mhx_plan *h)
     free_dev(p->d_twn32);
     free_dev(p->d_w64);
     free_dev(p->d_wn);
+    free_dev(p->d_wm);
     free_dev(p->d_syn16_P);
     free_dev(p->d_syn16_dP);
     free_dev(p->d_ana16_P);

@@ -422,10 +422,10 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
     if (nin == 0 || nout == 0) return fail(MHX_E_UNSUPPORTED, "radial loop: nothing to transform");
 
     // ---- buffers ----
-    const size_t four = (size_t)P->n_m * P->n_theta * 2;  // doubles per Fourier comp
+    const size_t four = 2 * f2_comp(P->n_m, P->n_theta);  // doubles per Fourier comp
     const size_t lmd = (size_t)nlev * ld_lm * 2;           // doubles per nl array
     if ((rc = grow(B->F, B->nF, (size_t)nlev * nin * four)) ||
-        (rc = grow(B->F2, B->nF2, (size_t)nlev * nout * 2 * f2_comp(P->n_m, P->n_theta))) ||
+        (rc = grow(B->F2, B->nF2, (size_t)nlev * nout * four)) ||
         (rc = grow(B->nl, B->nnl, (size_t)NL_N * lmd)) ||
         (rc = grow(B->rad, B->nrad, (size_t)(RL_NRAD + TR_NRAD + 2) * nlev)))
         return rc;
@@ -538,7 +538,7 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
 
     // ---- synthesis ----
     enum { W = 0, DW, DDW, Z, DZ, S_, XI, PHI, BB, DB, DDB, AJ, DJ };
-    const SynBatch sb{nlev, ld_lm, (size_t)nin * P->n_m * P->n_theta, B->lcut, d_or2};
+    const SynBatch sb{nlev, ld_lm, nin * four / 2, B->lcut, d_or2};
     SynJob jobs[MAX_SYN_JOBS];
     int njob = 0;
     auto add = [&](int kind, ColOp a, ColOp b, ColOp c, int c0, int c1, int c2) -> SynJob & {
@@ -660,7 +660,7 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
     if (ph->l_mag_nl) ana(ANA_QST, out_of[RO_VXBR], nl[NL_VXBR], nl[NL_VXBT], nl[NL_VXBP]);
     if (anel) ana(ANA_SH, out_of[RO_HEAT], nl[NL_HEAT]);
     if (phase) ana(ANA_SH, out_of[RO_PHI], dout[7]);
-    const AnaBatch ab{nlev, (size_t)nout * f2_comp(P->n_m, P->n_theta), ld_lm, B->lcut};
+    const AnaBatch ab{nlev, nout * four / 2, ld_lm, B->lcut};
     if ((rc = launch_ana(P, anas, nana, ab, s))) return rc;
 
     // ---- lm-space assembly ----

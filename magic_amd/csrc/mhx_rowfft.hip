@@ -6,8 +6,7 @@
 //
 // Bound by HBM: n_theta n_phi 8 + n_theta n_m 16 bytes per component and
 // level.  All components of a call run in one launch, 8 theta rows per
-// workgroup (whole 128-byte lines of F[m][theta] and of the forward side's
-// blocks of 8 rows).
+// workgroup (whole 128-byte lines of the Fourier arrays' blocks of 8 rows).
 #include "mhx_wavefft.h"
 
 namespace mhx {
@@ -44,12 +43,14 @@ template <int P> __global__ __launch_bounds__(64 * row_waves<P>()) void k_irow(R
     const int th = 2 * (tb * NW + wave);
     if (th >= a.n_theta) return;
     const double2 *X = reinterpret_cast<const double2 *>(a.F) + (size_t)lev * a.F_ld +
-                       (size_t)comp * a.n_m * a.n_theta + th;
+                       comp * f2_comp(a.n_m, a.n_theta) + (size_t)(th / 8) * a.n_m * 8 + th % 8;
     double2 x[P];
     // Y_k = X1_k + i X2_k, Y_{N-k} = conj X1_k + i conj X2_k (real parts of mode 0)
-    W::inverse(sm + wave * W::BUF, lane, a.w64, a.wn, [&](int k) {
+    const auto w64 = [&](int i) { return a.w64[8 * i + (lane & 7)]; };
+    const auto wn = [&](int k1) { return a.wn[64 * k1 + lane]; };
+    W::inverse(sm + wave * W::BUF, lane, w64, wn, [&](int, int, int k) {
         const int kk = k <= N / 2 ? k : N - k;
-        const double2 *p = X + (size_t)min(kk, a.n_m - 1) * a.n_theta;
+        const double2 *p = X + (size_t)min(kk, a.n_m - 1) * 8;
         const double2 u = p[0], v = p[1];
         double2 y = k <= N / 2 ? mk<double2>(u.x - v.y, u.y + v.x) : mk<double2>(u.x + v.y, v.x - u.y);
         if (k == 0) y = mk<double2>(u.x, v.x);
@@ -78,7 +79,7 @@ template <int P> __global__ __launch_bounds__(64 * row_waves<P>()) void k_frow(R
         const Pair p = *reinterpret_cast<const Pair *>(g + (size_t)(lane + 64 * q) * a.n_theta);
         x[q] = mk<double2>(p.x, p.y);
     }
-    W::forward(buf, lane, a.w64, a.wn, x);
+    W::forward(buf, lane, [&](int i) { return a.w64[8 * i + (lane & 7)]; }, [&](int k1) { return a.wn[64 * k1 + lane]; }, x);
     // X1_k = (Y_k + conj Y_{N-k}) / 2, X2_k = (Y_k - conj Y_{N-k}) / (2 i), scaled
     // by 1/N and, for the flagged comps, 1/sin^2(theta) (equal in the two rows)
     const double sc = (a.osin2_mask >> comp & 1u ? a.osin2[th] : 1.0) * (0.5 / (double)N);

@@ -122,12 +122,11 @@ template <int P> struct WaveFFT {
     static constexpr int N = 64 * P, TASKS = 8 * P, RND = (TASKS + 63) / 64;
     static constexpr int BUF = 72 * P;  // complex elements of the wave's buffer
 
-    // tables (device): w64[a][r] = exp(2 pi i a r / 64), 8 x 8; wn[k1][j] =
-    // exp(2 pi i j k1 / N), P x 64
-    // x[q] = sum_k Y_k exp(2 pi i k n / N), n = lane + 64 q; y(k) gives Y_k
-    template <class Y>
-    __device__ __forceinline__ static void inverse(C *buf, int lane, const C *__restrict__ w64,
-                                                   const C *__restrict__ wn, Y &&y, C *x)
+    // factors: w64(a) = exp(2 pi i a (lane % 8) / 64), wn(k1) = exp(2 pi i lane k1 / N)
+    // x[q] = sum_k Y_k exp(2 pi i k n / N), n = lane + 64 q; y(rd, s, k) gives
+    // Y_k, k = k1 + P (lane % 8 + 8 s) of the task of round rd
+    template <class W64, class Wn, class Y>
+    __device__ __forceinline__ static void inverse(C *buf, int lane, W64 &&w64, Wn &&wn, Y &&y, C *x)
     {
         const int r = lane & 7;
 #pragma unroll
@@ -136,11 +135,11 @@ template <int P> struct WaveFFT {
             if (8 * P % 64 == 0 || rd + 1 < RND || k1 < P) {
                 C v[8];
 #pragma unroll
-                for (int s = 0; s < 8; ++s) v[s] = y(k1 + P * (r + 8 * s));
+                for (int s = 0; s < 8; ++s) v[s] = y(rd, s, k1 + P * (r + 8 * s));
                 Dft<8, C>::run(v, +1);
 #pragma unroll
                 for (int a = 0; a < 8; ++a)
-                    buf[72 * k1 + 8 * a + ((r + a) & 7)] = a ? cmul(v[a], w64[8 * a + r]) : v[a];
+                    buf[72 * k1 + 8 * a + ((r + a) & 7)] = a ? cmul(v[a], w64(a)) : v[a];
             }
         }
         wave_order();
@@ -161,7 +160,7 @@ template <int P> struct WaveFFT {
 #pragma unroll
         for (int k1 = 0; k1 < P; ++k1) {
             x[k1] = buf[72 * k1 + lane];
-            if (k1) x[k1] = cmul(x[k1], wn[64 * k1 + lane]);
+            if (k1) x[k1] = cmul(x[k1], wn(k1));
         }
         wave_order();
         Dft<P, C>::run(x, +1);
@@ -169,13 +168,13 @@ template <int P> struct WaveFFT {
 
     // Y_k = sum_n x_n exp(-2 pi i k n / N) from x[q] = x_{lane + 64 q}, left in
     // buf at index k (N elements)
-    __device__ __forceinline__ static void forward(C *buf, int lane, const C *__restrict__ w64,
-                                                   const C *__restrict__ wn, C *x)
+    template <class W64, class Wn>
+    __device__ __forceinline__ static void forward(C *buf, int lane, W64 &&w64, Wn &&wn, C *x)
     {
         const int r = lane & 7;
         Dft<P, C>::run(x, -1);
 #pragma unroll
-        for (int k1 = 0; k1 < P; ++k1) buf[72 * k1 + lane] = k1 ? cmul(x[k1], cconj(wn[64 * k1 + lane])) : x[k1];
+        for (int k1 = 0; k1 < P; ++k1) buf[72 * k1 + lane] = k1 ? cmul(x[k1], cconj(wn(k1))) : x[k1];
         wave_order();
 #pragma unroll
         for (int rd = 0; rd < RND; ++rd) {
@@ -188,7 +187,7 @@ template <int P> struct WaveFFT {
                 Dft<8, C>::run(v, -1);
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    buf[72 * k1 + 8 * a + ((i + a) & 7)] = i ? cmul(v[i], cconj(w64[8 * i + a])) : v[i];
+                    buf[72 * k1 + 8 * a + ((i + a) & 7)] = i ? cmul(v[i], cconj(w64(i))) : v[i];
             }
         }
         wave_order();
