@@ -356,8 +356,12 @@ __global__ void k_axi(int l_max, int nh, const double *__restrict__ plm_syn,
 // loads all of its inputs before it stores any output.  Six slots work on one
 // theta row: the 18 inverse FFTs in three rounds of six, the 10 forward FFTs
 // in two.  Between rounds the block redistributes the row so that each thread
-// holds P / 3 grid points of every component for the products.
-
+// holds P / 3 grid points of every component for the products.  Slots of up to
+// four lanes share the block with those of NR - 1 further theta rows, which
+// are neighbouring lanes, so that the waves are full and the rows' Fourier
+// values are read in runs (one row per block, 12 of 64 lanes at work, took 46.5
+// us at n_phi = 48, l_max = 64 x 33 levels, against 29.4 us with 16 rows; at 16 and 8
+// lanes several rows per block are slower, 400 -> 470 us at n_phi = 384 x 65).
 
 template <typename T, int A, int B>
 __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict__ Fin,
@@ -372,19 +376,22 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
     typedef SlotFFT<A, B> FFT;
     constexpr int M = FFT::M, N = 2 * M, Q = FFT::Q;
     constexpr int NPT = FFT::P / 3;  // grid points per thread: N = NPT * 6 Q
+    constexpr int NR = FFT::NR, nthr = FFT::NTHR / NR;  // theta rows per block, threads per row
+    constexpr int MP = padded_row<M, FFT::P>();
     C *s_tw = reinterpret_cast<C *>(smem_raw);  // M + M / 8 (padded)
     C *s_twr = s_tw + M + M / 8;
-    C *rows = s_twr + M + 1;  // 6 slot rows of MP (padded)
-    constexpr int MP = padded_row<M, FFT::P>();
     int lb;
     {
         const int nx = 8, nb = gridDim.x, b = blockIdx.x;
         int per = nb / nx, rem = nb % nx, x = b % nx, i = b / nx;
         lb = (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + i;
     }
-    const int th = lb % n_theta, lev = lb / n_theta;
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int ntr = (n_theta + NR - 1) / NR, lev = lb / ntr, rowi = threadIdx.x % NR;
+    const int throw_ = (lb - lev * ntr) * NR + rowi, th = min(throw_, n_theta - 1);
+    const bool on = NR == 1 || throw_ < n_theta;  // past the last row: computed, not stored
+    const int tid = threadIdx.x / NR;  // thread of the row
     const int slot = tid / Q, t = tid - slot * Q;
+    C *rows = s_twr + M + 1 + rowi * FFT::row_stride(MP);  // 6 slot rows of MP (padded)
     const T o2 = T(osin2[th]);
     const T or2 = T(rad[lev]), or4 = T(rad[nlev + lev]), orho1 = T(rad[2 * nlev + lev]);
     const T LFfac = T(LFfac_d);
@@ -473,12 +480,12 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
                 if (q < M) {
                     zz = rows[r * MP + pidx<FFT::P>(q)];
                     const int comp = round == 0 ? r : (round == 1 ? 9 + r : (r < 3 ? 6 + r : 12 + r));
-                    if (full_grids) {
+                    if (full_grids && on) {
                         T *fg = full_grids + (((size_t)lev * 18 + comp) * N + 2 * q) * n_theta + th;
                         fg[0] = zz.x;
                         fg[n_theta] = zz.y;
                     }
-                    if (round == 2 && r < 3 && dgrid)
+                    if (round == 2 && r < 3 && dgrid && on)
                         *reinterpret_cast<C *>(dgrid + (((size_t)lev * 3 + r) * n_theta + th) * N + 2 * q) = zz;
                 }
                 val[r][2 * p2] = zz.x;
@@ -515,7 +522,8 @@ __global__ __launch_bounds__(384) void k_nl_slots(FFTArgs f, const T *__restrict
             // F2 theta-blocked: consecutive k are FS apart
             constexpr int FS = f2_th<T>();
             C *fo = Fo + f2_index<T>(comp, th, t, n_theta, n_m);
-            for (int k = t; k < n_m; k += Q, fo += Q * FS) *fo = rfft_post_padded<FFT::P>(z, k, M, s_twr, invN);
+            for (int k = t; k < n_m; k += Q, fo += Q * FS)
+                if (on) *fo = rfft_post_padded<FFT::P>(z, k, M, s_twr, invN);
         }
         __syncthreads();
     };
@@ -1028,8 +1036,9 @@ int launch_slots(const Plan *p, const FFTArgs &f, int nlev, const void *Fin, voi
                  const double *rad, double LFfac, void *dgrid, void *full_grids, hipStream_t s)
 {
     constexpr int M = SlotFFT<A, B>::M, NPT = SlotFFT<A, B>::P / 3, nthr = SlotFFT<A, B>::NTHR;
-    if (NPT * nthr < p->n_phi) return fail(MHX_E_UNSUPPORTED, "n_phi too large for the fused stage");
-    const size_t shm = ((size_t)2 * M + M / 8 + 1 + 6 * (size_t)padded_row<M, SlotFFT<A, B>::P>()) * 2 * sizeof(T);
+    static_assert(NPT * 6 * SlotFFT<A, B>::Q == 2 * M, "points do not tile the threads");
+    constexpr int NR = SlotFFT<A, B>::NR;
+    const size_t shm = ((size_t)2 * M + M / 8 + 1 + NR * (size_t)SlotFFT<A, B>::row_stride(padded_row<M, SlotFFT<A, B>::P>())) * 2 * sizeof(T);
     // set once per kernel (the attribute persists), so that a call under
     // graph capture makes no attribute call
     static int shm_set = 0;
@@ -1038,7 +1047,7 @@ int launch_slots(const Plan *p, const FFTArgs &f, int nlev, const void *Fin, voi
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
         shm_set = (int)shm;
     }
-    dim3 grid((unsigned)(p->n_theta * nlev));
+    dim3 grid((unsigned)((p->n_theta + NR - 1) / NR * nlev));
     k_nl_slots<T, A, B><<<grid, nthr, shm, s>>>(f, static_cast<const T *>(Fin), static_cast<T *>(Fout),
                                                 p->n_m, p->n_theta, nlev, p->d_osin2, rad, LFfac,
                                                 static_cast<T *>(dgrid), static_cast<T *>(full_grids),

@@ -396,8 +396,12 @@ constexpr int pow4(int a) { return a == 0 ? 1 : 4 * pow4(a - 1); }
 template <int A, int B> struct SlotFFT {
     static constexpr int M = 3 * pow4(A) * (B ? 2 : 1);
     static constexpr int Q = M / 12 <= 64 ? M / 12 : 64, P = M / Q;
-    // threads of the grid-stage block: six slots, at least one wave
-    static constexpr int NTHR = (6 * Q < 64 ? 64 : 6 * Q + 63) / 64 * 64;
+    // grid-stage block: NR theta rows of six slots each, neighbouring threads
+    // working on the same slot lane of the NR rows (192 threads), or one row (at
+    // least one wave)
+    static constexpr int NR = Q <= 4 ? 32 / Q : 1, NTHR = (6 * Q * NR + 63) / 64 * 64;
+    // LDS distance of the NR rows' slots (complex): the rows' lanes on distinct banks
+    static constexpr int row_stride(int mp) { return NR == 1 ? 6 * mp : (6 * mp + 15) / 16 * 16 + (NR >= 16 ? 1 : 2); }
     static_assert(Q * P == M && P % 12 == 0 && 64 % Q == 0, "unsupported slot length");
     template <int I, typename C>
     __device__ __forceinline__ static void radix4(C *buf, int t, const C *tw, int sign)

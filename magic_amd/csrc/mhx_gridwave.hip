@@ -253,11 +253,15 @@ template <int P> int launch_p(const GwArgs &a, hipStream_t s)
 
 }  // namespace
 
+// powers of two, where the slot FFTs (M = 3 4^A 2^B) do not apply: per launch
+// against the block-wide passes 402 -> 326 us (n_phi = 256 x 97 levels), 1050 ->
+// 720 us (512 x 65) and 2481 -> 1154 us (1024 x 16); slower for 640 (858 -> 987
+// us, five waves) and than the slots for 768 (2.2 -> 4.0 ms, registers)
 bool grid_wave_supported(const Plan *p)
 {
     if (!p->d_wm || p->n_phi % 128) return false;
     switch (p->n_phi / 128) {
-    case 2: case 4: case 5: case 8: return true;
+    case 2: case 4: case 8: return true;
     default: return false;
     }
 }
@@ -282,10 +286,7 @@ int launch_grid_wave(const Plan *p, int nlev, const void *Fin, void *Fout, const
     a.cour = p->cour;
     switch (p->n_phi / 128) {
     case 2: return launch_p<2>(a, s);
-    case 3: return launch_p<3>(a, s);
     case 4: return launch_p<4>(a, s);
-    case 5: return launch_p<5>(a, s);
-    case 6: return launch_p<6>(a, s);
     case 8: return launch_p<8>(a, s);
     default: return fail(MHX_E_UNSUPPORTED, "wave grid stage length");
     }
