@@ -839,80 +839,297 @@ __global__ __launch_bounds__(512) void k_rl_grid(FFTArgs f, RlGridArgs a)
     }
 }
 
-// k_rl_grid with wave-slot FFTs (the row length M = 3 4^A 2^B): the rows
-// are padded (index i at pidx<P>(i)) and every row is transformed in place
-// by one slot of Q lanes of a wave, all rows at once; no scratch rows and no
-// block barrier inside the FFTs
+// The same with wave-slot FFTs (row length M = 3 4^A 2^B): the blocks and slots
+// of k_nl_slots.  The components come in rounds of six, one slot each, and the
+// products are formed as they arrive, in the registers of the threads that own
+// the points:
+//   U  vr vt vp cvr and, with curl advection, cvt cvp, else dvpdp s
+//   S  s (curl advection), xi, phi, dvpdp (curl advection with heating terms)
+//      -> the phase terms, V s and V xi transformed back
+//   G  dvrdr dvtdr dvpdr dvrdt dvrdp dvtdp (u . grad u, viscous heating)
+//   M  br bt bp cbr cbt cbp -> Adv and V x B, then the heating terms
+// so that six LDS rows serve any number of components (all of a row's 18
+// components in LDS left one block per CU: 4.35 ms for Boussinesq MHD with
+// u . grad u at l_max = 255 x 97, against 2.8 ms).  Three waves per SIMD are
+// worth the spills that they cost (6.5 -> 6.2 ms per loop at that size).
 template <int A, int B>
-__global__ __launch_bounds__(512) void k_rl_grid_s(FFTArgs f, RlGridArgs a)
+__global__ __launch_bounds__((SlotFFT<A, B>::NTHR), A <= 3 ? 3 : 2) void k_rl_slots(FFTArgs f, RlGridArgs a)
 {
     typedef double2 C;
     typedef SlotFFT<A, B> FFT;
-    constexpr int M = FFT::M, N = 2 * M, Q = FFT::Q, P = FFT::P;
-    constexpr int MP = padded_row<M, P>(), SPW = 64 / Q;
+    constexpr int M = FFT::M, N = 2 * M, Q = FFT::Q, P = FFT::P, MP = padded_row<M, P>();
+    constexpr int NPT = P / 3, NR = FFT::NR, nthr = FFT::NTHR / NR;
     extern __shared__ char smem_raw[];
     C *s_tw = reinterpret_cast<C *>(smem_raw);  // M + M / 8 (padded)
     C *s_twr = s_tw + M + M / 8;                // M + 1
-    C *rows = s_twr + M + 1;                    // max(nin, nout) rows of MP
     int lb;
     {
         const int nx = 8, nb = gridDim.x, b = blockIdx.x;
         int per = nb / nx, rem = nb % nx, x = b % nx, i = b / nx;
         lb = (x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per) + i;
     }
-    const int n_theta = a.n_theta, n_m = a.n_m;
-    const int th = lb % n_theta, lev = lb / n_theta;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int lane = tid & 63, sw = lane / Q, t = lane - sw * Q;
-    const int slot = (tid >> 6) * SPW + sw, nslot = (nthr >> 6) * SPW;
-    const bool act = sw < SPW;
+    const int n_theta = a.n_theta, n_m = a.n_m, nlev = a.nlev;
+    const int ntr = (n_theta + NR - 1) / NR, lev = lb / ntr, rowi = threadIdx.x % NR;
+    const int throw_ = (lb - lev * ntr) * NR + rowi, th = min(throw_, n_theta - 1);
+    const bool on = NR == 1 || throw_ < n_theta;  // past the last row: computed, not stored
+    const int tid = threadIdx.x / NR, slot = tid / Q, t = tid - slot * Q;
+    C *rows = s_twr + M + 1 + rowi * FFT::row_stride(MP);
     {
         const C *tw = reinterpret_cast<const C *>(f.tw);
         const C *twr = reinterpret_cast<const C *>(f.twr);
-        for (int e = tid; e < M; e += nthr) s_tw[e + (e >> 3)] = tw[e];
-        for (int e = tid; e <= M; e += nthr) s_twr[e] = twr[e];
+        for (int e = threadIdx.x; e < M; e += blockDim.x) s_tw[e + (e >> 3)] = tw[e];
+        for (int e = threadIdx.x; e <= M; e += blockDim.x) s_twr[e] = twr[e];
     }
     __syncthreads();
+    const RlPhys &ph = a.ph;
+    const double *rad = a.rad;
+    const double r = rad[RR_R * nlev + lev], or1 = rad[RR_OR1 * nlev + lev], or2 = rad[RR_OR2 * nlev + lev];
+    const double or4 = rad[RR_OR4 * nlev + lev], orho1 = rad[RR_ORHO1 * nlev + lev];
+    const double beta = rad[RR_BETA * nlev + lev];
+    const bool lcr = rad[RR_LCR * nlev + lev] != 0.0;
+    const double o2 = a.th[RT_OSIN2 * n_theta + th], cosn2 = a.th[RT_COSN2 * n_theta + th];
 
-    // inverse FFTs of rows [0, nin), one slot per row
-    const C *Fi = reinterpret_cast<const C *>(a.Fin) + lev * a.nin * f1_size<double>(n_theta, n_m) + f1_row<double>(th, n_m);
-    if (act)
-        for (int c = slot; c < a.nin; c += nslot) {
-            C *z = rows + (size_t)c * MP;
-            const C *X = Fi + c * f1_size<double>(n_theta, n_m);
+    const size_t fcomp = f1_size<double>(n_theta, n_m);
+    const C *Fi = reinterpret_cast<const C *>(a.Fin) + lev * a.nin * fcomp + f1_row<double>(th, n_m);
+    C *Fo = reinterpret_cast<C *>(a.Fout) + lev * a.nout * fcomp;
+
+    double val[6][NPT];
+    // inverse FFTs of six comps (rows of F, -1: absent, value 0) into val
+    auto inverse6 = [&](int c0, int c1, int c2, int c3, int c4, int c5) {
+        const int cs[6] = {c0, c1, c2, c3, c4, c5};
+        int c = -1;
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+            if (slot == i) c = cs[i];
+        if (c >= 0) {
+            C *z = rows + slot * MP;
+            const C *X = Fi + c * fcomp;
             // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/N} (X_k - conj X_{M-k})
             for (int k = t; k <= M / 2; k += Q) {
                 const int k2 = M - k;
                 C xa = k < n_m ? X[(size_t)k * 8] : mk<C>(0.0, 0.0);
-                C xc = k2 < n_m ? X[(size_t)k2 * 8] : mk<C>(0.0, 0.0);
-                if (k == 0) {
-                    xa.y = 0.0;
-                    xc.y = 0.0;
-                }
-                z[pidx<P>(k)] = cadd(cadd(xa, cconj(xc)), cmuli(cmul(cconj(s_twr[k]), csub(xa, cconj(xc))), 1));
-                if (k2 < M && k2 != k)
-                    z[pidx<P>(k2)] = cadd(cadd(xc, cconj(xa)), cmuli(cmul(cconj(s_twr[k2]), csub(xc, cconj(xa))), 1));
+                const C xc = k2 < n_m ? X[(size_t)k2 * 8] : mk<C>(0.0, 0.0);
+                if (k == 0) xa.y = 0.0;
+                // Z_{M-k} shares the sum and the product of Z_k
+                const C e = mk<C>(xa.x + xc.x, xa.y - xc.y);
+                const C d = cmul(cconj(s_twr[k]), mk<C>(xa.x - xc.x, xa.y + xc.y));
+                z[pidx<P>(k)] = mk<C>(e.x - d.y, e.y + d.x);
+                if (k > 0) z[pidx<P>(k2)] = mk<C>(e.x + d.y, d.x - e.y);
             }
             wave_order();
             FFT::run(z, t, s_tw, +1);
         }
-    __syncthreads();
+        __syncthreads();
+        // thread owns the point pairs (2q, 2q+1), q = tid + p2 nthr
+#pragma unroll
+        for (int p2 = 0; p2 < NPT / 2; ++p2) {
+            const int q = tid + p2 * nthr;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                const C zz = q < M && cs[i] >= 0 ? rows[i * MP + pidx<P>(q)] : mk<C>(0.0, 0.0);
+                val[i][2 * p2] = zz.x;
+                val[i][2 * p2 + 1] = zz.y;
+            }
+        }
+        __syncthreads();
+    };
+    // forward FFTs of val into rows of F2 (-1: none)
+    auto forward6 = [&](int c0, int c1, int c2, int c3, int c4, int c5) {
+        const int cs[6] = {c0, c1, c2, c3, c4, c5};
+#pragma unroll
+        for (int p2 = 0; p2 < NPT / 2; ++p2) {
+            const int q = tid + p2 * nthr;
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+                if (q < M && cs[i] >= 0) {
+                    const double sc = a.out_osin2 >> cs[i] & 1u ? o2 : 1.0;
+                    rows[i * MP + pidx<P>(q)] = mk<C>(val[i][2 * p2] * sc, val[i][2 * p2 + 1] * sc);
+                }
+        }
+        __syncthreads();
+        int c = -1;
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+            if (slot == i) c = cs[i];
+        if (c >= 0) {
+            C *z = rows + slot * MP;
+            FFT::run(z, t, s_tw, -1);
+            const double invN = 1.0 / (double)N;
+            C *fo = Fo + f2_index<double>(c, th, t, n_theta, n_m);
+            for (int k = t; k < n_m; k += Q, fo += Q * 8)
+                if (on) *fo = rfft_post_padded<P>(z, k, M, s_twr, invN);
+        }
+        __syncthreads();
+    };
+#define RL_EACH(stmt) \
+    _Pragma("unroll") for (int p = 0; p < NPT; ++p) { stmt; }
+    const int *in = a.in_of, *out = a.out_of;
 
-    // the products: point j of row c is the (j mod 2) part of complex j / 2
-    rl_points(a, reinterpret_cast<double *>(rows),
-              [&](int c, int j) { return (size_t)c * 2 * MP + 2 * pidx<P>(j >> 1) + (j & 1); }, N, lev, th);
-    __syncthreads();
-
-    // forward FFTs of rows [0, nout) in place, then F2
-    if (act)
-        for (int c = slot; c < a.nout; c += nslot) FFT::run(rows + (size_t)c * MP, t, s_tw, -1);
-    __syncthreads();
-    C *Fo = reinterpret_cast<C *>(a.Fout) + (size_t)lev * a.nout * f2_size<double>(n_theta, n_m);
-    const double invN = 1.0 / (double)N;
-    for (int idx = tid; idx < a.nout * n_m; idx += nthr) {
-        const int r2 = idx / n_m, k = idx - r2 * n_m;
-        Fo[f2_index<double>(r2, th, k, n_theta, n_m)] = rfft_post_padded<P>(rows + (size_t)r2 * MP, k, M, s_twr, invN);
+    double u[3][NPT], adv[3][NPT], s[NPT], cvr[NPT], dvpdp[NPT];
+    // U
+    const bool curl = ph.adv_curl;
+    inverse6(in[RI_VR], in[RI_VT], in[RI_VP], in[RI_CVR], curl ? in[RI_CVT] : in[RI_DVPDP], curl ? in[RI_CVP] : in[RI_S]);
+    RL_EACH(u[0][p] = val[0][p]; u[1][p] = val[1][p]; u[2][p] = val[2][p]; cvr[p] = val[3][p];
+            adv[0][p] = adv[1][p] = adv[2][p] = 0.0; dvpdp[p] = s[p] = 0.0)
+    if (curl) {
+        // curl(u) x u (src/get_nl.f90:262-273)
+        if (ph.conv_nl)
+            RL_EACH(const double cvt = val[4][p]; const double cvp = val[5][p];
+                    adv[0][p] = -o2 * (cvt * u[2][p] - cvp * u[1][p]);
+                    adv[1][p] = -or4 * (cvp * u[0][p] - cvr[p] * u[2][p]);
+                    adv[2][p] = -or4 * (cvr[p] * u[1][p] - cvt * u[0][p]))
+    } else {
+        RL_EACH(dvpdp[p] = val[4][p]; s[p] = val[5][p])
     }
+    // S
+    double xi[NPT];
+    RL_EACH(xi[p] = 0.0)
+    if ((curl && (in[RI_S] >= 0 || in[RI_DVPDP] >= 0)) || ph.chem || ph.phase) {
+        inverse6(curl ? in[RI_S] : -1, in[RI_XI], in[RI_PHI], curl ? in[RI_DVPDP] : -1, -1, -1);
+        RL_EACH(xi[p] = val[1][p])
+        if (curl) RL_EACH(s[p] = val[0][p]; dvpdp[p] = val[3][p])
+        if (ph.phase) {
+            // phase field (src/get_nl.f90:333-344); the Lorentz force alone
+            // replaces Adv without nonlinear advection (src/rIter.f90:648-660)
+            const double e2 = 1.0 / (ph.epsPhase * ph.epsPhase), ph2 = e2 / (ph.penaltyFac * ph.penaltyFac);
+            const bool keep = ph.conv_nl || !ph.mag_LF;
+            RL_EACH(const double pc = val[2][p];
+                    val[0][p] = -e2 * pc * (1.0 - pc) * (ph.phaseDiffFac * (1.0 - 2.0 * pc) + s[p] - ph.tmelt);
+                    if (keep) {
+                        adv[0][p] -= pc * u[0][p] * ph2;
+                        adv[1][p] -= or2 * pc * u[1][p] * ph2;
+                        adv[2][p] -= or2 * pc * u[2][p] * ph2;
+                    })
+            if (out[RO_PHI] >= 0) forward6(out[RO_PHI], -1, -1, -1, -1, -1);
+        }
+    }
+    if (ph.prec || ph.centr) {
+        const double sinT = a.th[RT_SIN * n_theta + th], cosT = a.th[RT_COS * n_theta + th];
+        const double osinT = a.th[RT_OSIN * n_theta + th];
+        if (ph.prec)
+            // precession (src/get_nl.f90:346-356)
+            RL_EACH(const double ang = ph.oek * ph.time + (2 * (tid + p / 2 * nthr) + p % 2) * a.dphi;
+                    const double c = cos(ang); const double sn = sin(ang);
+                    adv[0][p] += ph.posnalp * osinT * r * (c * u[2][p] * cosT + sn * u[1][p]);
+                    adv[1][p] += -ph.posnalp * sinT * or2 * (c * u[2][p] + sn * or1 * u[0][p]);
+                    adv[2][p] += ph.posnalp * sinT * c * or2 * (u[1][p] - or1 * u[0][p] * cosT))
+        if (ph.centr) {
+            // centrifugal acceleration (src/get_nl.f90:358-374)
+            const double s2 = sinT * sinT, cf = -ph.dilution_fac * r * ph.ra * ph.opr;
+            RL_EACH(adv[0][p] += cf * (s2 * s2) * s[p]; adv[1][p] += cf * (s2 * sinT) * cosT * s[p])
+        }
+    }
+    if (out[RO_VSR] >= 0 || out[RO_VXIR] >= 0) {
+        // V s, V xi (src/get_nl.f90:320-331)
+        const double hs = ph.heat_nl ? 1.0 : 0.0;
+        RL_EACH(val[0][p] = hs * u[0][p] * s[p]; val[1][p] = hs * or2 * u[1][p] * s[p];
+                val[2][p] = hs * or2 * u[2][p] * s[p]; val[3][p] = u[0][p] * xi[p];
+                val[4][p] = or2 * u[1][p] * xi[p]; val[5][p] = or2 * u[2][p] * xi[p])
+        forward6(out[RO_VSR], out[RO_VST], out[RO_VSP], out[RO_VXIR], out[RO_VXIT], out[RO_VXIP]);
+    }
+    // G
+    double heat[NPT];
+    RL_EACH(heat[p] = 0.0)
+    if (in[RI_DVRDR] >= 0) {
+        inverse6(in[RI_DVRDR], in[RI_DVTDR], in[RI_DVPDR], in[RI_DVRDT], in[RI_DVRDP], in[RI_DVTDP]);
+        const double vh = ph.ViscHeatFac * or4 * orho1 * rad[RR_OTEMP1 * nlev + lev] * rad[RR_VISC * nlev + lev];
+#pragma unroll
+        for (int p = 0; p < NPT; ++p) {
+            const double vr = u[0][p], vt = u[1][p], vp = u[2][p];
+            const double dvrdr = val[0][p], dvtdr = val[1][p], dvpdr = val[2][p];
+            const double dvrdt = val[3][p], dvrdp = val[4][p], dvtdp = val[5][p];
+            if (ph.conv_nl && !curl) {
+                // u . grad u (src/get_nl.f90:274-308)
+                adv[0][p] += -or2 * orho1 * (vr * (dvrdr - (2.0 * or1 + beta) * vr) +
+                                             o2 * (vt * (dvrdt - r * vt) + vp * (dvrdp - r * vp)));
+                adv[1][p] += or4 * orho1 * (-vr * (dvtdr - beta * vt) + vt * (cosn2 * vt + dvpdp[p] + dvrdr) +
+                                            vp * (cosn2 * vp - dvtdp));
+                adv[2][p] += or4 * orho1 * (-vr * (dvpdr - beta * vp) - vt * (dvtdp + cvr[p]) - vp * dvpdp[p]);
+            }
+            if (ph.anel) {
+                // viscous heating (src/get_nl.f90:402-425)
+                const double t1 = dvrdr - (2.0 * or1 + beta) * vr;
+                const double t2 = cosn2 * vt + dvpdp[p] + dvrdr - or1 * vr;
+                const double t3 = dvpdp[p] + cosn2 * vt + or1 * vr;
+                const double t6 = 2.0 * dvtdp + cvr[p] - 2.0 * cosn2 * vp;
+                const double t4 = r * dvtdr - (2.0 + beta * r) * vt + or1 * dvrdt;
+                const double t5 = r * dvpdr - (2.0 + beta * r) * vp + or1 * dvrdp;
+                const double bv = beta * vr;
+                heat[p] = vh * (2.0 * (t1 * t1) + 2.0 * (t2 * t2) + 2.0 * (t3 * t3) + t6 * t6 +
+                                o2 * (t4 * t4 + t5 * t5) - 2.0 * (1.0 / 3.0) * (bv * bv));
+            }
+        }
+    }
+    // M; the Courant maxima (src/courant.f90:209-275, XSH_COURANT = 0)
+    const bool mag = in[RI_BR] >= 0;
+    if (mag) inverse6(in[RI_BR], in[RI_BT], in[RI_BP], in[RI_CBR], in[RI_CBT], in[RI_CBP]);
+    else RL_EACH(val[0][p] = val[1][p] = val[2][p] = 0.0)
+    if (a.cmax) {
+        const double orho2 = orho1 * orho1;
+        const double vri2 = rad[RR_VALRI2 * nlev + lev], vhi2 = rad[RR_VALHI2 * nlev + lev];
+        double mr = 0.0, mh = 0.0;
+#pragma unroll
+        for (int p = 0; p < NPT; ++p) {
+            if (tid + p / 2 * nthr >= M) continue;
+            const double vflr2 = orho2 * u[0][p] * u[0][p];
+            const double vflh2 = (u[1][p] * u[1][p] + u[2][p] * u[2][p]) * o2 * orho2;
+            if (ph.cour_mag) {
+                const double br = val[0][p], bt = val[1][p], bp = val[2][p];
+                const double valr = br * br * ph.LFfac * orho1;
+                mr = fmax(mr, or4 * (ph.cf2 * vflr2 + ph.af2 * (valr * valr / (valr + vri2))));
+                const double valh2 = (bt * bt + bp * bp) * ph.LFfac * o2 * orho1;
+                mh = fmax(mh, or2 * (ph.cf2 * vflh2 + ph.af2 * (valh2 * valh2 / (valh2 + vhi2))));
+            } else {
+                mr = fmax(mr, ph.cf2 * or4 * vflr2);
+                mh = fmax(mh, ph.cf2 * or2 * vflh2);
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            mr = fmax(mr, __shfl_xor(mr, off, 64));
+            mh = fmax(mh, __shfl_xor(mh, off, 64));
+        }
+        if ((threadIdx.x & 63) == 0) {
+            atomicMax(a.cmax + 2 * lev, (unsigned long long)__double_as_longlong(mr));
+            atomicMax(a.cmax + 2 * lev + 1, (unsigned long long)__double_as_longlong(mh));
+        }
+    }
+    {
+        const bool lf = mag && ph.mag_LF && !lcr;
+        const double oh = ph.OhmLossFac * or2 * rad[RR_OTEMP1 * nlev + lev] * rad[RR_LAMBDA * nlev + lev];
+#pragma unroll
+        for (int p = 0; p < NPT; ++p) {
+            const double br = val[0][p], bt = val[1][p], bp = val[2][p];
+            if (mag) {
+                const double cbr = val[3][p], cbt = val[4][p], cbp = val[5][p];
+                if (lf) {
+                    // Lorentz force (src/get_nl.f90:242-258)
+                    adv[0][p] += ph.LFfac * o2 * (cbt * bp - cbp * bt);
+                    adv[1][p] += ph.LFfac * or4 * (cbp * br - cbr * bp);
+                    adv[2][p] += ph.LFfac * or4 * (cbr * bt - cbt * br);
+                }
+                // Ohmic losses (src/get_nl.f90:426-436)
+                if (ph.anel && ph.mag_nl && !lcr)
+                    heat[p] += oh * (or2 * (cbr * cbr) + o2 * (cbt * cbt) + o2 * (cbp * cbp));
+            }
+            // V x B (src/get_nl.f90:376-388), outside the conducting region its
+            // horizontal part only (:389-391)
+            const double vr = u[0][p], vt = u[1][p], vp = u[2][p];
+            val[3][p] = lcr ? 0.0 : orho1 * o2 * (vt * bp - vp * bt);
+            val[4][p] = lcr ? or4 * orho1 * vp * br : orho1 * or4 * (vp * br - vr * bp);
+            val[5][p] = lcr ? -or4 * orho1 * vt * br : orho1 * or4 * (vr * bt - vt * br);
+            val[0][p] = adv[0][p];
+            val[1][p] = adv[1][p];
+            val[2][p] = adv[2][p];
+        }
+    }
+    if (out[RO_ADVR] >= 0 || out[RO_VXBR] >= 0)
+        forward6(out[RO_ADVR], out[RO_ADVT], out[RO_ADVP], out[RO_VXBR], out[RO_VXBT], out[RO_VXBP]);
+    if (out[RO_HEAT] >= 0) {
+        RL_EACH(val[0][p] = heat[p])
+        forward6(out[RO_HEAT], -1, -1, -1, -1, -1);
+    }
+#undef RL_EACH
 }
 
 FFTArgs make_args(const Plan *p)
@@ -1129,16 +1346,20 @@ int launch_nl_fused(const Plan *p, int nlev, const void *Fin, void *Fout, const 
 }
 
 template <int A, int B>
-int launch_rl_slots(const Plan *p, const FFTArgs &f, const RlGridArgs &a, size_t shm, hipStream_t s)
+int launch_rl_slots(const Plan *p, const FFTArgs &f, const RlGridArgs &a, hipStream_t s)
 {
-    static int shm_set = 0;
-    if (shm > 64 * 1024 && (int)shm > shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_rl_grid_s<A, B>,
+    typedef SlotFFT<A, B> FFT;
+    constexpr int M = FFT::M, NR = FFT::NR;
+    constexpr size_t shm = ((size_t)2 * M + M / 8 + 1 + NR * (size_t)FFT::row_stride(padded_row<M, FFT::P>())) * sizeof(double2);
+    // set once per kernel (the attribute persists)
+    static bool shm_set = false;
+    if (shm > 64 * 1024 && !shm_set) {
+        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_rl_slots<A, B>,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        shm_set = (int)shm;
+        shm_set = true;
     }
-    dim3 grid((unsigned)(p->n_theta * a.nlev));
-    k_rl_grid_s<A, B><<<grid, 512, shm, s>>>(f, a);
+    dim3 grid((unsigned)((p->n_theta + NR - 1) / NR * a.nlev));
+    k_rl_slots<A, B><<<grid, FFT::NTHR, shm, s>>>(f, a);
     MHX_HIP_CHECK(hipGetLastError());
     return MHX_OK;
 }
@@ -1152,25 +1373,22 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &args, hipStream_t s)
     const int nrow = std::max(a.nin, a.nout);
     if (nrow <= 0 || nrow > 32) return fail(MHX_E_INVALID, "radial loop: bad component count");
     const size_t lds_max = 160 * 1024;
-    // rows of M = 3 4^A 2^B: wave-slot FFTs on padded rows, all rows at once,
-    // when they fit the LDS (measured at l_max = 255 x 97, Boussinesq MHD:
-    // 10.2 -> 8.7 ms per mhx_rloop call against the block-wide FFTs below)
+    // rows of M = 3 4^A 2^B, M <= 768: wave-slot FFTs in rounds, where the rows
+    // of all components would fit the LDS too
     {
         int A, B;
-        if (slot_form(p, A, B)) {
-            const int M = p->M, P = M / 12 <= 64 ? 12 : M / 64;
-            const size_t MP = P == 12 ? (size_t)M + (M >> 5) + 1 : (size_t)M;
-            const size_t shm = ((size_t)2 * M + M / 8 + 1 + (size_t)nrow * MP) * cs;
-            if (shm <= lds_max) {
+        if (slot_form(p, A, B) && p->M <= 768) {
+            const int M = p->M;
+            const size_t MP = (size_t)M + (M >> 5) + 1;
+            if (((size_t)2 * M + M / 8 + 1 + (size_t)nrow * MP) * cs <= lds_max) {
                 switch (2 * A + B) {
-                case 2: return launch_rl_slots<1, 0>(p, f, a, shm, s);
-                case 3: return launch_rl_slots<1, 1>(p, f, a, shm, s);
-                case 4: return launch_rl_slots<2, 0>(p, f, a, shm, s);
-                case 5: return launch_rl_slots<2, 1>(p, f, a, shm, s);
-                case 6: return launch_rl_slots<3, 0>(p, f, a, shm, s);
-                case 7: return launch_rl_slots<3, 1>(p, f, a, shm, s);
-                case 8: return launch_rl_slots<4, 0>(p, f, a, shm, s);
-                case 9: return launch_rl_slots<4, 1>(p, f, a, shm, s);
+                case 2: return launch_rl_slots<1, 0>(p, f, a, s);
+                case 3: return launch_rl_slots<1, 1>(p, f, a, s);
+                case 4: return launch_rl_slots<2, 0>(p, f, a, s);
+                case 5: return launch_rl_slots<2, 1>(p, f, a, s);
+                case 6: return launch_rl_slots<3, 0>(p, f, a, s);
+                case 7: return launch_rl_slots<3, 1>(p, f, a, s);
+                case 8: return launch_rl_slots<4, 0>(p, f, a, s);
                 default: break;
                 }
             }

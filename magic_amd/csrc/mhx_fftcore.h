@@ -167,7 +167,6 @@ __device__ __forceinline__ void wave_order()
     asm volatile("" ::: "memory");
 }
 
-
 // Courant maxima of one level (src/courant.f90:209-275, magnetic branch with
 // the Alfven damping terms valri2/valhi2): over this thread's points the
 // maxima of or4 (cf^2 orho2 vr^2 + af^2 valr^2 / (valr + valri2)) and or2

@@ -10,6 +10,7 @@ import pytest
 from conftest import rel_l2
 from magic_amd import sht, workload
 from nl_reference import oracle_step, radial
+import rloop_cases as rc
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +87,41 @@ def test_nl_step_matches_oracle(L, nt, nph, minc, nlev):
     for k in range(18):
         assert rel_l2(grids[:, k].cpu().numpy(), want_g[:, k]) < TOL, sht.NL_GRIDS[k]
     p.close()
+
+
+# the radial loop's grid stage: slots of 2, 4, 16 and 32 lanes, block-wide
+# passes (n_phi = 160), under the switches of every dump of the reference
+@pytest.mark.parametrize("case", rc.CASES)
+@pytest.mark.parametrize("L,nt,nph", [(15, 24, 48), (15, 28, 96), (20, 36, 160), (30, 44, 384), (20, 36, 768)])
+def test_rloop_matches_oracle(case, L, nt, nph):
+    """Two interior levels, one cut below l_max, against the oracle's radial
+    loop.  The Courant steps and explicit terms are held to 1e-11, the bar of
+    the loop's comparison at l_max = 255: the Lorentz force and the Coriolis
+    terms of the dumps' parameters cancel a few digits."""
+    from oracle import oracle
+    from rloop_reference import oracle_rloop
+    nlev = 2
+    ph = rc.phys_of(rc.load(case))
+    print("rloop", case, L, nt, nph, flush=True)
+    ins = workload.nl_inputs(L, nlev, stream=13)
+    fields = {n: None for n in sht.RLOOP_IN}
+    fields.update(dict(zip(sht.NL_INPUTS, ins)))
+    fields["xi"] = np.stack([workload.coefficients(L, 13, 20, i, potential=False) for i in range(nlev)])
+    fields["phi"] = np.stack([workload.coefficients(L, 13, 21, i, potential=False) for i in range(nlev)])
+    r = np.array([0.8, 1.2])
+    one = np.ones(nlev)
+    rad = {"r": r, "or1": 1 / r, "or2": 1 / r ** 2, "or4": 1 / r ** 4, "orho1": 1 / (1 + 0.1 * r),
+           "beta": -0.1 / (1 + 0.1 * r), "otemp1": 1 / (1.5 - 0.2 * r), "visc": one, "lambda": 1 + 0.1 * r,
+           "temp0": one, "epscProf": one, "delxr2": np.full(nlev, 1e-3), "delxh2": np.full(nlev, 2e-2),
+           "nR": np.array([5, 9], dtype=np.int32), "l_R": np.array([L, L - 2], dtype=np.int32)}
+    names = rc.outputs_of(dict(ph, **{k: ph.get(k, 0) for k in sht.RLOOP_INT}))
+    p = sht.Plan(L, nt, nph, max_levels=nlev)
+    outs = {n: np.zeros((nlev, p.lm_max), dtype=np.complex128) for n in names}
+    dtr, dth = np.zeros(nlev), np.zeros(nlev)
+    sht.rloop(p, ph, nlev, rad, fields, outs, dtr, dth)
+    p.close()
+    o = oracle.Plan(L, nt, nph)
+    want, wtr, wth = oracle_rloop(o, ph, nlev, rad, fields, 1)
+    for n in names:
+        assert rel_l2(outs[n], want[n]) < 1e-11, n
+    assert rel_l2(dtr, wtr) < 1e-11 and rel_l2(dth, wth) < 1e-11
