@@ -67,6 +67,17 @@ __device__ inline d4 mfma64(double a, double b, d4 c)
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// x of the lane before (wave_shr:1), after (wave_shl:1) and of the other lane of
+// the pair (quad_perm 1 0 3 2), by data-parallel moves: no LDS permutation
+template <int CTRL> __device__ __forceinline__ double dpp(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int DPP_PREV = 0x138, DPP_NEXT = 0x130, DPP_PAIR = 0xb1;
+
 // ------------------------------------------------------------- synthesis
 __device__ inline double2 czero() { return make_double2(0.0, 0.0); }
 __device__ inline double2 cimul(double m, double2 z) { return make_double2(-m * z.y, m * z.x); }  // i m z
@@ -162,8 +173,8 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
             const double fm = (double)(l - 1) * cr[0], fp = (double)(l + 2) * cr[1];
             // x' from the neighbours of x
             auto prime = [&](double2 x, double2 h) {
-                double2 lo = make_double2(__shfl_up(x.x, 1, 32), __shfl_up(x.y, 1, 32));
-                double2 hi = make_double2(__shfl_down(x.x, 1, 32), __shfl_down(x.y, 1, 32));
+                double2 lo = make_double2(dpp<DPP_PREV>(x.x), dpp<DPP_PREV>(x.y));
+                double2 hi = make_double2(dpp<DPP_NEXT>(x.x), dpp<DPP_NEXT>(x.y));
                 if (j == 0) lo = h;
                 if (j == 31) hi = h;
                 return make_double2(fm * lo.x - fp * hi.x, fm * lo.y - fp * hi.y);
@@ -259,7 +270,7 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
             for (int pr = 0; pr < NP; ++pr) {
                 const double n = acc[s][pr][0][jj] + acc[s][pr][1][jj];
                 const double so = acc[s][pr][0][jj] - acc[s][pr][1][jj];
-                const double other = __shfl_xor(odd ? n : so, 1, 64);
+                const double other = dpp<DPP_PAIR>(odd ? n : so);
                 double2 v = odd ? make_double2(other, so) : make_double2(n, other);
                 if (job.row_scale) v = make_double2(sc * v.x, sc * v.y);
                 auto store = [&](int o, double2 w) {
