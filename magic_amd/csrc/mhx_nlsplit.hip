@@ -105,11 +105,21 @@ template <> struct NSyn<NS_QSTC> {
 // exponent is renormalised once per chunk, so no value leaves the double
 // range however small P_mm is).  The coefficients of the block's order sit
 // in LDS.
+//
+// Stored tables (!REC): one theta tile per wave, eight waves per block, so that
+// the accumulators (48 registers) leave 128 per wave and two blocks, 16 waves, run
+// per CU: the blocks wait on their sources and table fragments, chunk by chunk, and
+// only other waves cover that.  Two tiles per wave (226 registers, one block of six
+// waves per CU) took 490 / 510 / 394 us for QST / QSTC / SG at l_max = 511 x 32
+// levels, this 294 / 346 / 217 (1.1 GB of tables, sources and Fourier data: 3.9
+// TB/s).  Fragments loaded a step ahead instead cost the second block
+// or spill: the whole step 5.4 -> 6.2 - 8.3 ms.
 constexpr int RLMAX = 1152;  // coefficient entries l - m (l_max <= 1023)
 
 template <int V, bool REC>
-__global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
+__global__ __launch_bounds__(REC ? 256 : 512, REC ? 2 : 4) void k_nsyn16(NSynArgs a)
 {
+    constexpr int TW = REC ? 2 : 1;  // theta tiles per wave
     using S = NSyn<V>;
     constexpr int NPL = S::NPL, NOUT = S::NOUT, NPROD = S::NPROD, NSRC = S::NSRC;
     __shared__ __align__(16) _Float16 bhi[NPL * PLANE];
@@ -180,25 +190,25 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
     __syncthreads();
     if (tid < 2 * LGS) lvsc[tid] = bscale((double)__uint_as_float(lvmax[tid]));
 
-    f4 acc[NOUT][2][2][TNC];  // [out][Sym/Anti][theta tile][column tile]
+    f4 acc[NOUT][2][TW][TNC];  // [out][Sym/Anti][theta tile][column tile]
 #pragma unroll
     for (int o = 0; o < NOUT; ++o)
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < TW; ++t)
 #pragma unroll
                 for (int n = 0; n < TNC; ++n) acc[o][s][t][n] = f4{0.f, 0.f, 0.f, 0.f};
-    const int tile0 = gz * a.tpb + wave * 2;
-    bool tok[2];
-    tok[0] = tile0 < a.nt16;
-    tok[1] = tile0 + 1 < a.nt16;
+    const int tile0 = gz * a.tpb + wave * TW;
+    bool tok[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) tok[t] = tile0 + t < a.nt16;
 
     // REC: recurrence coefficients (A_l, eps_l), l = m + i, zero past l_max + 1
     __shared__ double2 rco[REC ? RLMAX : 1];
     const int rg = lane >> 4;  // lane group: l offset 16 rg within a chunk
-    double rp[2], rq[2], rct[2], reps = 0.0;  // P_{l-1}, P_l (x 2^-E), cos(theta), eps_l
-    int rE[2];
+    double rp[TW], rq[TW], rct[TW], reps = 0.0;  // P_{l-1}, P_l (x 2^-E), cos(theta), eps_l
+    int rE[TW];
     if constexpr (REC) {
         for (int i = tid; i < RLMAX; i += nthr) {
             const int l = m + i;
@@ -212,7 +222,7 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
             rco[i] = make_double2(A, e);
         }
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+        for (int tt = 0; tt < TW; ++tt) {
             const int th = (tile0 + tt) * 16 + (lane & 15);
             const bool ok = tok[tt] && th < a.nh;
             const double2 sd = ok ? a.seed[(size_t)mc * a.nh + th] : make_double2(0.0, 0.0);
@@ -227,7 +237,7 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
             if (j < 16 * rg) {
                 const double2 ce = rco[j + 1];
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
+                for (int tt = 0; tt < TW; ++tt) {
                     const double pn = ce.x * (rct[tt] * rq[tt] - reps * rp[tt]);
                     rp[tt] = rq[tt];
                     rq[tt] = pn;
@@ -237,34 +247,55 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
         }
     }
 
+    // stored tables: fragments [theta tile][P hi, P lo, dP hi, dP lo] of a chunk
+    // and parity
+    h8 f[TW][4];
+    auto load_tab = [&](int c, int par) {
+#pragma unroll
+        for (int tt = 0; tt < TW; ++tt) {
+            if (!tok[tt]) continue;
+            const size_t to = a.off[2 * mc + par] + (((size_t)c * a.nt16 + tile0 + tt) * 64 + lane) * 16;
+            f[tt][0] = *reinterpret_cast<const h8 *>(a.tP + to);
+            f[tt][1] = *reinterpret_cast<const h8 *>(a.tP + to + 8);
+            f[tt][2] = *reinterpret_cast<const h8 *>(a.tdP + to);
+            f[tt][3] = *reinterpret_cast<const h8 *>(a.tdP + to + 8);
+        }
+    };
+    // sources of the chunk: this thread's four l, all loads issued first at
+    // addresses clamped into the order's range, masked when staged
+    constexpr int SPAR = REC ? 2 : 1;  // parities per staging thread
+    const int sg = tid & 15, slevl = (tid >> 4) & (LGS - 1), spar0 = REC ? 0 : tid >> 8;
+    const bool slok = slevl < nlh;
+    double2 xv[SPAR][2][NSRC];  // [par][q][source]
+    auto load_src = [&](int c) {
+#pragma unroll
+        for (int par = 0; par < SPAR; ++par)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int l = min(m + 64 * c + 4 * sg + 2 * q + spar0 + par, a.l_max);
+                const size_t o = ((size_t)(slok ? lev0 + slevl : 0) * a.src_ld + (size_t)(l0 + l - m)) * 2;
+#pragma unroll
+                for (int s2 = 0; s2 < NSRC; ++s2)
+                    xv[par][q][s2] = *reinterpret_cast<const double2 *>(a.src[s2] + o);
+            }
+    };
     for (int c = 0; c < nks0; ++c) {
         __syncthreads();  // lvsc ready / previous chunk consumed
         // ---- stage l = m + 64 c + 4 g + j (j < 4) for LGS levels: 16 LGS
         // threads; parity par = j & 1 holds k = 32 c + 2 g + (j >> 1)
-        if (tid < 16 * LGS) {
-            const int g = tid & 15, levl = tid >> 4;
+        {
+            const int g = sg, levl = slevl;
             const int lev = lev0 + levl;
-            const bool lok = levl < nlh;
+            const bool lok = slok;
             const int lhi = lok ? min(a.l_max, a.lcut[lev]) : -1;
             const double o2 = (V == NS_QSTC && lok) ? a.or2[lev] : 0.0;
             const float sc0 = lvsc[levl], sc1 = lvsc[LGS + levl];
             const float fm = (float)dm;
-            // the four l of this thread, all loads issued first at addresses
-            // clamped into the order's range, then masked
-            double2 xv[2][2][NSRC];  // [par][q][source]
-#pragma unroll
-            for (int par = 0; par < 2; ++par)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const int l = min(m + 64 * c + 4 * g + 2 * q + par, a.l_max);
-                    const size_t o = ((size_t)(lok ? lev : 0) * a.src_ld + (size_t)(l0 + l - m)) * 2;
-#pragma unroll
-                    for (int s2 = 0; s2 < NSRC; ++s2)
-                        xv[par][q][s2] = *reinterpret_cast<const double2 *>(a.src[s2] + o);
-                }
+            load_src(c);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int par = 0; par < 2; ++par) {
+            for (int sp = 0; sp < SPAR; ++sp) {
+                const int par = spar0 + sp;
                 // planes of the two l of this parity, FP32, scaled
                 float pr[NPL][2], pi[NPL][2];
 #pragma unroll
@@ -274,8 +305,8 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
                     double xr[NSRC], xi[NSRC];
 #pragma unroll
                     for (int s2 = 0; s2 < NSRC; ++s2) {
-                        xr[s2] = valid ? xv[par][q][s2].x : 0.0;
-                        xi[s2] = valid ? xv[par][q][s2].y : 0.0;
+                        xr[s2] = valid ? xv[sp][q][s2].x : 0.0;
+                        xi[s2] = valid ? xv[sp][q][s2].y : 0.0;
                     }
                     const double ll = (double)l * (double)(l + 1);
                     if constexpr (V == NS_SG) {
@@ -326,7 +357,7 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
             const int i0 = 64 * c + 16 * rg;
             const double dl0 = (double)(m + i0), reps0 = reps, dlmax = (double)a.l_max;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
+            for (int tt = 0; tt < TW; ++tt) {
                 if (!tok[tt]) continue;
                 // renormalise: |P| within [2^-256, 2^256] x 2^E at the chunk start
                 {
@@ -404,18 +435,7 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
 #pragma unroll
         for (int par = 0; par < 2; ++par) {
             if (c >= (par ? nks1 : nks0)) continue;
-            h8 aPh[2], aPl[2], adPh[2], adPl[2];
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                if (tok[tt]) {
-                    const size_t to = a.off[2 * mc + par] +
-                                      (((size_t)c * a.nt16 + tile0 + tt) * 64 + lane) * 16;
-                    aPh[tt] = *reinterpret_cast<const h8 *>(a.tP + to);
-                    aPl[tt] = *reinterpret_cast<const h8 *>(a.tP + to + 8);
-                    adPh[tt] = *reinterpret_cast<const h8 *>(a.tdP + to);
-                    adPl[tt] = *reinterpret_cast<const h8 *>(a.tdP + to + 8);
-                }
-            }
+            load_tab(c, par);
 #pragma unroll
             for (int tn = 0; tn < TNC; ++tn) {
                 if (tn >= ntn) break;
@@ -427,10 +447,10 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
                     const h8 bh = *reinterpret_cast<const h8 *>(bhi + bo);
                     const h8 bl = *reinterpret_cast<const h8 *>(blo + bo);
 #pragma unroll
-                    for (int tt = 0; tt < 2; ++tt) {
+                    for (int tt = 0; tt < TW; ++tt) {
                         if (!tok[tt]) continue;
-                        const h8 ah = tab == 0 ? aPh[tt] : adPh[tt];
-                        const h8 al = tab == 0 ? aPl[tt] : adPl[tt];
+                        const h8 ah = f[tt][tab == 0 ? 0 : 2];
+                        const h8 al = f[tt][tab == 0 ? 1 : 3];
                         f4 t = acc[o][tgt][tt][tn];
                         t = mfma16(ah, bl, t);
                         t = mfma16(al, bh, t);
@@ -443,30 +463,48 @@ __global__ __launch_bounds__(REC ? 256 : 384, 2) void k_nsyn16(NSynArgs a)
     }
 
     // ---- epilogue: north = Sym + Anti, south = Sym - Anti; remove the row
-    // and level factors; F[lev][comp][m][theta] FP32 complex
+    // and level factors; F[lev][comp][m][theta] FP32 complex.  After one exchange
+    // with its re/im partner a lane owns two theta_h (j = p + 2 ri) and stores
+    // the complex (North, South) pair of each as 16 contiguous bytes
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
+    for (int tt = 0; tt < TW; ++tt) {
         if (!tok[tt]) continue;
 #pragma unroll
         for (int tn = 0; tn < TNC; ++tn) {
             if (tn >= ntn) break;
             const int n = tn * 16 + (lane & 15), levl = n >> 1, ri = n & 1;
-            if (levl >= nlh) continue;
+            const bool lvok = levl < nlh;
             const float inv0 = 1.f / lvsc[levl], inv1 = 1.f / lvsc[LGS + levl];
-            float *fo = a.fout + (size_t)(lev0 + levl) * a.fout_ld * 2;
+            float *fo = a.fout + (size_t)(lev0 + (lvok ? levl : 0)) * a.fout_ld * 2;
+            float rrs[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int th = (tile0 + tt) * 16 + 4 * (lane >> 4) + j;
-                if (th >= a.nh) continue;
-                const float rrs = 1.f / a.rowscale[(size_t)mc * a.nh + th];
+                rrs[j] = 1.f / a.rowscale[(size_t)mc * a.nh + min(th, a.nh - 1)];
+            }
 #pragma unroll
-                for (int o = 0; o < NOUT; ++o) {
-                    const float rs = rrs * (S::ogrp[o] ? inv1 : inv0);
-                    const size_t base =
-                        (((size_t)(a.comp0 + o) * a.n_m + mc) * a.n_theta + 2 * th) * 2;
+            for (int o = 0; o < NOUT; ++o) {
+                float vn[4], vs[4];  // North, South of this lane's re or im part
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float rs = rrs[j] * (S::ogrp[o] ? inv1 : inv0);
                     const float sy = acc[o][0][tt][tn][j], an = acc[o][1][tt][tn][j];
-                    fo[base + ri] = (sy + an) * rs;
-                    fo[base + 2 + ri] = (sy - an) * rs;
+                    vn[j] = (sy + an) * rs;
+                    vs[j] = (sy - an) * rs;
+                }
+                const size_t base = ((size_t)(a.comp0 + o) * a.n_m + mc) * a.n_theta * 2;
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const float on = ri ? vn[p + 2] : vn[p], os = ri ? vs[p + 2] : vs[p];
+                    const float gn = __shfl_xor(ri ? vn[p] : vn[p + 2], 1);
+                    const float gs = __shfl_xor(ri ? vs[p] : vs[p + 2], 1);
+                    const int th = (tile0 + tt) * 16 + 4 * (lane >> 4) + p + 2 * ri;
+                    f4 w;
+                    w[0] = ri ? gn : on;
+                    w[1] = ri ? on : gn;
+                    w[2] = ri ? gs : os;
+                    w[3] = ri ? os : gs;
+                    if (lvok && th < a.nh) *reinterpret_cast<f4 *>(fo + base + 4 * th) = w;
                 }
             }
         }
@@ -914,9 +952,17 @@ constexpr int ROWA = 32 + 8;   // halves per LDS row of generated fragments (pad
 constexpr int RNG = 1;         // level groups per block with generated fragments
 constexpr int RLB = 256 + 8;   // recurrence coefficients held per block
 
+// a complex value at 8-byte alignment (the caller's arrays)
+struct cpair { double x, y; };
+
+// Stored tables: one l tile per wave, eight waves per block, two blocks per CU, for
+// the reason given at k_nsyn16, and whole complex values stored (8-byte halves wrote
+// 468 MB for 201): QST 612 -> 505 us, SH 192 -> 170 at l_max = 511 x 32 levels
+// (1.4 GB: 2.7 TB/s; what is left is the wait on each chunk's loads).
 template <int V, bool REC>
-__global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
+__global__ __launch_bounds__(REC ? 256 : 512, REC ? 1 : 4) void k_nana16(NAnaArgs a)
 {
+    constexpr int TW = REC ? 2 : 1;  // l tiles per wave
     using S = NAna<V>;
     constexpr int NPL = S::NPL, NOUT = S::NOUT, NPROD = S::NPROD, NIN = S::NIN;
     constexpr bool DP = V == NA_QST;  // dP fragments needed
@@ -946,11 +992,11 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
     const int l0 = a.lstart[mc];
     const int K0 = (a.l_max - m) / 2 + 1;
     const int ntl = (K0 + 15) / 16;           // l tiles per parity
-    const int t0 = gz * 8 + wave * 2;         // this wave's l tiles t0, t0+1
+    const int t0 = gz * 8 + wave * TW;        // this wave's first l tile
     if (gz * 8 >= ntl) return;                // no l tile of this order here
-    bool tok[2];
-    tok[0] = t0 < ntl;
-    tok[1] = t0 + 1 < ntl;
+    bool tok[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) tok[t] = t0 + t < ntl;
     if constexpr (REC) {
         for (int i = tid; i < RLB; i += nthr) {
             const int l = m + 256 * gz + i;
@@ -1009,7 +1055,7 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
         lvsc[tid] = bscale(f * (double)__uint_as_float(lvmax[tid]));
     }
 
-    f4 acc[NG][NOUT][2][2][2];  // [level group][out][parity][l tile][column tile]
+    f4 acc[NG][NOUT][2][TW][2];  // [level group][out][parity][l tile][column tile]
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
@@ -1017,7 +1063,7 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
 #pragma unroll
             for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < TW; ++t)
 #pragma unroll
                     for (int n = 0; n < 2; ++n) acc[g][o][s][t][n] = f4{0.f, 0.f, 0.f, 0.f};
 
@@ -1026,7 +1072,7 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
     bool stage_lev_ok[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-        const int levl = tid >> 4;
+        const int levl = (tid >> 4) & (LGS - 1);
         stage_lev_ok[g] = false;
         if (levl < nlh_of(g)) {
             const int lc = a.lcut[levb + LGS * g + levl];
@@ -1046,6 +1092,38 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
         nE = a.aexp[seg_base + th0];
         nx = a.cost[th0];
     }
+    // stored tables: fragments [l tile][P hi, P lo, dP hi, dP lo] of a chunk
+    // and parity
+    h8 f[TW][4];
+    auto load_tab = [&](int kc, int par) {
+#pragma unroll
+        for (int tt = 0; tt < TW; ++tt) {
+            if (!tok[tt]) continue;
+            const size_t to = a.off[2 * mc + par] + (((size_t)(t0 + tt) * a.nq32 + kc) * 64 + lane) * 16;
+            f[tt][0] = *reinterpret_cast<const h8 *>(a.tP + to);
+            f[tt][1] = *reinterpret_cast<const h8 *>(a.tP + to + 8);
+            if constexpr (DP) {
+                f[tt][2] = *reinterpret_cast<const h8 *>(a.tdP + to);
+                f[tt][3] = *reinterpret_cast<const h8 *>(a.tdP + to + 8);
+            }
+        }
+    };
+    // F2 values of the chunk for this thread, loads issued unconditionally at
+    // clamped addresses (level and theta block in range; the second row pair of
+    // a block is padding past n_theta), masked when staged
+    f4 xv0[NIN], xv1[NIN];
+    auto load_f2 = [&](int kc, int sg) {
+        const int q = tid & 3, tb = (tid >> 2) & 3, levl = (tid >> 4) & (LGS - 1);
+        const int lev = levb + LGS * sg + levl, thb = kc * 4 + tb;
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) {
+            const size_t o = ((size_t)(levl < nlh_of(sg) ? lev : 0) * a.fin_ld +
+                              (((size_t)a.in_comp[k] * a.ntb + min(thb, a.ntb - 1)) * a.n_m + mc) * 16 +
+                              4 * q) * 2;
+            xv0[k] = *reinterpret_cast<const f4 *>(fin + o);
+            xv1[k] = *reinterpret_cast<const f4 *>(fin + o + 4);
+        }
+    };
     // F2 layout: [lev][comp][theta block of 16 rows][m][16] complex
     for (int kc = 0; kc < a.nq32; ++kc) {
         __syncthreads();
@@ -1101,27 +1179,14 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
         const int ntn = nlh > 8 ? 2 : 1;
         // ---- stage theta_h = 32 kc + 8 tb + 2 q + (0, 1): rows 64 kc + 16 tb + 4 q .. +3
         {
-            const int q = tid & 3, tb = (tid >> 2) & 3, levl = tid >> 4;
-            const int lev = lev0 + levl;
-            const int thb = kc * 4 + tb;        // theta block (16 rows)
+            const int q = tid & 3, tb = (tid >> 2) & 3, levl = (tid >> 4) & (LGS - 1);
             const int th0 = 32 * kc + 8 * tb + 2 * q;
             const bool valid = stage_lev_ok[sg] && th0 < a.nh;
             const bool ok1 = th0 + 1 < a.nh;  // rows past n_theta are padding
             const float sc0 = lvsc[sg * 2 * LGS + levl], sc1 = lvsc[sg * 2 * LGS + LGS + levl];
             // rows 2 th, 2 th + 1 for th = th0, th0 + 1: 4 complex, 32 bytes
             float x[NIN][8];
-            // loads issued unconditionally at clamped addresses (level and
-            // theta block in range; the second row pair of a block is padding
-            // past n_theta), then masked
-            f4 xv0[NIN], xv1[NIN];
-#pragma unroll
-            for (int k = 0; k < NIN; ++k) {
-                const size_t o = ((size_t)(levl < nlh ? lev : 0) * a.fin_ld +
-                                  (((size_t)a.in_comp[k] * a.ntb + min(thb, a.ntb - 1)) * a.n_m + mc) * 16 +
-                                  4 * q) * 2;
-                xv0[k] = *reinterpret_cast<const f4 *>(fin + o);
-                xv1[k] = *reinterpret_cast<const f4 *>(fin + o + 4);
-            }
+            load_f2(kc, sg);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < NIN; ++k) {
@@ -1138,7 +1203,8 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
             const float fm = (float)dm;
             const int kk = 8 * tb + 2 * q;  // theta_h within the chunk
 #pragma unroll
-            for (int sa = 0; sa < 2; ++sa) {
+            for (int sp = 0; sp < (REC ? 2 : 1); ++sp) {
+                const int sa = REC ? sp : tid >> 8;  // wave-uniform
                 float pr[NPL][2], pi[NPL][2];
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
@@ -1181,27 +1247,16 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
         // ---- contraction
 #pragma unroll
         for (int par = 0; par < 2; ++par) {
-            h8 aPh[2], aPl[2], adPh[2], adPl[2];
+            if constexpr (REC) {
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                if constexpr (REC) {
+                for (int tt = 0; tt < TW; ++tt) {
                     const int ai = (par * 128 + 16 * (wave * 2 + tt) + (lane & 15)) * ROWA + 8 * (lane >> 4);
-                    aPh[tt] = *reinterpret_cast<const h8 *>(gA + ai);
-                    aPl[tt] = *reinterpret_cast<const h8 *>(gA + 2 * 128 * ROWA + ai);
-                    if constexpr (DP) {
-                        adPh[tt] = *reinterpret_cast<const h8 *>(gA + 4 * 128 * ROWA + ai);
-                        adPl[tt] = *reinterpret_cast<const h8 *>(gA + 6 * 128 * ROWA + ai);
-                    }
-                } else if (tok[tt]) {
-                    const size_t to = a.off[2 * mc + par] +
-                                      (((size_t)(t0 + tt) * a.nq32 + kc) * 64 + lane) * 16;
-                    aPh[tt] = *reinterpret_cast<const h8 *>(a.tP + to);
-                    aPl[tt] = *reinterpret_cast<const h8 *>(a.tP + to + 8);
-                    if constexpr (V == NA_QST) {
-                        adPh[tt] = *reinterpret_cast<const h8 *>(a.tdP + to);
-                        adPl[tt] = *reinterpret_cast<const h8 *>(a.tdP + to + 8);
-                    }
+#pragma unroll
+                    for (int k = 0; k < (DP ? 4 : 2); ++k)
+                        f[tt][k] = *reinterpret_cast<const h8 *>(gA + k * 2 * 128 * ROWA + ai);
                 }
+            } else {
+                load_tab(kc, par);
             }
 #pragma unroll
             for (int tn = 0; tn < 2; ++tn) {
@@ -1214,10 +1269,10 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
                     const h8 bh = *reinterpret_cast<const h8 *>(bhi + bo);
                     const h8 bl = *reinterpret_cast<const h8 *>(blo + bo);
 #pragma unroll
-                    for (int tt = 0; tt < 2; ++tt) {
+                    for (int tt = 0; tt < TW; ++tt) {
                         if (!tok[tt]) continue;
-                        const h8 ah = tab == 0 ? aPh[tt] : adPh[tt];
-                        const h8 al = tab == 0 ? aPl[tt] : adPl[tt];
+                        const h8 ah = f[tt][tab == 0 ? 0 : 2];
+                        const h8 al = f[tt][tab == 0 ? 1 : 3];
                         f4 t = acc[sg][o][par][tt][tn];
                         t = mfma16(ah, bl, t);
                         t = mfma16(al, bh, t);
@@ -1246,27 +1301,34 @@ __global__ __launch_bounds__(256) void k_nana16(NAnaArgs a)
         const bool mkeep = m <= (lc < a.m_max ? lc : a.m_max);
         const double inv0 = 1.0 / (double)lvsc[sg * 2 * LGS + levl];
         const double inv1 = 1.0 / (double)lvsc[sg * 2 * LGS + LGS + levl];
+        // after one exchange with its re/im partner a lane owns the parity ri and
+        // stores its complex value as a whole
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+        for (int tt = 0; tt < TW; ++tt) {
             if (!tok[tt]) continue;
 #pragma unroll
-            for (int par = 0; par < 2; ++par)
+            for (int j = 0; j < 4; ++j) {
+                const int kk = 16 * (t0 + tt) + 4 * (lane >> 4) + j;
+                const int l = m + ri + 2 * kk;
+                const double rrs = 1.0 / (double)a.rowscale[a.soff[2 * mc + ri] + kk];
+                const bool keep = mkeep && l <= lc;
+                const double dll = (double)l * (double)(l + 1);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int kk = 16 * (t0 + tt) + 4 * (lane >> 4) + j;
-                    const int l = m + par + 2 * kk;
-                    if (l > a.l_max) continue;
-                    const double rrs = 1.0 / (double)a.rowscale[a.soff[2 * mc + par] + kk];
-                    const bool keep = mkeep && l <= lc;
-                    const double dll = (double)l * (double)(l + 1);
-#pragma unroll
-                    for (int o = 0; o < NOUT; ++o) {
-                        const double rs = rrs * (S::ogrp[o] ? inv1 : inv0);
-                        double v = keep ? (double)acc[sg][o][par][tt][tn][j] * rs : 0.0;
-                        if (S::divll[o] && l > 0) v /= dll;
-                        a.out[o][((size_t)lev * a.out_ld + (size_t)(l0 + l - m)) * 2 + ri] = v;
+                for (int o = 0; o < NOUT; ++o) {
+                    const float a0 = acc[sg][o][0][tt][tn][j], a1 = acc[sg][o][1][tt][tn][j];
+                    const float own = ri ? a1 : a0, got = __shfl_xor(ri ? a0 : a1, 1);
+                    const double rs = rrs * (S::ogrp[o] ? inv1 : inv0);
+                    cpair w;
+                    w.x = keep ? (double)(ri ? got : own) * rs : 0.0;
+                    w.y = keep ? (double)(ri ? own : got) * rs : 0.0;
+                    if (S::divll[o] && l > 0) {
+                        w.x /= dll;
+                        w.y /= dll;
                     }
+                    if (l <= a.l_max)
+                        *reinterpret_cast<cpair *>(a.out[o] + ((size_t)lev * a.out_ld + (size_t)(l0 + l - m)) * 2) = w;
                 }
+            }
         }
       }
     }
@@ -2004,11 +2066,10 @@ int launch_nsyn16(const Plan *p, int kind, const NSynArgs &args, hipStream_t s)
         MHX_HIP_CHECK(hipGetLastError());
         return MHX_OK;
     }
-    // 12 theta tiles per block from stored tables (all of l_max = 255); 8 with
-    // the recurrence (its fragments of both parities live in registers);
-    // 256 threads stage B
-    const int nw = p->rec ? 4 : 6;
-    a.tpb = 2 * nw;
+    // 8 theta tiles per block: one per wave from stored tables, two with the
+    // recurrence (its fragments of both parities live in registers)
+    const int nw = p->rec ? 4 : 8;
+    a.tpb = 8;
     a.ngz = (p->nt16 + a.tpb - 1) / a.tpb;
     const int ng = (a.nlev + LGS - 1) / LGS;
     dim3 grid((unsigned)(8 * ((p->n_m + 7) / 8) * ng * a.ngz));
@@ -2090,8 +2151,8 @@ int launch_nana16(const Plan *p, int kind, const NAnaArgs &args, hipStream_t s)
         }
     } else {
         switch (kind) {
-        case NA_QST: k_nana16<NA_QST, false><<<grid, 256, 0, s>>>(a); break;
-        case NA_SH: k_nana16<NA_SH, false><<<grid, 256, 0, s>>>(a); break;
+        case NA_QST: k_nana16<NA_QST, false><<<grid, 512, 0, s>>>(a); break;
+        case NA_SH: k_nana16<NA_SH, false><<<grid, 512, 0, s>>>(a); break;
         default: return fail(MHX_E_INVALID, "unknown nonlinear-step analysis kind");
         }
     }
