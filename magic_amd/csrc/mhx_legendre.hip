@@ -541,6 +541,7 @@ int launch_ana_np(const AnaArgs &a, int tpw, unsigned grid, hipStream_t s)
     switch (tpw) {
     case 1: return launch_ana_t<1, NP>(a, grid, s);
     case 3: return launch_ana_t<3, NP>(a, grid, s);
+    case 4: return launch_ana_t<4, NP>(a, grid, s);
     default: return launch_ana_t<5, NP>(a, grid, s);
     }
 }
@@ -639,9 +640,13 @@ int launch_ana(const Plan *p, const AnaJob *jobs, int njob, const AnaBatch &b, h
     a.nq8 = (p->nh + 7) / 8;
     a.ng = (b.nlev + LEV_GROUP - 1) / LEV_GROUP;
     // tiles per wave: all of m = 0's tile pairs in one workgroup where five
-    // per wave hold them (120 accumulator registers), else groups of ten
+    // per wave hold them (120 accumulator registers) and the epilogue's areas,
+    // 288 (l_max + 2) bytes, leave room for a second workgroup on the CU; else
+    // groups of eight pairs, 74 KB (groups of ten, 92 KB and one workgroup per CU,
+    // took 5.37 / 6.92 / 4.57 ms per step at l_max = 341 x 40, 426 x 20, 511 x 12
+    // levels, eight 5.17 / 6.70 / 4.33, six 5.22 / 6.75 / 4.41)
     const int nt = (p->l_max + 2 + 31) / 32;
-    const int tpw = nt <= 2 ? 1 : (nt <= 6 ? 3 : 5);
+    const int tpw = nt <= 2 ? 1 : (nt <= 6 ? 3 : (p->l_max + 2 <= 284 ? 5 : 4));
     a.erows = std::min(64 * tpw, p->l_max + 2);
     a.gz = nt <= 2 * tpw ? 1 : (nt - 1 + 2 * tpw - 2) / (2 * tpw - 1);
     const unsigned grid = (unsigned)((p->n_m + 7) / 8 * 8 * njob * a.ng * a.gz);

@@ -17,11 +17,13 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-12
 
 # (l_max, n_theta, n_phi, minc): n_phi = 64 P for P = 1, 2, 3, 4, 5, 6, 8, 9, 10,
-# 12, 15, 16, 18, 20, 24, then other lengths
+# 12, 15, 16, 18, 20, 24, then other lengths, then one and two groups of degrees
+# in the analysis
 GRIDS = [(13, 20, 64, 1), (20, 36, 128, 1), (42, 64, 128, 1), (31, 52, 192, 1), (85, 128, 256, 1),
          (20, 68, 320, 1), (33, 84, 384, 2), (30, 60, 512, 1), (20, 44, 576, 1), (21, 36, 640, 1),
          (20, 100, 768, 4), (11, 20, 960, 1), (20, 32, 1024, 1), (12, 20, 1152, 1), (15, 28, 1280, 1),
-         (10, 20, 1536, 1), (15, 24, 48, 1), (31, 48, 96, 1), (26, 40, 80, 1), (33, 100, 400, 1)]
+         (10, 20, 1536, 1), (15, 24, 48, 1), (31, 48, 96, 1), (26, 40, 80, 1), (33, 100, 400, 1),
+         (282, 424, 64, 16), (283, 428, 64, 16), (345, 520, 64, 16)]
 
 
 @pytest.mark.parametrize("L,nt,nph,minc", GRIDS)
