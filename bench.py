@@ -28,8 +28,9 @@ PEAK = {"fp64": 78.6, "fp16": 2500.0}   # dense MFMA TFLOP/s
 PEAK_HBM_GBS = 8000.0
 
 # launch order of mhx_nl_step: (role, kind, Legendre weight, sources / comps)
-# Legendre weights are flops per (N_h * lm_max) per level (FMA = 2), charged
-# the FP64-equivalent count in both forms.
+# Legendre weights are flops per (N_h * lm_max) per level (FMA = 2) of the P and
+# dP sums, the FP64-equivalent count that the split form is charged; the FP64
+# form, which contracts P alone, is charged what it executes (P_ONLY).
 LAUNCHES = [
     ("syn_sg", "syn", 12, 1),
     ("syn_qst", "syn", 20, 3),   # u: w dw z
@@ -43,6 +44,7 @@ LAUNCHES = [
     ("ana_qst", "ana", 20, 3),
     ("ana_sh", "ana", 4, 1),
 ]
+P_ONLY = {20: 12, 12: 8, 4: 4}
 # kernels behind each role (prefix of the rocprofv3 kernel name)
 KERNELS = {
     "split16": {"syn_sg": "k_nsyn16p<0", "syn_qst": "k_nsyn16p<", "grid": "k_grid_tile",
@@ -53,8 +55,8 @@ KERNELS = {
     # l_max > 255: the chunked split Legendre kernels
     "split16_chunked": {"syn_sg": "k_nsyn16<0", "syn_qst": "k_nsyn16<", "grid": "k_nl_slots<float",
                         "ana_qst": "k_nana16<0", "ana_sh": "k_nana16<1"},
-    "fp64": {"syn_sg": "k_syn<2>", "syn_qst": "k_syn<3>", "grid": "k_nl_slots<double",
-             "ana_qst": "k_ana<2>", "ana_sh": "k_ana<0>"},
+    "fp64": {"syn_sg": "k_syn<3, 2", "syn_qst": "k_syn<3, 3", "grid": "k_nl_slots<double",
+             "ana_qst": "k_ana<5, 3", "ana_sh": "k_ana<5, 1"},
 }
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "nl_step_l255_traffic.json")
 
@@ -68,7 +70,7 @@ def algorithmic(kind, w, nsrc, nh, lm_max, n_theta, n_phi, n_m, nlev, word, twor
     """(flops, HBM bytes) of one launch.  Legendre: w N_h lm_max flops per
     level; bytes = coefficient arrays (16 B per lm) + Fourier comps (n_theta x
     n_m complex of 2 word bytes) + the tables read once (P and dP, or P alone
-    for the split kernels that fold dP onto P; tword bytes per entry: 8 FP64,
+    for the kernels that fold dP onto P; tword bytes per entry: 8 FP64,
     4 for the FP16 hi/lo pair; none for a synthesis that generates its tables
     by recurrence).  Grid stage: 18 Fourier comps in, 10 out, 3
     du/dr grids (n_theta x n_phi) out."""
@@ -327,8 +329,10 @@ def run_form(precision, L, nlev, steps, warmup, tin, rad, lcut, courant=False):
     total_flop = flop_ms = 0.0
     for (role, kind, w, nsrc), t in zip(LAUNCHES, lt):
         fl, by = algorithmic(kind, w, nsrc, nh, lm_max, nt, nph, n_m, nlev, word, tword,
-                             p_only=split and L <= 255,
+                             p_only=not split or L <= 255,
                              rec=precision == sht.PREC_SPLIT16_REC)
+        if not split and w:
+            fl *= P_ONLY[w] / w
         d = per_kernel.setdefault(role, {"ms": 0.0, "n": 0, "flop": 0.0, "bytes": 0.0})
         d["ms"] += t
         d["n"] += 1

@@ -13,7 +13,8 @@
 // theta-blocked, F[lev][comp][theta/8][m][theta%8], in FP64 (whole 128-byte
 // lines of the synthesis either way); the forward side theta-blocked,
 // F2[lev][comp][theta/TH][m][theta%TH] with TH = 8 in FP64 and 16 in FP32: the
-// analysis reads one 128-byte line per (comp, m, block); m < n_m, modes up to N/2 beyond n_m are zero (src/shtransforms.f90:224-232).
+// analysis reads one 128-byte line per (comp, m, block); m < n_m, modes up to
+// N/2 beyond n_m are zero (src/shtransforms.f90:224-232).
 #include "mhx_fftcore.h"
 
 namespace mhx {
@@ -140,7 +141,7 @@ __global__ void k_fft_rows(FFTArgs f, const T *__restrict__ g, size_t g_ld_lev, 
 // and forward FFTs of the 10 products.  Grid values live in registers (P
 // points per thread); only Fourier rows are read and written.
 //
-// Fin comps (layout [lev][comp][m][theta]):
+// Fin comps (layout: head of this file):
 //             vr vt vp | cvr cvt cvp | dvr dvt dvp | br bt bp | cbr cbt cbp |
 //             s dsdt dsdp
 // Fout (theta-blocked F2):

@@ -330,9 +330,10 @@ struct Plan {
     hipStream_t stream = nullptr;
     hipEvent_t ev_user = nullptr;  // orders the plan stream after a caller's stream
     hipEvent_t ev_done = nullptr;  // orders a caller's stream after the plan stream
-    // branch streams of the nonlinear step: its six synthesis launches and
-    // its four analysis launches are mutually independent and are dealt
-    // over nbranch streams (the plan stream and nbranch - 1 of these)
+    // branch streams of the split nonlinear step: its six synthesis launches
+    // and its four analysis launches are mutually independent and are dealt
+    // over nbranch streams (the plan stream and nbranch - 1 of these); the FP64
+    // step has one launch of each
     static constexpr int MAXBR = 4;
     int nbranch = 3;
     hipStream_t br[MAXBR - 1] = {};

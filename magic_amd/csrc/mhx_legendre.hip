@@ -99,6 +99,14 @@ template <int KIND> constexpr int syn_np() { return KIND == SYN_QST ? 3 : (KIND 
 // chunk is enough; the table fragments (16 bytes per lane: two quads) are
 // loaded one step of 2 NP TPW products ahead.  Loads are unconditional at
 // clamped addresses, the values masked at their use.
+//
+// Bound by the matrix pipe, which a step keeps busy 36 % of the time (two waves
+// per SIMD: 144 accumulator registers; the rest is the column forming and the
+// waits at the chunk's barrier).  QST at l_max = 255 x 97 levels: 0.65 ms with
+// five products, one launch per field and 8-byte table loads; 0.31 on P alone;
+// 0.28 (26 of 72.8 TFLOP/s) with the neighbour exchange by data-parallel moves.
+// Not faster: four fragments in flight, smaller theta groups; six waves of two
+// tiles per workgroup at three waves per SIMD spill (0.65 ms).
 template <int TPW, int KIND>
 __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, int mc, int lev0, int gz, double *sB)
 {
@@ -335,6 +343,11 @@ constexpr int AE_ROW = 18;
 // buffer; table fragments are loaded a step (8 theta) ahead.  Where the
 // order's tiles need more than one workgroup they overlap by one tile pair,
 // whose rows each workgroup's edge needs as neighbours.
+//
+// Bound by the matrix pipe and by the reads of F2, 3 n_theta n_m 16 bytes per
+// level.  QST at l_max = 255 x 97 levels: 0.72 ms with five sums, 16-byte gathers
+// one per (theta, m) and 16-byte stores; 0.325 (23 of 72.8 TFLOP/s) on wP alone
+// with whole lines read and 512-byte runs stored.
 template <int TPW, int KIND>
 __device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, int mc, int lev0, int gz, double *sB)
 {
@@ -546,8 +559,6 @@ int launch_ana_np(const AnaArgs &a, int tpw, unsigned grid, hipStream_t s)
     }
 }
 
-// theta tiles per wave and theta groups: 12 tiles per workgroup at most
-// (three per wave: 144 accumulator registers of the 256 at two waves per SIMD)
 template <int NP>
 int launch_syn_np(const SynArgs &a, int tpw, unsigned grid, hipStream_t s)
 {
@@ -596,6 +607,9 @@ int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, h
     a.n_theta = p->n_theta;
     a.nt16 = p->nt16;
     a.ng = (b.nlev + LEV_GROUP - 1) / LEV_GROUP;
+    // theta tiles: 12 per workgroup at most (three per wave: 144 accumulator
+    // registers of the 256 at two waves per SIMD), spread evenly over the groups
+    // and their waves
     a.gz = (p->nt16 + 11) / 12;
     const int tpw = (p->nt16 + 4 * a.gz - 1) / (4 * a.gz);
     const unsigned grid = (unsigned)((p->n_m + 7) / 8 * 8 * njob * a.ng * a.gz);

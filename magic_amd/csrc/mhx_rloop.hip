@@ -10,13 +10,13 @@
 //               curl B = torpol_to_curl(b, ddb, aj, dj)
 //   grid stage  get_nl (src/get_nl.f90:240-436) merged as
 //               transform_to_lm_space (:644-680), Courant maxima
-//               (src/courant.f90:209-275) - k_rl_grid, mhx_fft.hip
+//               (src/courant.f90:209-275) - k_rl_slots, k_rl_grid, mhx_fft.hip
 //   analysis    spat_to_qst of Adv, V s, V xi, V x B; scal_to_SH of the
 //               heating terms and of the phase-field terms (:682-707)
 //   lm space    nonlinear_lm_t (src/get_td.f90:133-589) - k_rl_td below
 //
-// One launch per stage for all levels; the synthesis and analysis launches
-// are the plan's FP64 Legendre kernels (mhx_legendre.hip).
+// One launch per stage for all levels and fields; the synthesis and analysis
+// launches are the plan's FP64 Legendre kernels (mhx_legendre.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -7,6 +7,10 @@
 // Bound by HBM: n_theta n_phi 8 + n_theta n_m 16 bytes per component and
 // level.  All components of a call run in one launch, 8 theta rows per
 // workgroup (whole 128-byte lines of the Fourier arrays' blocks of 8 rows).
+//
+// Three components at n_phi = 512, l_max = 170 x 65 levels: 229 us by block-wide
+// radix-4 passes and 16-byte gathers, one component per launch, 105 us so (341 MB:
+// 3.2 TB/s; a large copy reaches 4.8).
 #include "mhx_wavefft.h"
 
 namespace mhx {
