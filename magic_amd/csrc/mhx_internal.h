@@ -61,6 +61,12 @@ enum AnaKind { ANA_SH = 0, ANA_SPHTOR = 1, ANA_QST = 2 };
 constexpr int MAX_OUT = 3;
 constexpr int LEV_GROUP = 8;   // radial levels per MFMA column tile (re/im -> 16)
 constexpr int MAX_SYN_JOBS = 12;  // jobs of one synthesis launch
+// levels whose cut-offs can travel with a Legendre launch's arguments: a call that
+// hands them over on the host copies nothing to the device for them (a copy of a
+// few bytes takes about 4 us of the stream and of the caller: one level at l_max = 64
+// through module sht 138 -> 130 us, l_max = 106 x 41 levels 79 -> 76 us; 256 bytes of
+// arguments, which every launch of these kernels carries)
+constexpr int LEV_ARG = 128;
 
 struct SynJob {
     int kind;
@@ -75,8 +81,10 @@ struct SynBatch {
     int nlev;
     size_t src_ld;         // complex elements per level of the coefficients
     size_t fout_ld;        // complex elements per level of the Fourier arrays
-    const int *lcut;       // device, per level
-    const double *or2;     // device, per level (may be null)
+    const int *lcut;       // device, per level; null: the levels' in lcut_host
+    const double *or2;     // device, per level; null: or2_all for every level
+    const int *lcut_host;  // host, nlev <= LEV_ARG
+    double or2_all;
 };
 
 constexpr int MAX_ANA_JOBS = 8;   // jobs of one analysis launch
@@ -93,7 +101,8 @@ struct AnaBatch {
     int nlev;
     size_t fin_ld;         // complex elements per level of the Fourier arrays
     size_t out_ld;         // complex elements per level of the outputs
-    const int *lcut;       // device, per level
+    const int *lcut;       // device, per level; null: the levels' in lcut_host
+    const int *lcut_host;  // host, nlev <= LEV_ARG
 };
 
 // complex elements of one comp of the FP64 Fourier arrays (theta in blocks of 8)

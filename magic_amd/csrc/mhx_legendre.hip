@@ -44,7 +44,9 @@ struct SynArgs {
     const double *crec;
     const int *lstart;
     const double *osin2;
+    double or2_all;
     int l_max, minc, n_m, nh, n_theta, nt16;
+    short lc_arg[LEV_ARG];  // lcut null: the levels' cut-offs
 };
 
 struct AnaArgs {
@@ -58,7 +60,23 @@ struct AnaArgs {
     const int *lstart;
     int l_max, m_max, minc, n_m, nh, n_theta, nq8;
     int erows;             // rows of one epilogue area in LDS
+    short lc_arg[LEV_ARG];
 };
+
+template <class Args> __device__ __forceinline__ int lcut_of(const Args &a, int lev)
+{
+    return a.lcut ? a.lcut[lev] : (int)a.lc_arg[lev];
+}
+
+// a batch's cut-offs into the arguments
+template <class Args, class Batch> int set_lcut(Args &a, const Batch &b)
+{
+    a.lcut = b.lcut;
+    if (b.lcut) return MHX_OK;
+    if (!b.lcut_host || b.nlev > LEV_ARG) return fail(MHX_E_INVALID, "levels of a Legendre launch without cut-offs");
+    for (int i = 0; i < b.nlev; ++i) a.lc_arg[i] = (short)b.lcut_host[i];
+    return MHX_OK;
+}
 
 // v_mfma_f64_16x16x4f64 operands: A lane l holds A[l % 16][l / 16], B lane l
 // holds B[l / 16][l % 16]; D element j of lane l is D[l / 16 + 4 j][l % 16].
@@ -121,15 +139,15 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
 
     // the thread's (level, degree) of a chunk
     const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
-    const int lc = lev < a.nlev ? min(a.lcut[lev], L) : -1;
+    const int lc = lev < a.nlev ? min(lcut_of(a, lev), L) : -1;
     int lcm = -1;  // largest cut-off of the level group
 #pragma unroll
-    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, min(a.lcut[min(lev0 + i, a.nlev - 1)], L));
+    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, min(lcut_of(a, min(lev0 + i, a.nlev - 1)), L));
     const int nrow = max(lcm + 2 - m, 0);  // degrees m .. lcm + 1
     const int nch = (nrow + 31) >> 5;
     const int nquad[2] = {((nrow + 1) / 2 + 3) >> 2, (nrow / 2 + 3) >> 2};
     const int levc = min(lev, a.nlev - 1);
-    const double or2 = a.or2 ? a.or2[levc] : 0.0;
+    const double or2 = a.or2 ? a.or2[levc] : a.or2_all;
     const size_t src0 = ((size_t)levc * a.src_ld + (size_t)(l0 - m)) * 2;
 
     const double *const q0 = job.col[0].x0, *const s0 = job.col[CS].x0;
@@ -363,11 +381,11 @@ __device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, in
     const int l0 = a.lstart[mc];
 
     const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
-    const int lc = lev < a.nlev ? a.lcut[lev] : -1;
+    const int lc = lev < a.nlev ? lcut_of(a, lev) : -1;
     const bool lev_on = lev < a.nlev && m <= min(lc, a.m_max);
     int lcm = -1;
 #pragma unroll
-    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, a.lcut[min(lev0 + i, a.nlev - 1)]);
+    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, lcut_of(a, min(lev0 + i, a.nlev - 1)));
     const int nch = m <= min(lcm, a.m_max) ? (a.nh + 31) >> 5 : 0;
 
     // F2[lev][comp][theta/8][m][theta%8]
@@ -593,8 +611,9 @@ int launch_syn(const Plan *p, const SynJob *jobs, int njob, const SynBatch &b, h
     a.nlev = b.nlev;
     a.src_ld = b.src_ld;
     a.fout_ld = b.fout_ld;
-    a.lcut = b.lcut;
+    if (int rc = set_lcut(a, b)) return rc;
     a.or2 = b.or2;
+    a.or2_all = b.or2_all;
     a.tab = p->d_synx;
     a.off = p->d_synx_off;
     a.crec = p->d_crec64;
@@ -640,7 +659,7 @@ int launch_ana(const Plan *p, const AnaJob *jobs, int njob, const AnaBatch &b, h
     a.nlev = b.nlev;
     a.fin_ld = b.fin_ld;
     a.out_ld = b.out_ld;
-    a.lcut = b.lcut;
+    if (int rc = set_lcut(a, b)) return rc;
     a.tab = p->d_anax;
     a.off = p->d_anax_off;
     a.crec = p->d_crec64;

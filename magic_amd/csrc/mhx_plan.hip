@@ -126,12 +126,14 @@ int check_lcut(const Plan *p, int lcut)
     return MHX_OK;
 }
 
-int upload_lcut(Plan *p, const int *lcut, int nlev)
+// cut-offs of a batched call: past LEV_ARG levels on the device
+int stage_lcut(Plan *p, const int *lcut, int nlev)
 {
     for (int i = 0; i < nlev; ++i) {
         int rc = check_lcut(p, lcut[i]);
         if (rc) return rc;
     }
+    if (nlev <= LEV_ARG) return MHX_OK;
     MHX_HIP_CHECK(hipMemcpyAsync(p->d_lcut, lcut, sizeof(int) * nlev, hipMemcpyHostToDevice,
                                  p->stream));
     return MHX_OK;
@@ -166,10 +168,13 @@ SynJob syn_job(Plan *p, int kind, ColOp c0, ColOp c1 = ColOp(), ColOp c2 = ColOp
     return j;
 }
 
-// levels of the synthesis launches into ws_F (18 comps per level)
-SynBatch syn_batch(Plan *p, int nlev, size_t src_ld)
+// levels of the synthesis launches into ws_F (18 comps per level); a call's own
+// cut-offs travel with the launch where they fit
+SynBatch syn_batch(Plan *p, int nlev, size_t src_ld, const int *lcut_host = nullptr, double or2 = 0.0)
 {
-    return SynBatch{nlev, src_ld, 18 * f2_comp(p->n_m, p->n_theta), p->d_lcut, p->d_rad};
+    const bool arg = lcut_host && nlev <= LEV_ARG;
+    return SynBatch{nlev, src_ld, 18 * f2_comp(p->n_m, p->n_theta), arg ? nullptr : p->d_lcut,
+                    lcut_host ? nullptr : p->d_rad, lcut_host, or2};
 }
 
 // Fourier comps [0, ncomp) of ws_F -> grids at separate destinations (level
@@ -234,9 +239,10 @@ AnaJob ana_job(Plan *p, int kind, double *o0, double *o1 = nullptr, double *o2 =
 }
 
 // levels of the analysis launches from ws_F2 (10 comps per level)
-AnaBatch ana_batch(Plan *p, int nlev, size_t out_ld)
+AnaBatch ana_batch(Plan *p, int nlev, size_t out_ld, const int *lcut_host = nullptr)
 {
-    return AnaBatch{nlev, 10 * f2_comp(p->n_m, p->n_theta), out_ld, p->d_lcut};
+    const bool arg = lcut_host && nlev <= LEV_ARG;
+    return AnaBatch{nlev, 10 * f2_comp(p->n_m, p->n_theta), out_ld, arg ? nullptr : p->d_lcut, lcut_host};
 }
 
 // ---- per-call helpers: grids staged through ws_G, coefficients through ws_C
@@ -265,9 +271,7 @@ int synth_call(Plan *p, const SynJob &j, int ncomp, int lcut, double or2, double
 {
     int rc = check_lcut(p, lcut);
     if (rc) return rc;
-    MHX_HIP_CHECK(hipMemcpyAsync(p->d_lcut, &lcut, sizeof(int), hipMemcpyHostToDevice, p->stream));
-    MHX_HIP_CHECK(hipMemcpyAsync(p->d_rad, &or2, sizeof(double), hipMemcpyHostToDevice, p->stream));
-    if ((rc = launch_syn(p, &j, 1, syn_batch(p, 1, 0), p->stream))) return rc;
+    if ((rc = launch_syn(p, &j, 1, syn_batch(p, 1, 0, &lcut, or2), p->stream))) return rc;
     double *dst[3] = {p->ws_G, p->ws_G + (size_t)p->n_phi * p->n_theta,
                       p->ws_G + (size_t)2 * p->n_phi * p->n_theta};
     if ((rc = ifft_to(p, ncomp, 1, dst, 0))) return rc;
@@ -279,7 +283,6 @@ int analysis_call(Plan *p, int kind, int ngrid, const double *const *grids, cons
 {
     int rc = check_lcut(p, lcut);
     if (rc) return rc;
-    MHX_HIP_CHECK(hipMemcpyAsync(p->d_lcut, &lcut, sizeof(int), hipMemcpyHostToDevice, p->stream));
     size_t gsz = (size_t)p->n_phi * p->n_theta;
     const double *src[3];
     for (int c = 0; c < ngrid; ++c) {
@@ -295,7 +298,7 @@ int analysis_call(Plan *p, int kind, int ngrid, const double *const *grids, cons
     double *o[3] = {};
     for (int c = 0; c < nout; ++c) o[c] = p->ws_C + (size_t)(4 + c) * p->lm_max * 2;
     const AnaJob j = ana_job(p, kind, o[0], o[1], o[2]);
-    if ((rc = launch_ana(p, &j, 1, ana_batch(p, 1, 0), p->stream))) return rc;
+    if ((rc = launch_ana(p, &j, 1, ana_batch(p, 1, 0, &lcut), p->stream))) return rc;
     return finish_coefs(p, nout, out);
 }
 
@@ -880,10 +883,10 @@ int mhx_torpol_to_spat_batch(mhx_plan *h, int nlev, const double *W, const doubl
     if (!W || !dW || !Z || !vr || !vt || !vp || !lcut) return fail(MHX_E_INVALID, "null pointer");
     int rc;
     if ((rc = order_after(P, stream)) || (rc = ensure_ws(P, nlev)) ||
-        (rc = upload_lcut(P, lcut, nlev)))
+        (rc = stage_lcut(P, lcut, nlev)))
         return rc;
     SynJob j = syn_job(P, SYN_QST, op(W, G_LL), op(dW), op(Z));
-    if ((rc = launch_syn(P, &j, 1, syn_batch(P, nlev, ld_lm), P->stream))) return rc;
+    if ((rc = launch_syn(P, &j, 1, syn_batch(P, nlev, ld_lm, lcut), P->stream))) return rc;
     double *dst[3] = {vr, vt, vp};
     if ((rc = ifft_to(P, 3, nlev, dst, ld_grid))) return rc;
     MHX_HIP_CHECK(hipStreamSynchronize(P->stream));
@@ -900,13 +903,13 @@ int mhx_spat_to_qst_batch(mhx_plan *h, int nlev, const double *f, const double *
     if (!f || !g || !hh || !q || !s || !t || !lcut) return fail(MHX_E_INVALID, "null pointer");
     int rc;
     if ((rc = order_after(P, stream)) || (rc = ensure_ws(P, nlev)) ||
-        (rc = upload_lcut(P, lcut, nlev)))
+        (rc = stage_lcut(P, lcut, nlev)))
         return rc;
     const double *src[3] = {f, g, hh};
     bool os[3] = {false, true, true};
     if ((rc = fft_from(P, 3, nlev, src, ld_grid, os))) return rc;
     const AnaJob j = ana_job(P, ANA_QST, q, s, t);
-    if ((rc = launch_ana(P, &j, 1, ana_batch(P, nlev, ld_lm), P->stream))) return rc;
+    if ((rc = launch_ana(P, &j, 1, ana_batch(P, nlev, ld_lm, lcut), P->stream))) return rc;
     MHX_HIP_CHECK(hipStreamSynchronize(P->stream));
     return MHX_OK;
 }

@@ -538,7 +538,7 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
 
     // ---- synthesis ----
     enum { W = 0, DW, DDW, Z, DZ, S_, XI, PHI, BB, DB, DDB, AJ, DJ };
-    const SynBatch sb{nlev, ld_lm, nin * four / 2, B->lcut, d_or2};
+    const SynBatch sb{nlev, ld_lm, nin * four / 2, B->lcut, d_or2, nullptr, 0.0};
     SynJob jobs[MAX_SYN_JOBS];
     int njob = 0;
     auto add = [&](int kind, ColOp a, ColOp b, ColOp c, int c0, int c1, int c2) -> SynJob & {
@@ -660,7 +660,7 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
     if (ph->l_mag_nl) ana(ANA_QST, out_of[RO_VXBR], nl[NL_VXBR], nl[NL_VXBT], nl[NL_VXBP]);
     if (anel) ana(ANA_SH, out_of[RO_HEAT], nl[NL_HEAT]);
     if (phase) ana(ANA_SH, out_of[RO_PHI], dout[7]);
-    const AnaBatch ab{nlev, nout * four / 2, ld_lm, B->lcut};
+    const AnaBatch ab{nlev, nout * four / 2, ld_lm, B->lcut, nullptr};
     if ((rc = launch_ana(P, anas, nana, ab, s))) return rc;
 
     // ---- lm-space assembly ----

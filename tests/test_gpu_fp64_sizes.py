@@ -59,6 +59,32 @@ def test_levels_batched_match_oracle(L, nt, nph, minc):
     p.close()
 
 
+@pytest.mark.parametrize("nlev", [128, 129])
+def test_cutoffs_of_many_levels(nlev):
+    """Every level's own cut-off at the number of levels whose cut-offs travel
+    with the launch, and one past it."""
+    import torch
+    from oracle import oracle
+    L, nt, nph = 10, 16, 64
+    p = sht.Plan(L, nt, nph, max_levels=nlev)
+    o = oracle.Plan(L, nt, nph)
+    lcut = [1 + i % L for i in range(nlev)]
+    co = [np.stack([workload.coefficients(L, 6, f, i) for i in range(nlev)]) for f in range(3)]
+    dev = torch.device("cuda")
+    tin = [torch.from_numpy(x).to(dev) for x in co]
+    g = [torch.zeros((nlev, nph, nt), dtype=torch.float64, device=dev) for _ in range(3)]
+    p.torpol_to_spat_batch(*tin, lcut, *g)
+    c = [torch.zeros_like(tin[0]) for _ in range(3)]
+    p.spat_to_qst_batch(*g, lcut, *c)
+    for i in range(nlev):
+        want = o.torpol_to_spat(co[0][i], co[1][i], co[2][i], lcut[i])
+        back = o.spat_to_qst(*want, lcut[i])
+        for k in range(3):
+            assert rel_l2(g[k][i].cpu().numpy(), want[k]) < TOL, (i, k)
+            assert rel_l2(c[k][i].cpu().numpy(), back[k]) < TOL, (i, k)
+    p.close()
+
+
 # the grid stage's forms: slots of 2, 4, 8, 16, 32, 64 lanes (two of them with
 # several theta rows per workgroup, the last one partly filled), waves per
 # component (n_phi = 256, 512, 1024), block-wide passes (128, 160)
