@@ -284,7 +284,6 @@ struct Plan {
     double *d_cour_par = nullptr;
     unsigned long long *d_cour_max = nullptr;
     int cour_nlev = 0;
-    std::vector<double> h_cour;
     // per-level factors of mhx_get_td (or2, or4, epsc; l_R)
     double *d_ek = nullptr;  int ek_nlev = 0;  // energy sums: radial factors + outputs
     double *d_td_rad = nullptr;
@@ -360,6 +359,26 @@ struct Plan {
     double stage_ms[5] = {0, 0, 0, 0, 0};
     hipEvent_t ev[NEV] = {};
 };
+
+// the Courant inputs of the nonlinear step (host)
+struct CourIn {
+    double courfac, alffac;
+    const double *valri2, *valhi2;
+    double *vr2max, *vh2max;
+};
+
+// the lm-space assembly appended to the step (mhx_nl_step_td)
+struct TdIn {
+    double *const *out;  // dwdt dzdt dpdt dsdt dbdt djdt dVxBhLM
+    const double *epsc;  // per level
+    double CorFac;
+};
+
+// the step with the Courant maxima and, where ti is not null, the assembly; the
+// step and its copies are complete on return
+int nl_step_courant(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm, double *const *out,
+                    const double *or2, const double *or4, const double *orho1, double LFfac, const int *lcut,
+                    const CourIn &ci, const TdIn *ti, void *stream);
 
 // ------------------------------------------------------------- launchers
 int build_tables(Plan *p);

@@ -922,20 +922,6 @@ __global__ void k_zero_u64(unsigned long long *p, int n)
     if (i < n) p[i] = 0ull;
 }
 
-// the Courant inputs of mhx_nl_step_courant (host)
-struct CourIn {
-    double courfac, alffac;
-    const double *valri2, *valhi2;
-    double *vr2max, *vh2max;
-};
-
-// the lm-space assembly appended to the step (mhx_nl_step_td)
-struct TdIn {
-    double *const *out;  // dwdt dzdt dpdt dsdt dbdt djdt dVxBhLM
-    const double *epsc;  // per level
-    double CorFac;
-};
-
 static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm,
                         double *const *out, const double *or2, const double *or4,
                         const double *orho1, double LFfac, const int *lcut, double *grids,
@@ -1007,42 +993,6 @@ static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t l
         rad[nlev + i] = or4[i];
         rad[2 * nlev + i] = orho1[i];
     }
-    {
-        // per-level factors and lcut through a pinned buffer: the copies are
-        // then asynchronous (the previous call's copies completed before its
-        // end-of-call synchronisation, so the buffer is free to refill)
-        const size_t ntd = ti ? 3 * (size_t)nlev : 0;
-        const size_t need = (rad.size() + ntd) * sizeof(double) + (size_t)nlev * sizeof(int);
-        if (P->h_pin_bytes < need) {
-            if (P->h_pin) (void)hipHostFree(P->h_pin);
-            P->h_pin = nullptr;
-            P->h_pin_bytes = 0;
-            MHX_HIP_CHECK(hipHostMalloc(&P->h_pin, need, hipHostMallocDefault));
-            P->h_pin_bytes = need;
-        }
-        if (P->pin_pending) MHX_HIP_CHECK(hipEventSynchronize(P->ev_pin));  // previous copies read
-        P->pin_pending = false;
-        double *hr = static_cast<double *>(P->h_pin);
-        int *hl = reinterpret_cast<int *>(hr + rad.size() + ntd);
-        std::memcpy(hr, rad.data(), rad.size() * sizeof(double));
-        std::memcpy(hl, lcut, (size_t)nlev * sizeof(int));
-        MHX_HIP_CHECK(hipMemcpyAsync(P->d_rad, hr, rad.size() * sizeof(double), hipMemcpyHostToDevice,
-                                     P->stream));
-        if (ti) {
-            double *ht = hr + rad.size();
-            for (int i = 0; i < nlev; ++i) {
-                ht[i] = or2[i];
-                ht[nlev + i] = or4[i];
-                ht[2 * nlev + i] = ti->epsc[i];
-            }
-            MHX_HIP_CHECK(hipMemcpyAsync(P->d_td_rad, ht, ntd * sizeof(double), hipMemcpyHostToDevice,
-                                         P->stream));
-        }
-        MHX_HIP_CHECK(hipMemcpyAsync(P->d_lcut, hl, (size_t)nlev * sizeof(int), hipMemcpyHostToDevice,
-                                     P->stream));
-        MHX_HIP_CHECK(hipEventRecord(P->ev_pin, P->stream));
-        P->pin_pending = true;
-    }
     // Courant maxima: device parameters and per-level maxima (zeroed by a
     // kernel at the start of the step's launches)
     P->cour = CourArgs();
@@ -1057,18 +1007,55 @@ static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t l
             MHX_HIP_CHECK(hipMalloc(&P->d_cour_max, 2 * (size_t)nlev * sizeof(unsigned long long)));
             P->cour_nlev = nlev;
         }
-        MHX_HIP_CHECK(hipStreamSynchronize(P->stream));  // the previous upload has been read
-        P->h_cour.assign(2 + 2 * (size_t)nlev, 0.0);
-        P->h_cour[0] = ci->courfac * ci->courfac;
-        P->h_cour[1] = ci->alffac * ci->alffac;
-        for (int i = 0; i < nlev; ++i) {
-            P->h_cour[2 + i] = ci->valri2[i];
-            P->h_cour[2 + nlev + i] = ci->valhi2[i];
-        }
-        MHX_HIP_CHECK(hipMemcpyAsync(P->d_cour_par, P->h_cour.data(), P->h_cour.size() * sizeof(double),
-                                     hipMemcpyHostToDevice, P->stream));
         P->cour.par = P->d_cour_par;
         P->cour.max = P->d_cour_max;
+    }
+    {
+        // per-level factors and lcut through a pinned buffer: the copies are
+        // then asynchronous (the previous call's copies completed before its
+        // end-of-call synchronisation, so the buffer is free to refill)
+        const size_t ntd = ti ? 3 * (size_t)nlev : 0, ncour = ci ? 2 + 2 * (size_t)nlev : 0;
+        const size_t need = (rad.size() + ntd + ncour) * sizeof(double) + (size_t)nlev * sizeof(int);
+        if (P->pin_pending) MHX_HIP_CHECK(hipEventSynchronize(P->ev_pin));  // previous copies read
+        P->pin_pending = false;
+        if (P->h_pin_bytes < need) {
+            if (P->h_pin) (void)hipHostFree(P->h_pin);
+            P->h_pin = nullptr;
+            P->h_pin_bytes = 0;
+            MHX_HIP_CHECK(hipHostMalloc(&P->h_pin, need, hipHostMallocDefault));
+            P->h_pin_bytes = need;
+        }
+        double *hr = static_cast<double *>(P->h_pin);
+        double *hc = hr + rad.size() + ntd;
+        int *hl = reinterpret_cast<int *>(hc + ncour);
+        std::memcpy(hr, rad.data(), rad.size() * sizeof(double));
+        std::memcpy(hl, lcut, (size_t)nlev * sizeof(int));
+        MHX_HIP_CHECK(hipMemcpyAsync(P->d_rad, hr, rad.size() * sizeof(double), hipMemcpyHostToDevice,
+                                     P->stream));
+        if (ti) {
+            double *ht = hr + rad.size();
+            for (int i = 0; i < nlev; ++i) {
+                ht[i] = or2[i];
+                ht[nlev + i] = or4[i];
+                ht[2 * nlev + i] = ti->epsc[i];
+            }
+            MHX_HIP_CHECK(hipMemcpyAsync(P->d_td_rad, ht, ntd * sizeof(double), hipMemcpyHostToDevice,
+                                         P->stream));
+        }
+        if (ci) {
+            hc[0] = ci->courfac * ci->courfac;
+            hc[1] = ci->alffac * ci->alffac;
+            for (int i = 0; i < nlev; ++i) {
+                hc[2 + i] = ci->valri2[i];
+                hc[2 + nlev + i] = ci->valhi2[i];
+            }
+            MHX_HIP_CHECK(hipMemcpyAsync(P->d_cour_par, hc, ncour * sizeof(double), hipMemcpyHostToDevice,
+                                         P->stream));
+        }
+        MHX_HIP_CHECK(hipMemcpyAsync(P->d_lcut, hl, (size_t)nlev * sizeof(int), hipMemcpyHostToDevice,
+                                     P->stream));
+        MHX_HIP_CHECK(hipEventRecord(P->ev_pin, P->stream));
+        P->pin_pending = true;
     }
     hipStream_t s = P->stream;
     // a split-precision plan runs the Legendre stage in scaled FP16 x3 and
@@ -1484,14 +1471,12 @@ int mhx_get_td(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm, dou
     return MHX_OK;
 }
 
-int mhx_nl_step_courant(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm,
-                        double *const *out, const double *or2, const double *or4,
-                        const double *orho1, double LFfac, const int *lcut, double courfac,
-                        double alffac, const double *valri2, const double *valhi2,
-                        double *vr2max, double *vh2max, void *stream)
+extern "C++" int mhx::nl_step_courant(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm,
+                                      double *const *out, const double *or2, const double *or4,
+                                      const double *orho1, double LFfac, const int *lcut, const CourIn &ci,
+                                      const TdIn *ti, void *stream)
 {
-    CourIn ci{courfac, alffac, valri2, valhi2, vr2max, vh2max};
-    int rc = nl_step_impl(h, nlev, in, ld_lm, out, or2, or4, orho1, LFfac, lcut, nullptr, stream, &ci);
+    int rc = nl_step_impl(h, nlev, in, ld_lm, out, or2, or4, orho1, LFfac, lcut, nullptr, stream, &ci, ti);
     Plan *P = h ? &h->p : nullptr;
     if (rc) {
         if (P) P->cour = CourArgs();
@@ -1507,9 +1492,21 @@ int mhx_nl_step_courant(mhx_plan *h, int nlev, const double *const *in, size_t l
         double a, b;
         std::memcpy(&a, &mx[2 * i], sizeof(a));
         std::memcpy(&b, &mx[2 * i + 1], sizeof(b));
-        vr2max[i] = a;
-        vh2max[i] = b;
+        ci.vr2max[i] = a;
+        ci.vh2max[i] = b;
     }
+    return MHX_OK;
+}
+
+int mhx_nl_step_courant(mhx_plan *h, int nlev, const double *const *in, size_t ld_lm,
+                        double *const *out, const double *or2, const double *or4,
+                        const double *orho1, double LFfac, const int *lcut, double courfac,
+                        double alffac, const double *valri2, const double *valhi2,
+                        double *vr2max, double *vh2max, void *stream)
+{
+    const CourIn ci{courfac, alffac, valri2, valhi2, vr2max, vh2max};
+    const int rc = mhx::nl_step_courant(h, nlev, in, ld_lm, out, or2, or4, orho1, LFfac, lcut, ci, nullptr, stream);
+    if (rc) return rc;
     return finish_step(h, stream);
 }
 

@@ -270,10 +270,13 @@ void rl_free(Plan *p)
 // The switch sets the fused step covers (src/rIter.f90:483-707 with curl
 // advection, heat, the full MHD terms and no double curl, composition, phase
 // field, precession or centrifugal term): the fused step with its Courant
-// maxima (mhx_nl_step_courant), then its lm-space assembly (mhx_get_td), in
-// the plan's precision, as magic_amd/rloop.py composes them; returns when
-// done.  The Courant steps of src/courant.f90:271-272 (1e10 where a level has
-// no flow) from the maxima on the host.
+// maxima and its lm-space assembly as the step's last launch (the launches of
+// mhx_nl_step_courant and mhx_get_td), in the plan's precision, as
+// magic_amd/rloop.py composes them; returns when done.  With host arrays each field
+// is copied in once and the host waits once (w, dw, z copied for each of two calls
+// and a wait between them: 577 against 502 us per call at l_max = 64 x 31 levels
+// with fourfold symmetry).  The Courant steps of src/courant.f90:271-272 (1e10
+// where a level has no flow) from the maxima on the host.
 bool rl_fused_covers(const mhx_rloop_phys *ph)
 {
     return (ph->l_conv || ph->l_mag_kin) && ph->l_conv_nl && ph->l_adv_curl && !ph->l_anel &&
@@ -308,25 +311,30 @@ int rl_fused(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_ra
     // the step's du/dr grids are not among the loop's outputs
     const bool keep = P->dudr;
     P->dudr = false;
-    rc = mhx_nl_step_courant(h, nlev, fin, ld_lm, nl, rad->or2, rad->or4, rad->orho1, ph->LFfac, rad->l_R,
-                             ph->courfac, ph->alffac, vri.data(), vhi.data(), vr2.data(), vh2.data(), stream);
+    // with the lm-space assembly as its last launch
+    double *tout[7] = {out->dwdt, out->dzdt, out->dpdt, out->dsdt, out->dbdt, out->djdt, out->dVxBhLM};
+    const CourIn ci{ph->courfac, ph->alffac, vri.data(), vhi.data(), vr2.data(), vh2.data()};
+    const TdIn ti{tout, eps.data(), ph->l_corr ? ph->CorFac : 0.0};
+    rc = nl_step_courant(h, nlev, fin, ld_lm, nl, rad->or2, rad->or4, rad->orho1, ph->LFfac, rad->l_R, ci, &ti,
+                         stream);
     P->dudr = keep;
     if (rc) return rc;
-    // AdvrLM AdvtLM AdvpLM VStLM VxBrLM VxBtLM VxBpLM, then w dw z
-    const double *tin[10] = {nl[0], nl[1], nl[2], nl[4], nl[6], nl[7], nl[8], in->w, in->dw, in->z};
-    double *tout[7] = {out->dwdt, out->dzdt, out->dpdt, out->dsdt, out->dbdt, out->djdt, out->dVxBhLM};
-    if ((rc = mhx_get_td(h, nlev, tin, ld_lm, tout, rad->or2, rad->or4, eps.data(),
-                         ph->l_corr ? ph->CorFac : 0.0, rad->l_R, stream)))
-        return rc;
     for (int i = 0; i < nlev; ++i) {
         dt[i] = vr2[i] != 0.0 ? std::min(1e10, std::sqrt(rad->delxr2[i] / vr2[i])) : 1e10;
         dt[nlev + i] = vh2[i] != 0.0 ? std::min(1e10, std::sqrt(rad->delxh2[i] / vh2[i])) : 1e10;
     }
-    MHX_HIP_CHECK(hipMemcpyAsync(out->dtrkc, dt.data(), (size_t)nlev * sizeof(double), hipMemcpyDefault,
-                                 P->stream));
-    MHX_HIP_CHECK(hipMemcpyAsync(out->dthkc, dt.data() + nlev, (size_t)nlev * sizeof(double),
-                                 hipMemcpyDefault, P->stream));
-    MHX_HIP_CHECK(hipStreamSynchronize(P->stream));  // dt leaves scope
+    double *const steps[2] = {out->dtrkc, out->dthkc};
+    bool wait = false;
+    for (int k = 0; k < 2; ++k) {
+        const double *src = dt.data() + (size_t)k * nlev;
+        if (!is_device_ptr(steps[k])) {
+            std::memcpy(steps[k], src, (size_t)nlev * sizeof(double));
+            continue;
+        }
+        MHX_HIP_CHECK(hipMemcpyAsync(steps[k], src, (size_t)nlev * sizeof(double), hipMemcpyDefault, P->stream));
+        wait = true;
+    }
+    if (wait) MHX_HIP_CHECK(hipStreamSynchronize(P->stream));  // dt leaves scope
     return MHX_OK;
 }
 
