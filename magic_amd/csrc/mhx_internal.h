@@ -497,7 +497,8 @@ void rl_free(Plan *p);
 int launch_rl_grid(const Plan *p, const RlGridArgs &a, hipStream_t s);
 // FP64 tables (mhx_tables.hip): table_layout fills the offsets, build_tables
 // also allocates and computes the tables; ensure_fp64_tables builds them on
-// first use where plan creation left them out (recurrence-table plans);
+// first use where plan creation left them out (FP64 plans, for the axisymmetric
+// calls and the table export; recurrence-table plans);
 // split_rowscales_rec computes the split tables' row factors from the
 // recurrence, without FP64 tables
 int table_layout(Plan *p);
@@ -507,7 +508,7 @@ int ensure_fp64_tables(Plan *p);
 int ensure_p_tables(Plan *p);
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff);
 // the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768
-// the FP64 step's grid stage on wave FFTs (mhx_gridwave.hip): n_phi = 128 P, P <= 10
+// the FP64 step's grid stage on wave FFTs (mhx_gridwave.hip): n_phi = 256, 512, 1024
 bool grid_wave_supported(const Plan *p);
 int launch_grid_wave(const Plan *p, int nlev, const void *Fin, void *Fout, const double *rad,
                      double LFfac, void *dgrid, void *full_grids, hipStream_t s);

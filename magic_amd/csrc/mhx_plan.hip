@@ -472,10 +472,13 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         mhx_plan_destroy(h);
         return fail(MHX_E_HIP, "hipStreamCreate failed");
     }
-    // recurrence-table plans above l_max = 255 keep no FP64 tables: their
-    // split kernels generate the tables in-kernel, and the per-call entries
-    // that read FP64 tables build them on first use (ensure_fp64_tables)
-    if ((rc = (rec && l_max > 255) ? table_layout(p) : build_tables(p)) ||
+    // the P and dP tables are built here for the split tables made from them.
+    // FP64 plans, whose Legendre kernels have tables of their own, leave them to
+    // the first axisymmetric call (ensure_fp64_tables; a plan takes 2.17 ms so, 2.43
+    // with them, at l_max = 255), recurrence-table plans above l_max = 255, whose kernels
+    // generate theirs, to the first FP64 call
+    const bool later = precision == MHX_PREC_FP64 || (rec && l_max > 255);
+    if ((rc = later ? table_layout(p) : build_tables(p)) ||
         (precision == MHX_PREC_FP64 && (rc = ensure_p_tables(p))) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
         (rc = ensure_ws(p, std::max(1, max_levels)))) {
