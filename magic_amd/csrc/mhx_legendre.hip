@@ -68,6 +68,19 @@ template <class Args> __device__ __forceinline__ int lcut_of(const Args &a, int 
     return a.lcut ? a.lcut[lev] : (int)a.lc_arg[lev];
 }
 
+// the cut-off (at most l_max) of level lev0 + lv, -1 past the levels, and the
+// largest of the group of 8 levels from lev0: one load, lane i holding level i of
+// eight, where eight scalar loads held up the head of every workgroup
+template <class Args> __device__ __forceinline__ int group_cut(const Args &a, int lev0, int lv, int lane, int &lcm)
+{
+    const int v = min(lcut_of(a, min(lev0 + (lane & 7), a.nlev - 1)), a.l_max);
+    const int own = __shfl(v, lv);
+    int x = max(v, __shfl_xor(v, 1));
+    x = max(x, __shfl_xor(x, 2));
+    lcm = __builtin_amdgcn_readfirstlane(max(x, __shfl_xor(x, 4)));
+    return lev0 + lv < a.nlev ? own : -1;
+}
+
 // a batch's cut-offs into the arguments
 template <class Args, class Batch> int set_lcut(Args &a, const Batch &b)
 {
@@ -118,19 +131,24 @@ template <int KIND> constexpr int syn_np() { return KIND == SYN_QST ? 3 : (KIND 
 // loaded one step of 2 NP TPW products ahead.  Loads are unconditional at
 // clamped addresses, the values masked at their use.
 //
-// Bound by the matrix pipe, which a step keeps busy 36 % of the time (two waves
+// Bound by the matrix pipe, which a step keeps busy 40 % of the time (two waves
 // per SIMD: 144 accumulator registers; the rest is the column forming and the
 // waits at the chunk's barrier).  QST at l_max = 255 x 97 levels: 0.65 ms with
 // five products, one launch per field and 8-byte table loads; 0.31 on P alone;
-// 0.28 (26 of 72.8 TFLOP/s) with the neighbour exchange by data-parallel moves.
+// 0.28 with the neighbour exchange by data-parallel moves; 0.25 (29 of 72.8
+// TFLOP/s) with every load unconditional and the cut-offs in one load (same box:
+// 0.264 before).  Level groups in one workgroup one after the other, the next one's
+// first chunk formed during the last, gave 0.5 % of a step more and cost the small
+// ones (64 x 33 levels, fourfold symmetry) 5 %.
 // Not faster: four fragments in flight, smaller theta groups; six waves of two
 // tiles per workgroup at three waves per SIMD spill (0.65 ms).
 template <int TPW, int KIND>
-__device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, int mc, int lev0, int gz, double *sB)
+__device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &ajob, int mc, int lev0, int gz, double *sB)
 {
     constexpr int NP = syn_np<KIND>();
     constexpr bool QST = KIND == SYN_QST, TWO = KIND == SYN_QST || KIND == SYN_SPHTOR;
     constexpr int CS = QST ? 1 : 0, CT = QST ? 2 : 1;  // fields S (or x) and T
+    const SynJob job = ajob;  // in scalar registers, not read again at each use
     const int m = mc * a.minc, L = a.l_max;
     const double dm = (double)m;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -139,10 +157,8 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
 
     // the thread's (level, degree) of a chunk
     const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
-    const int lc = lev < a.nlev ? min(lcut_of(a, lev), L) : -1;
-    int lcm = -1;  // largest cut-off of the level group
-#pragma unroll
-    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, min(lcut_of(a, min(lev0 + i, a.nlev - 1)), L));
+    int lcm;  // largest cut-off of the level group
+    const int lc = group_cut(a, lev0, lv, lane, lcm);
     const int nrow = max(lcm + 2 - m, 0);  // degrees m .. lcm + 1
     const int nch = (nrow + 31) >> 5;
     const int nquad[2] = {((nrow + 1) / 2 + 3) >> 2, (nrow / 2 + 3) >> 2};
@@ -238,21 +254,22 @@ __device__ __forceinline__ void syn_body(const SynArgs &a, const SynJob &job, in
     const bool act = tt0 < a.nt16;
     double2 fa[2][TPW];
 
-    if (nch > 0) {
-        load(0);
-        if (nquad[0] > 0) load_A(fa[0], 0, 0);
-        build(0, 0);
-    }
+    // no load of the sources or tables stands under a branch, here on the cut-offs
+    // (whose own load it would wait for) or below on what is left to do: a load
+    // under a branch makes the next wait cover every load in flight
+    load(0);
+    load_A(fa[0], 0, 0);
+    if (nch > 0) build(0, 0);
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
         const int buf = c & 1;
-        if (c + 1 < nch) load(c + 1);
+        load(min(c + 1, nch - 1));
         if (act) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int par = k & 1, pair = k >> 1;
                 // the next step's fragments
-                if (nquad[1 - par] > 0) load_A(fa[1 - par], 2 * c + ((k + 1) >> 1), 1 - par);
+                load_A(fa[1 - par], 2 * c + ((k + 1) >> 1), 1 - par);
                 const int qq = 4 * c + 2 * pair;  // first quad of this step
                 if (qq < nquad[par]) {
                     double2 b[NP];
@@ -364,8 +381,8 @@ constexpr int AE_ROW = 18;
 //
 // Bound by the matrix pipe and by the reads of F2, 3 n_theta n_m 16 bytes per
 // level.  QST at l_max = 255 x 97 levels: 0.72 ms with five sums, 16-byte gathers
-// one per (theta, m) and 16-byte stores; 0.325 (23 of 72.8 TFLOP/s) on wP alone
-// with whole lines read and 512-byte runs stored.
+// one per (theta, m) and 16-byte stores; 0.32 on wP alone with whole lines read and
+// 512-byte runs stored; 0.28 (26 of 72.8 TFLOP/s) with every load unconditional.
 template <int TPW, int KIND>
 __device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, int mc, int lev0, int gz, double *sB)
 {
@@ -381,11 +398,9 @@ __device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, in
     const int l0 = a.lstart[mc];
 
     const int lv = tid >> 5, j = tid & 31, lev = lev0 + lv;
-    const int lc = lev < a.nlev ? lcut_of(a, lev) : -1;
+    int lcm;
+    const int lc = group_cut(a, lev0, lv, lane, lcm);
     const bool lev_on = lev < a.nlev && m <= min(lc, a.m_max);
-    int lcm = -1;
-#pragma unroll
-    for (int i = 0; i < LEV_GROUP; ++i) lcm = max(lcm, lcut_of(a, min(lev0 + i, a.nlev - 1)));
     const int nch = m <= min(lcm, a.m_max) ? (a.nh + 31) >> 5 : 0;
 
     // F2[lev][comp][theta/8][m][theta%8]
@@ -427,20 +442,17 @@ __device__ __forceinline__ void ana_body(const AnaArgs &a, const AnaJob &job, in
     auto load_A = [&](double2 *f, int p) {
         const double2 *t = tab + (size_t)min(p, npair - 1) * 64;
 #pragma unroll
-        for (int s = 0; s < TPW; ++s)
-            if (s < nmine) f[s] = t[(size_t)(t0 + 2 * s) * (npair * 64)];
+        for (int s = 0; s < TPW; ++s) f[s] = t[(size_t)min(t0 + 2 * s, nt - 1) * (npair * 64)];
     };
     double2 fa[2][TPW];
 
-    if (nch > 0) {
-        load(0);
-        load_A(fa[0], 0);
-        build(0, 0);
-    }
+    load(0);
+    load_A(fa[0], 0);
+    if (nch > 0) build(0, 0);
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
         const int buf = c & 1;
-        if (c + 1 < nch) load(c + 1);
+        load(min(c + 1, nch - 1));
         if (nmine > 0) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
