@@ -34,10 +34,36 @@ bool is_device_ptr(const void *ptr);
 #define MHX_HIP_CHECK(expr)                                                   \
     do {                                                                      \
         hipError_t e_ = (expr);                                               \
-        if (e_ != hipSuccess)                                                 \
+        if (e_ != hipSuccess) {                                               \
+            (void)hipGetLastError(); /* reported here, not by a later check */ \
             return ::mhx::fail(MHX_E_HIP, std::string(#expr) + ": " +         \
                                                hipGetErrorString(e_));        \
+        }                                                                     \
     } while (0)
+
+// device memory that is freed again unless it is given away: what a builder
+// fills before it hands the whole of it to the plan
+template <typename T> struct DevMem {
+    T *p = nullptr;
+    DevMem() = default;
+    DevMem(const DevMem &) = delete;
+    DevMem &operator=(const DevMem &) = delete;
+    ~DevMem()
+    {
+        if (p) (void)hipFree(p);
+    }
+    int alloc(size_t n)
+    {
+        MHX_HIP_CHECK(hipMalloc(&p, n * sizeof(T)));
+        return MHX_OK;
+    }
+    T *give()
+    {
+        T *q = p;
+        p = nullptr;
+        return q;
+    }
+};
 
 // ----------------------------------------------------- Legendre job model
 // A synthesis job runs one kind of Legendre contraction for a group of radial

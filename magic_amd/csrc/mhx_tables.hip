@@ -235,6 +235,9 @@ int table_layout(Plan *p)
     return MHX_OK;
 }
 
+// the tables are filled in memory of their own and given to the plan when all
+// of them are complete: a plan whose tables could not be built has none, and the
+// next call that needs them builds them
 int build_tables(Plan *p)
 {
     int rc;
@@ -242,24 +245,27 @@ int build_tables(Plan *p)
     if (p->d_syn_P) return MHX_OK;
     const int nh = p->nh;
     const size_t so = p->syn_size, ao = p->ana_size;
-    MHX_HIP_CHECK(hipMalloc(&p->d_syn_P, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMalloc(&p->d_syn_dP, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(p->d_syn_P, 0, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(p->d_syn_dP, 0, so * sizeof(double)));
     // the analysis pair feeds the split tables only (the FP64 kernels read
     // the P-only tables)
-    if (p->precision == MHX_PREC_SPLIT16 && !p->rec) {
-        MHX_HIP_CHECK(hipMalloc(&p->d_ana_wP, ao * sizeof(double)));
-        MHX_HIP_CHECK(hipMalloc(&p->d_ana_wdP, ao * sizeof(double)));
-        MHX_HIP_CHECK(hipMemset(p->d_ana_wP, 0, ao * sizeof(double)));
-        MHX_HIP_CHECK(hipMemset(p->d_ana_wdP, 0, ao * sizeof(double)));
+    const bool ana = p->precision == MHX_PREC_SPLIT16 && !p->rec;
+    DevMem<double> P, dP, wP, wdP;
+    if ((rc = P.alloc(so)) || (rc = dP.alloc(so)) || (ana && ((rc = wP.alloc(ao)) || (rc = wdP.alloc(ao))))) return rc;
+    MHX_HIP_CHECK(hipMemset(P.p, 0, so * sizeof(double)));
+    MHX_HIP_CHECK(hipMemset(dP.p, 0, so * sizeof(double)));
+    if (ana) {
+        MHX_HIP_CHECK(hipMemset(wP.p, 0, ao * sizeof(double)));
+        MHX_HIP_CHECK(hipMemset(wdP.p, 0, ao * sizeof(double)));
     }
     int n = p->n_m * nh;
     k_plm_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, nh, p->nt16, p->nq4,
                                            p->d_theta, p->d_gauss, p->d_syn_off, p->d_ana_off,
-                                           p->d_syn_P, p->d_syn_dP, p->d_ana_wP, p->d_ana_wdP);
+                                           P.p, dP.p, wP.p, wdP.p);
     MHX_HIP_CHECK(hipGetLastError());
     MHX_HIP_CHECK(hipDeviceSynchronize());
+    p->d_syn_P = P.give();
+    p->d_syn_dP = dP.give();
+    p->d_ana_wP = wP.give();
+    p->d_ana_wdP = wdP.give();
     return MHX_OK;
 }
 
@@ -282,27 +288,29 @@ int ensure_p_tables(Plan *p)
         }
         nc = (size_t)p->lstart[mc] + 2 * mc + nrow + 1;
     }
-    auto alloc = [&](auto *&dst, size_t n) -> int {
-        if (!dst) MHX_HIP_CHECK(hipMalloc(&dst, n * sizeof(*dst)));
-        return MHX_OK;
-    };
-    double *synx = nullptr;
+    DevMem<size_t> soff, aoff;
+    DevMem<double> crec, anax, synx;
     int rc;
-    if ((rc = alloc(p->d_synx_off, so.size())) || (rc = alloc(p->d_anax_off, ao.size())) ||
-        (rc = alloc(p->d_crec64, nc)) || (rc = alloc(p->d_anax, na)) || (rc = alloc(synx, ns)))
+    if ((rc = soff.alloc(so.size())) || (rc = aoff.alloc(ao.size())) || (rc = crec.alloc(nc)) || (rc = anax.alloc(na)) ||
+        (rc = synx.alloc(ns)))
         return rc;
-    p->d_synx = synx;
-    MHX_HIP_CHECK(hipMemcpy(p->d_synx_off, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
-    MHX_HIP_CHECK(hipMemcpy(p->d_anax_off, ao.data(), ao.size() * sizeof(size_t), hipMemcpyHostToDevice));
-    MHX_HIP_CHECK(hipMemset(p->d_synx, 0, ns * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(p->d_anax, 0, na * sizeof(double)));
+    MHX_HIP_CHECK(hipMemcpy(soff.p, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMemcpy(aoff.p, ao.data(), ao.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMemset(synx.p, 0, ns * sizeof(double)));
+    MHX_HIP_CHECK(hipMemset(anax.p, 0, na * sizeof(double)));
     const int n = p->n_m * p->nh;
-    k_p_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, p->nh, p->nt16, nq8, p->d_theta, p->d_gauss,
-                                         p->d_synx_off, p->d_anax_off, p->d_synx, p->d_anax);
+    k_p_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, p->nh, p->nt16, nq8, p->d_theta, p->d_gauss, soff.p,
+                                         aoff.p, synx.p, anax.p);
+    MHX_HIP_CHECK(hipGetLastError());
     k_crec64<<<dim3((unsigned)((p->l_max + 3 + 127) / 128), (unsigned)p->n_m), 128>>>(p->l_max, p->minc, p->d_lstart,
-                                                                                      p->d_crec64);
+                                                                                      crec.p);
     MHX_HIP_CHECK(hipGetLastError());
     MHX_HIP_CHECK(hipDeviceSynchronize());
+    p->d_synx = synx.give();
+    p->d_anax = anax.give();
+    p->d_synx_off = soff.give();
+    p->d_anax_off = aoff.give();
+    p->d_crec64 = crec.give();
     return MHX_OK;
 }
 

@@ -1,0 +1,131 @@
+"""Scenarios of the library's host code on the stand-in runtime of
+hip_stub.cpp, one per process: python stub_cases.py STUB LIBRARY SCENARIO."""
+import ctypes
+import sys
+
+FP64, SPLIT16, SPLIT16_REC = 0, 1, 2
+# a plan of each kind at its smallest: l_max, minc, n_theta, n_phi
+PLANS = {FP64: (16, 1, 32, 64), SPLIT16: (16, 1, 32, 64), SPLIT16_REC: (256, 16, 16, 64)}
+
+
+class Stub:
+    def __init__(self, stub, library):
+        self.s = ctypes.CDLL(stub, mode=ctypes.RTLD_GLOBAL)
+        self.s.stub_log.restype = ctypes.c_char_p
+        self.s.stub_fail.argtypes = [ctypes.c_long]
+        self.s.stub_bytes.restype = self.s.stub_live.restype = ctypes.c_size_t
+        self.L = ctypes.CDLL(library)
+        self.L.mhx_last_error.restype = ctypes.c_char_p
+
+    def log(self):
+        return [x.split() for x in self.s.stub_log().decode().splitlines()]
+
+    def plan(self, precision, levels=2, shape=None):
+        l_max, minc, nt, nph = shape or PLANS[precision]
+        h = ctypes.c_void_p()
+        rc = self.L.mhx_plan_create(l_max, 0, minc, nt, nph, precision, levels, ctypes.byref(h))
+        assert rc == 0, self.L.mhx_last_error()
+        lm = ctypes.c_int()
+        self.L.mhx_plan_info(h, ctypes.byref(lm), None, None, None)
+        return Handle(self, h, lm.value, l_max, nt, nph)
+
+
+class Handle:
+    def __init__(self, stub, h, lm_max, l_max, nt, nph):
+        self.stub, self.L, self.h = stub, stub.L, h
+        self.lm_max, self.l_max, self.nt, self.nph = lm_max, l_max, nt, nph
+
+    def close(self):
+        self.L.mhx_plan_destroy(self.h)
+
+    def host(self, n):
+        return (ctypes.c_double * int(n))()
+
+    def call(self, name):
+        """one call on host arrays; its return code"""
+        c, g, L = self.host(2 * self.lm_max), [self.host(self.nt * self.nph) for _ in range(3)], self.L
+        a = self.host(2 * (self.l_max + 1))
+        t = self.host(self.nt // 2 * self.lm_max)
+        z = ctypes.c_double
+        return {"axi_to_spat": lambda: L.mhx_axi_to_spat(self.h, a, g[0]),
+                "toraxi_to_spat": lambda: L.mhx_toraxi_to_spat(self.h, a, g[0], g[1], self.l_max),
+                "tables": lambda: L.mhx_plan_tables(self.h, None, None, t, t),
+                "scal_to_spat": lambda: L.mhx_scal_to_spat(self.h, c, g[0], self.l_max),
+                "spat_to_qst": lambda: L.mhx_spat_to_qst(self.h, *g, c, self.host(2 * self.lm_max),
+                                                         self.host(2 * self.lm_max), self.l_max)}[name]()
+
+    def step(self, nlev=2):
+        """one nonlinear step on device arrays"""
+        def dev():
+            p = ctypes.c_void_p()
+            assert self.stub.s.hipMalloc(ctypes.byref(p), ctypes.c_size_t(16 * nlev * self.lm_max)) == 0
+            return p.value
+        if not hasattr(self, "arrays"):
+            self.arrays = (ctypes.c_void_p * 11)(*[dev() for _ in range(11)]), \
+                (ctypes.c_void_p * 10)(*[dev() for _ in range(10)])
+        r = (ctypes.c_double * nlev)(*[1.0] * nlev)
+        lc = (ctypes.c_int * nlev)(*[self.l_max] * nlev)
+        return self.L.mhx_nl_step(self.h, nlev, self.arrays[0], ctypes.c_size_t(self.lm_max), self.arrays[1], r, r, r,
+                                  ctypes.c_double(1.0), lc, None)
+
+
+def launched(entry, kernel):
+    return entry[0] == "launch" and kernel in entry[1]
+
+
+def check_filled(log, kernel, ptrs):
+    """the tables at ptrs are allocated, and since then written whole by one
+    launch of `kernel` and waited for"""
+    for p in ptrs:
+        assert p != "0", "null table"
+        state = "none"
+        for e in log:
+            if e[0] == "malloc" and e[1] == p:
+                state = "raw"
+            elif e[0] == "free" and e[1] == p:
+                state = "none"
+            elif launched(e, kernel) and p in e[2:] and state != "none":
+                state = "written"
+            elif e[0] == "sync" and state == "written":
+                state = "filled"
+        assert state == "filled", (kernel, p, state)
+
+
+def failed_first_call(st, precision, name):
+    """Every way in which a call's resources can fail, then the same call
+    again: it reads whole tables or reports an error, and nothing is lost."""
+    p = st.plan(precision)
+    assert p.call(name) == 0
+    live = st.s.stub_live()
+    p.close()
+    failures = 0
+    for n in range(1, 200):
+        p = st.plan(precision)
+        st.s.stub_fail(n)
+        rc = p.call(name)
+        st.s.stub_fail(0)
+        if rc == 0:
+            p.close()
+            break
+        failures += 1
+        assert st.L.mhx_last_error()
+        assert p.call(name) == 0, st.L.mhx_last_error()
+        log = st.log()
+        if name == "scal_to_spat":
+            last = [e for e in log if launched(e, "k_p_tables")][-1]
+            check_filled(log, "k_p_tables", last[4:6])
+            check_filled(log, "k_crec64", [e for e in log if launched(e, "k_crec64")][-1][2:])
+        elif name != "tables":
+            check_filled(log, "k_plm_tables", [e for e in log if launched(e, "k_axi")][-1][2:])
+        else:
+            check_filled(log, "k_plm_tables", [e for e in log if launched(e, "k_plm_tables")][-1][2:4])
+        assert st.s.stub_live() == live, (n, st.s.stub_live(), live)
+        p.close()
+        assert st.s.stub_live() == 0
+        st.s.stub_clear()
+    assert failures > 0
+
+
+if __name__ == "__main__":
+    fn = globals()[sys.argv[3]]
+    fn(Stub(sys.argv[1], sys.argv[2]), *[int(x) if x.isdigit() else x for x in sys.argv[4:]])
