@@ -523,8 +523,7 @@ void rl_free(Plan *p);
 int launch_rl_grid(const Plan *p, const RlGridArgs &a, hipStream_t s);
 // FP64 tables (mhx_tables.hip): table_layout fills the offsets, build_tables
 // also allocates and computes the tables; ensure_fp64_tables builds them on
-// first use where plan creation left them out (FP64 plans, for the axisymmetric
-// calls and the table export; recurrence-table plans);
+// first use where plan creation left them out (recurrence-table plans);
 // split_rowscales_rec computes the split tables' row factors from the
 // recurrence, without FP64 tables
 int table_layout(Plan *p);

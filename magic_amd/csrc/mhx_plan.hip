@@ -472,13 +472,14 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         mhx_plan_destroy(h);
         return fail(MHX_E_HIP, "hipStreamCreate failed");
     }
-    // the P and dP tables are built here for the split tables made from them.
-    // FP64 plans, whose Legendre kernels have tables of their own, leave them to
-    // the first axisymmetric call (ensure_fp64_tables; a plan takes 2.17 ms so, 2.43
-    // with them, at l_max = 255), recurrence-table plans above l_max = 255, whose kernels
-    // generate theirs, to the first FP64 call
-    const bool later = precision == MHX_PREC_FP64 || (rec && l_max > 255);
-    if ((rc = later ? table_layout(p) : build_tables(p)) ||
+    // every table a plan stores is built here, so that no call allocates one or waits
+    // for the device: P and dP serve the axisymmetric calls, the table export and the
+    // split tables.  (Left to the first axisymmetric call, an FP64 plan at l_max = 255
+    // took 2.17 ms instead of 2.43, and that call waited for every stream of the device
+    // and failed beside a capture or where memory had run short by then.)
+    // Recurrence-table plans above l_max = 255, whose kernels generate theirs, build
+    // them at the first FP64 call.
+    if ((rc = (rec && l_max > 255) ? table_layout(p) : build_tables(p)) ||
         (precision == MHX_PREC_FP64 && (rc = ensure_p_tables(p))) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
         (rc = ensure_ws(p, std::max(1, max_levels)))) {

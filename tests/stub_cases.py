@@ -126,6 +126,19 @@ def failed_first_call(st, precision, name):
     assert failures > 0
 
 
+def tables_at_creation(st, precision):
+    """After its creation a plan's calls allocate, build and wait for nothing
+    beyond their own work."""
+    p = st.plan(precision)
+    for name in ("axi_to_spat", "toraxi_to_spat", "tables", "scal_to_spat", "spat_to_qst"):
+        st.s.stub_clear()
+        assert p.call(name) == 0, st.L.mhx_last_error()
+        log = st.log()
+        assert not [e for e in log if e[0] in ("malloc", "free", "memset", "sync")], (name, log)
+        assert not [e for e in log if launched(e, "tables")], (name, log)
+    p.close()
+
+
 if __name__ == "__main__":
     fn = globals()[sys.argv[3]]
     fn(Stub(sys.argv[1], sys.argv[2]), *[int(x) if x.isdigit() else x for x in sys.argv[4:]])

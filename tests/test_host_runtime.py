@@ -36,3 +36,10 @@ def test_tables_of_a_failed_first_call_are_built_by_the_next(scenario, precision
     """A plan whose tables could not be built by a first call builds them in
     the next: no kernel reads a missing or an unfilled one."""
     scenario("failed_first_call", precision, name)
+
+
+@pytest.mark.parametrize("precision", [FP64])
+def test_calls_after_plan_creation_build_no_tables(scenario, precision):
+    """Plans that store tables have all of them from their creation on: no first
+    call allocates, launches a table kernel or waits for the device."""
+    scenario("tables_at_creation", precision)
