@@ -528,8 +528,9 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &a, hipStream_t s);
 // recurrence, without FP64 tables
 int table_layout(Plan *p);
 int ensure_fp64_tables(Plan *p);
-// the P-only tables of the FP64 Legendre kernels, built at plan creation for
-// FP64 plans, else by the first call that runs those kernels
+// the P-only tables of the FP64 Legendre kernels, built at plan creation or, for
+// recurrence-table plans, by the first call that runs those kernels, together with
+// the P, dP pair: a later axisymmetric call or table export then builds nothing
 int ensure_p_tables(Plan *p);
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff);
 // the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768

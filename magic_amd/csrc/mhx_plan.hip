@@ -477,11 +477,14 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
     // split tables.  (Left to the first axisymmetric call, an FP64 plan at l_max = 255
     // took 2.17 ms instead of 2.43, and that call waited for every stream of the device
     // and failed beside a capture or where memory had run short by then.)
-    // Recurrence-table plans above l_max = 255, whose kernels generate theirs, build
-    // them at the first FP64 call.
-    if ((rc = (rec && l_max > 255) ? table_layout(p) : build_tables(p)) ||
-        (precision == MHX_PREC_FP64 && (rc = ensure_p_tables(p))) ||
+    // Recurrence-table plans (l_max > 255), whose kernels generate theirs, build them
+    // at the first FP64 call.
+    // The P-only tables of a split plan's FP64 calls take the room of the analysis
+    // pair, which only the split tables are made from (0.3 ms of 3.6 at l_max = 255,
+    // 0.9 of 12.5 at 511).
+    if ((rc = rec ? table_layout(p) : build_tables(p)) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
+        (!rec && (rc = ensure_p_tables(p))) ||
         (rc = ensure_ws(p, std::max(1, max_levels)))) {
         mhx_plan_destroy(h);
         return rc;

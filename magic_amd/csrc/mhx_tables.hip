@@ -272,8 +272,9 @@ int build_tables(Plan *p)
 int ensure_p_tables(Plan *p)
 {
     if (p->d_synx) return MHX_OK;
-    if (p->precision != MHX_PREC_FP64)
-        if (int rc = ensure_fp64_tables(p)) return rc;
+    // a recurrence-table plan's first FP64 call builds the P, dP pair too, which the
+    // axisymmetric calls and the export read
+    if (int rc = ensure_fp64_tables(p)) return rc;
     const int nq8 = (p->nh + 7) / 8;
     std::vector<size_t> so(2 * (size_t)p->n_m), ao(2 * (size_t)p->n_m);
     size_t ns = 0, na = 0, nc = 0;

@@ -139,6 +139,16 @@ def tables_at_creation(st, precision):
     p.close()
 
 
+def analysis_pair_freed(st):
+    """The 2 pi w P, dP pair that the split tables are made from is not held."""
+    p = st.plan(SPLIT16)
+    log = st.log()
+    pair = [e for e in log if launched(e, "k_plm_tables")][0][4:6]
+    for t in pair:
+        assert t != "0" and [e[0] for e in log if e[0] in ("malloc", "free") and e[1] == t][:2] == ["malloc", "free"], t
+    p.close()
+
+
 if __name__ == "__main__":
     fn = globals()[sys.argv[3]]
     fn(Stub(sys.argv[1], sys.argv[2]), *[int(x) if x.isdigit() else x for x in sys.argv[4:]])

@@ -38,8 +38,12 @@ def test_tables_of_a_failed_first_call_are_built_by_the_next(scenario, precision
     scenario("failed_first_call", precision, name)
 
 
-@pytest.mark.parametrize("precision", [FP64])
+@pytest.mark.parametrize("precision", [FP64, SPLIT16])
 def test_calls_after_plan_creation_build_no_tables(scenario, precision):
     """Plans that store tables have all of them from their creation on: no first
     call allocates, launches a table kernel or waits for the device."""
     scenario("tables_at_creation", precision)
+
+
+def test_split_plan_holds_no_tables_it_does_not_read(scenario):
+    scenario("analysis_pair_freed")
