@@ -1257,14 +1257,7 @@ int launch_slots(const Plan *p, const FFTArgs &f, int nlev, const void *Fin, voi
     static_assert(NPT * 6 * SlotFFT<A, B>::Q == 2 * M, "points do not tile the threads");
     constexpr int NR = SlotFFT<A, B>::NR;
     const size_t shm = ((size_t)2 * M + M / 8 + 1 + NR * (size_t)SlotFFT<A, B>::row_stride(padded_row<M, SlotFFT<A, B>::P>())) * 2 * sizeof(T);
-    // set once per kernel (the attribute persists), so that a call under
-    // graph capture makes no attribute call
-    static int shm_set = 0;
-    if (shm > 64 * 1024 && (int)shm > shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_nl_slots<T, A, B>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        shm_set = (int)shm;
-    }
+    if (int rc = allow_lds((const void *)k_nl_slots<T, A, B>, shm)) return rc;
     dim3 grid((unsigned)((p->n_theta + NR - 1) / NR * nlev));
     k_nl_slots<T, A, B><<<grid, nthr, shm, s>>>(f, static_cast<const T *>(Fin), static_cast<T *>(Fout),
                                                 p->n_m, p->n_theta, nlev, p->d_osin2, rad, LFfac,
@@ -1318,14 +1311,7 @@ int launch_fused_t(const Plan *p, int nlev, const void *Fin, void *Fout, const d
         k_nl_fused<T, 3><<<grid, nthr, shm, s>>>(f, fi, fo, p->n_m, p->n_theta, nlev, p->d_osin2,
                                                   rad, LFfac, dg, fg, p->cour);
     } else {
-        // set once per instance and raised only (the attribute persists), so
-        // that a call under graph capture makes no attribute call
-        static int shm_set = 0;
-        if (shm > 64 * 1024 && (int)shm > shm_set) {
-            MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_nl_fused<T, 1>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-            shm_set = (int)shm;
-        }
+        if (int rc = allow_lds((const void *)k_nl_fused<T, 1>, shm)) return rc;
         k_nl_fused<T, 1><<<grid, nthr, shm, s>>>(f, fi, fo, p->n_m, p->n_theta, nlev, p->d_osin2,
                                                   rad, LFfac, dg, fg, p->cour);
     }
@@ -1352,13 +1338,7 @@ int launch_rl_slots(const Plan *p, const FFTArgs &f, const RlGridArgs &a, hipStr
     typedef SlotFFT<A, B> FFT;
     constexpr int M = FFT::M, NR = FFT::NR;
     constexpr size_t shm = ((size_t)2 * M + M / 8 + 1 + NR * (size_t)FFT::row_stride(padded_row<M, FFT::P>())) * sizeof(double2);
-    // set once per kernel (the attribute persists)
-    static bool shm_set = false;
-    if (shm > 64 * 1024 && !shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_rl_slots<A, B>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        shm_set = true;
-    }
+    if (int rc = allow_lds((const void *)k_rl_slots<A, B>, shm)) return rc;
     dim3 grid((unsigned)((p->n_theta + NR - 1) / NR * a.nlev));
     k_rl_slots<A, B><<<grid, FFT::NTHR, shm, s>>>(f, a);
     MHX_HIP_CHECK(hipGetLastError());
@@ -1409,12 +1389,7 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &args, hipStream_t s)
     G = std::max(1, std::min(G, nrow));
     a.G = G;
     const size_t shm = fixed + (size_t)G * p->M * cs;
-    static int shm_set = 0;
-    if (shm > 64 * 1024 && (int)shm > shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_rl_grid,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        shm_set = (int)shm;
-    }
+    if (int rc = allow_lds((const void *)k_rl_grid, shm)) return rc;
     dim3 grid((unsigned)(p->n_theta * a.nlev));
     k_rl_grid<<<grid, 512, shm, s>>>(f, a);
     MHX_HIP_CHECK(hipGetLastError());

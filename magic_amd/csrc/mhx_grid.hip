@@ -448,12 +448,7 @@ template <int TR>
 int launch_tr(const Plan *p, const GtArgs &a, int nlev, hipStream_t s)
 {
     constexpr size_t lds = gt_lds<TR>();
-    static bool shm_set = false;
-    if (!shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_grid_tile<TR>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        shm_set = true;
-    }
+    if (int rc = allow_lds((const void *)k_grid_tile<TR>, lds)) return rc;
     dim3 grid((unsigned)(p->n_theta / TR * nlev));
     k_grid_tile<TR><<<grid, 64 * TR, lds, s>>>(a);
     MHX_HIP_CHECK(hipGetLastError());

@@ -243,14 +243,7 @@ template <int P> __global__ __launch_bounds__(64 * gw_waves<P>(), P <= 6 ? 3 : 2
 template <int P> int launch_p(const GwArgs &a, hipStream_t s)
 {
     constexpr size_t shm = gw_lds<P>();
-    // set once per kernel (the attribute persists), so that a call under
-    // graph capture makes no attribute call
-    static bool shm_set = false;
-    if (shm > 64 * 1024 && !shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_grid_wave<P>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)shm));
-        shm_set = true;
-    }
+    if (int rc = allow_lds((const void *)k_grid_wave<P>, shm)) return rc;
     k_grid_wave<P><<<dim3((unsigned)(a.n_theta * a.nlev)), 64 * gw_waves<P>(), shm, s>>>(a);
     MHX_HIP_CHECK(hipGetLastError());
     return MHX_OK;

@@ -41,6 +41,12 @@ bool is_device_ptr(const void *ptr);
         }                                                                     \
     } while (0)
 
+// the kernel may be launched with that many bytes of dynamic LDS on the current
+// device: its attribute, which a size past 64 KB needs, set once per device and
+// raised only (it persists), so that a call under graph capture makes no attribute
+// call; any thread
+int allow_lds(const void *kernel, size_t bytes);
+
 // device memory that is freed again unless it is given away: what a builder
 // fills before it hands the whole of it to the plan
 template <typename T> struct DevMem {

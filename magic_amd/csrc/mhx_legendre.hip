@@ -565,14 +565,7 @@ int launch_ana_t(const AnaArgs &a, unsigned grid, hipStream_t s)
     // the two B buffers, reused by the epilogue's areas (vt and vp; f alone
     // in a scalar launch)
     const size_t shm = std::max((size_t)2 * NP * AB_COL, (size_t)(NP > 1 ? 2 : 1) * a.erows * AE_ROW) * sizeof(double);
-    // set once per kernel and raised only, so that a call under graph capture
-    // makes no attribute call
-    static int shm_set = 0;
-    if (shm > 64 * 1024 && (int)shm > shm_set) {
-        MHX_HIP_CHECK(hipFuncSetAttribute((const void *)k_ana<TPW, NP>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)shm));
-        shm_set = (int)shm;
-    }
+    if (int rc = allow_lds((const void *)k_ana<TPW, NP>, shm)) return rc;
     k_ana<TPW, NP><<<grid, WG, shm, s>>>(a);
     MHX_HIP_CHECK(hipGetLastError());
     return MHX_OK;

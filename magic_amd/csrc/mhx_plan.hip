@@ -6,6 +6,9 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
+#include <utility>
 
 namespace mhx {
 
@@ -29,6 +32,22 @@ bool is_device_ptr(const void *ptr)
         return false;
     }
     return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
+}
+
+int allow_lds(const void *kernel, size_t bytes)
+{
+    if (bytes <= 64 * 1024) return MHX_OK;
+    static std::mutex mtx;
+    static std::map<std::pair<int, const void *>, size_t> set;
+    int dev = 0;
+    MHX_HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(mtx);
+    size_t &have = set[{dev, kernel}];
+    if (bytes > have) {
+        MHX_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+        have = bytes;
+    }
+    return MHX_OK;
 }
 
 namespace {

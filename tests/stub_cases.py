@@ -149,6 +149,29 @@ def analysis_pair_freed(st):
     p.close()
 
 
+def lds_per_device(st):
+    """A kernel's LDS attribute is set on every device that launches it, once
+    and for a larger size again."""
+    def attributes(device, shape, precision, name):
+        st.s.stub_device(device)
+        p = st.plan(precision, shape=shape)
+        st.s.stub_clear()
+        for _ in range(2):
+            assert (p.step() if name == "step" else p.call(name)) == 0, st.L.mhx_last_error()
+        got = [(int(e[1]), e[2], int(e[3])) for e in st.log() if e[0] == "attribute"]
+        p.close()
+        return got
+    # l_max, minc, n_theta, n_phi whose grid stage or epilogue takes over 64 KB
+    for shape, precision, name in (((20, 1, 32, 1536), FP64, "step"), ((20, 1, 32, 1024), FP64, "step"),
+                                   ((20, 1, 32, 3072), FP64, "step"), ((20, 1, 32, 768), SPLIT16, "step"),
+                                   ((20, 1, 32, 3072), SPLIT16, "step"), ((240, 16, 32, 64), FP64, "spat_to_qst"),
+                                   ((282, 16, 32, 64), FP64, "spat_to_qst")):
+        first = attributes(0, shape, precision, name)
+        assert first and all(d == 0 and n > 65536 for d, _, n in first), (shape, first)
+        assert attributes(0, shape, precision, name) == []
+        assert attributes(1, shape, precision, name) == [(1, k, n) for _, k, n in first], shape
+
+
 if __name__ == "__main__":
     fn = globals()[sys.argv[3]]
     fn(Stub(sys.argv[1], sys.argv[2]), *[int(x) if x.isdigit() else x for x in sys.argv[4:]])
