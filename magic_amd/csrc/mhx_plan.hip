@@ -530,6 +530,8 @@ int mhx_plan_destroy(mhx_plan *h)
     if (!h) return MHX_OK;
     Plan *p = &h->p;
     if (p->stream) (void)hipStreamSynchronize(p->stream);
+    // before the streams and events that the step was captured on
+    if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
     rl_free(p);
     free_dev(p->d_lstart);
     free_dev(p->d_syn_P);
@@ -600,7 +602,6 @@ int mhx_plan_destroy(mhx_plan *h)
         if (p->ev_join[i]) (void)hipEventDestroy(p->ev_join[i]);
         if (p->br[i]) (void)hipStreamDestroy(p->br[i]);
     }
-    if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
     if (p->h_pin) (void)hipHostFree(p->h_pin);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete h;

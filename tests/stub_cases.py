@@ -172,6 +172,19 @@ def lds_per_device(st):
         assert attributes(1, shape, precision, name) == [(1, k, n) for _, k, n in first], shape
 
 
+def graph_destroyed_first(st, precision):
+    """A plan's captured step goes before the streams and events it was
+    captured on and the memory it addresses."""
+    p = st.plan(precision)
+    for _ in range(3):
+        assert p.step() == 0, st.L.mhx_last_error()
+    st.s.stub_clear()
+    p.close()
+    log = [e for e in st.log() if e[0] in ("destroy", "free")]
+    assert log[0] == ["destroy", "exec"], log[:3]
+    assert log.count(["destroy", "exec"]) == 1
+
+
 if __name__ == "__main__":
     fn = globals()[sys.argv[3]]
     fn(Stub(sys.argv[1], sys.argv[2]), *[int(x) if x.isdigit() else x for x in sys.argv[4:]])

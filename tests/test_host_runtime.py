@@ -51,3 +51,8 @@ def test_split_plan_holds_no_tables_it_does_not_read(scenario):
 
 def test_lds_sizes_are_set_on_every_device(scenario):
     scenario("lds_per_device")
+
+
+@pytest.mark.parametrize("precision", [FP64, SPLIT16, SPLIT16_REC])
+def test_captured_step_is_destroyed_before_what_it_uses(scenario, precision):
+    scenario("graph_destroyed_first", precision)
