@@ -1021,10 +1021,10 @@ __global__ __launch_bounds__((SlotFFT<A, B>::NTHR), A <= 3 ? 3 : 2) void k_rl_sl
         }
     }
     if (out[RO_VSR] >= 0 || out[RO_VXIR] >= 0) {
-        // V s, V xi (src/get_nl.f90:320-331)
-        const double hs = ph.heat_nl ? 1.0 : 0.0;
-        RL_EACH(val[0][p] = hs * u[0][p] * s[p]; val[1][p] = hs * or2 * u[1][p] * s[p];
-                val[2][p] = hs * or2 * u[2][p] * s[p]; val[3][p] = u[0][p] * xi[p];
+        // V s, zero without nonlinear heat advection, and V xi (src/get_nl.f90:320-331)
+        const bool hs = ph.heat_nl;
+        RL_EACH(val[0][p] = hs ? u[0][p] * s[p] : 0.0; val[1][p] = hs ? or2 * u[1][p] * s[p] : 0.0;
+                val[2][p] = hs ? or2 * u[2][p] * s[p] : 0.0; val[3][p] = u[0][p] * xi[p];
                 val[4][p] = or2 * u[1][p] * xi[p]; val[5][p] = or2 * u[2][p] * xi[p])
         forward6(out[RO_VSR], out[RO_VST], out[RO_VSP], out[RO_VXIR], out[RO_VXIT], out[RO_VXIP]);
     }
