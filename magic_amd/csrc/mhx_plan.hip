@@ -494,13 +494,14 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
     // every table a plan stores is built here, so that no call allocates one or waits
     // for the device: P and dP serve the axisymmetric calls, the table export and the
     // split tables.  (Left to the first axisymmetric call, an FP64 plan at l_max = 255
-    // took 2.17 ms instead of 2.43, and that call waited for every stream of the device
+    // took 1.60 ms instead of 1.84, and that call waited for every stream of the device
     // and failed beside a capture or where memory had run short by then.)
     // Recurrence-table plans (l_max > 255), whose kernels generate theirs, build them
     // at the first FP64 call.
-    // The P-only tables of a split plan's FP64 calls take the room of the analysis
-    // pair, which only the split tables are made from (0.3 ms of 3.6 at l_max = 255,
-    // 0.9 of 12.5 at 511).
+    // The P-only tables of a split plan's FP64 calls take the memory of the analysis
+    // pair, which only the split tables are made from (a plan takes 3.6 ms so instead
+    // of 3.5 without them at l_max = 255, 13.1 instead of 12.4 at 511; freeing the pair
+    // and allocating again 5.2 and 14.5).
     if ((rc = rec ? table_layout(p) : build_tables(p)) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
         (!rec && (rc = ensure_p_tables(p))) ||
@@ -1186,8 +1187,7 @@ static int nl_step_impl(mhx_plan *h, int nlev, const double *const *in, size_t l
             if (dudr) jobs[nj++] = torpol(DW, DDW, DZ, 6);
             jobs[nj++] = torpol(B, DB, AJ, 9);
             jobs[nj++] = curl(B, DDB, AJ, DJ, 12);
-            // all in one launch (one by one when timed); the scalar's short
-            // blocks last
+            // all in one launch (one by one when timed)
             const SynBatch sb = syn_batch(P, nlev, ld_lm);
             if (P->timing) {
                 for (int v = 0; v < nj; ++v)

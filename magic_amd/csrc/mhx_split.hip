@@ -494,10 +494,6 @@ int build_split_tables(Plan *p)
     if ((rc = crec_table(p))) return rc;
     MHX_HIP_CHECK(hipGetLastError());
     MHX_HIP_CHECK(hipDeviceSynchronize());
-    // nothing else reads the analysis pair: its memory for the P-only FP64 tables
-    (void)hipFree(p->d_ana_wP);
-    (void)hipFree(p->d_ana_wdP);
-    p->d_ana_wP = p->d_ana_wdP = nullptr;
     return MHX_OK;
 }
 

@@ -18,7 +18,9 @@
 //     anax[anax_off[2mc+p] + ((kk/16) * nq8 + th/8) * 128 + ((kk%16) + 16*(th%4)) * 2 + (th/4)%2]
 #include "mhx_internal.h"
 
+#include <algorithm>
 #include <cmath>
+#include <utility>
 
 namespace mhx {
 
@@ -235,6 +237,32 @@ int table_layout(Plan *p)
     return MHX_OK;
 }
 
+// offsets and sizes of the P-only tables
+struct PLayout {
+    std::vector<size_t> so, ao;
+    size_t ns = 0, na = 0, nc = 0;
+};
+
+static PLayout p_layout(const Plan *p)
+{
+    PLayout y;
+    y.so.resize(2 * (size_t)p->n_m);
+    y.ao.resize(2 * (size_t)p->n_m);
+    const int nq8 = (p->nh + 7) / 8;
+    for (int mc = 0; mc < p->n_m; ++mc) {
+        const int nrow = p->l_max + 2 - mc * p->minc;
+        const int K[2] = {(nrow + 1) / 2, nrow / 2};
+        for (int par = 0; par < 2; ++par) {
+            y.so[2 * mc + par] = y.ns;
+            y.ns += (size_t)((K[par] + 7) / 8) * p->nt16 * 128;
+            y.ao[2 * mc + par] = y.na;
+            y.na += (size_t)((K[0] + 15) / 16) * nq8 * 128;  // pair tiles: both parities use K[0]'s count
+        }
+        y.nc = (size_t)p->lstart[mc] + 2 * mc + nrow + 1;
+    }
+    return y;
+}
+
 // the tables are filled in memory of their own and given to the plan when all
 // of them are complete: a plan whose tables could not be built has none, and the
 // next call that needs them builds them
@@ -245,11 +273,15 @@ int build_tables(Plan *p)
     if (p->d_syn_P) return MHX_OK;
     const int nh = p->nh;
     const size_t so = p->syn_size, ao = p->ana_size;
-    // the analysis pair feeds the split tables only (the FP64 kernels read
-    // the P-only tables)
+    // the analysis pair feeds the split tables only, and its memory then holds the
+    // P-only tables (ensure_p_tables)
     const bool ana = p->precision == MHX_PREC_SPLIT16 && !p->rec;
     DevMem<double> P, dP, wP, wdP;
-    if ((rc = P.alloc(so)) || (rc = dP.alloc(so)) || (ana && ((rc = wP.alloc(ao)) || (rc = wdP.alloc(ao))))) return rc;
+    if ((rc = P.alloc(so)) || (rc = dP.alloc(so))) return rc;
+    if (ana) {
+        const PLayout y = p_layout(p);
+        if ((rc = wP.alloc(std::max(ao, y.ns))) || (rc = wdP.alloc(std::max(ao, y.na)))) return rc;
+    }
     MHX_HIP_CHECK(hipMemset(P.p, 0, so * sizeof(double)));
     MHX_HIP_CHECK(hipMemset(dP.p, 0, so * sizeof(double)));
     if (ana) {
@@ -276,27 +308,20 @@ int ensure_p_tables(Plan *p)
     // axisymmetric calls and the export read
     if (int rc = ensure_fp64_tables(p)) return rc;
     const int nq8 = (p->nh + 7) / 8;
-    std::vector<size_t> so(2 * (size_t)p->n_m), ao(2 * (size_t)p->n_m);
-    size_t ns = 0, na = 0, nc = 0;
-    for (int mc = 0; mc < p->n_m; ++mc) {
-        const int nrow = p->l_max + 2 - mc * p->minc;
-        const int K[2] = {(nrow + 1) / 2, nrow / 2};
-        for (int par = 0; par < 2; ++par) {
-            so[2 * mc + par] = ns;
-            ns += (size_t)((K[par] + 7) / 8) * p->nt16 * 128;
-            ao[2 * mc + par] = na;
-            na += (size_t)((K[0] + 15) / 16) * nq8 * 128;  // pair tiles: both parities use K[0]'s count
-        }
-        nc = (size_t)p->lstart[mc] + 2 * mc + nrow + 1;
-    }
+    const PLayout y = p_layout(p);
+    const size_t ns = y.ns, na = y.na;
     DevMem<size_t> soff, aoff;
     DevMem<double> crec, anax, synx;
     int rc;
-    if ((rc = soff.alloc(so.size())) || (rc = aoff.alloc(ao.size())) || (rc = crec.alloc(nc)) || (rc = anax.alloc(na)) ||
-        (rc = synx.alloc(ns)))
+    if ((rc = soff.alloc(y.so.size())) || (rc = aoff.alloc(y.ao.size())) || (rc = crec.alloc(y.nc))) return rc;
+    if (p->d_ana_wP) {  // a split plan's analysis pair, read by its split tables' kernels only, gives its memory
+        std::swap(synx.p, p->d_ana_wP);
+        std::swap(anax.p, p->d_ana_wdP);
+    } else if ((rc = anax.alloc(na)) || (rc = synx.alloc(ns))) {
         return rc;
-    MHX_HIP_CHECK(hipMemcpy(soff.p, so.data(), so.size() * sizeof(size_t), hipMemcpyHostToDevice));
-    MHX_HIP_CHECK(hipMemcpy(aoff.p, ao.data(), ao.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    }
+    MHX_HIP_CHECK(hipMemcpy(soff.p, y.so.data(), y.so.size() * sizeof(size_t), hipMemcpyHostToDevice));
+    MHX_HIP_CHECK(hipMemcpy(aoff.p, y.ao.data(), y.ao.size() * sizeof(size_t), hipMemcpyHostToDevice));
     MHX_HIP_CHECK(hipMemset(synx.p, 0, ns * sizeof(double)));
     MHX_HIP_CHECK(hipMemset(anax.p, 0, na * sizeof(double)));
     const int n = p->n_m * p->nh;

@@ -139,14 +139,22 @@ def tables_at_creation(st, precision):
     p.close()
 
 
-def analysis_pair_freed(st):
-    """The 2 pi w P, dP pair that the split tables are made from is not held."""
-    p = st.plan(SPLIT16)
-    log = st.log()
-    pair = [e for e in log if launched(e, "k_plm_tables")][0][4:6]
-    for t in pair:
-        assert t != "0" and [e[0] for e in log if e[0] in ("malloc", "free") and e[1] == t][:2] == ["malloc", "free"], t
-    p.close()
+def analysis_pair_given_up(st):
+    """The 2 pi w P, dP pair, from which the split tables are made, is not held
+    besides the P-only tables: they take its memory, large enough for either."""
+    for shape in (PLANS[SPLIT16], (17, 1, 28, 64), (31, 3, 40, 96)):
+        st.s.stub_clear()
+        p = st.plan(SPLIT16, shape=shape)
+        log = st.log()
+        pair = [e for e in log if launched(e, "k_plm_tables")][0][4:6]
+        fill = [i for i, e in enumerate(log) if launched(e, "k_p_tables")][0]
+        assert pair == log[fill][4:6]
+        split = [i for i, e in enumerate(log) if launched(e, "k_split")]
+        assert ["sync"] in log[split[-1]:fill]  # the split tables' kernels have read it
+        for t in pair:
+            size = [int(e[2]) for e in log if e[0] == "malloc" and e[1] == t][-1]
+            assert [int(e[2]) for e in log[:fill] if e[0] == "memset" and e[1] == t][-1] <= size
+        p.close()
 
 
 def lds_per_device(st):

@@ -46,7 +46,7 @@ def test_calls_after_plan_creation_build_no_tables(scenario, precision):
 
 
 def test_split_plan_holds_no_tables_it_does_not_read(scenario):
-    scenario("analysis_pair_freed")
+    scenario("analysis_pair_given_up")
 
 
 def test_lds_sizes_are_set_on_every_device(scenario):
