@@ -1354,8 +1354,11 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &args, hipStream_t s)
     const int nrow = std::max(a.nin, a.nout);
     if (nrow <= 0 || nrow > 32) return fail(MHX_E_INVALID, "radial loop: bad component count");
     const size_t lds_max = 160 * 1024;
-    // rows of M = 3 4^A 2^B, M <= 768: wave-slot FFTs in rounds, where the rows
-    // of all components would fit the LDS too
+    // rows of M = 3 4^A 2^B, M <= 768: wave-slot FFTs in rounds of six rows.  The
+    // bound on all components' rows binds at M = 768 only (n_phi = 1536, more than ten
+    // components): those switch sets keep the generic form below, which refuses more
+    // than twelve.  A six-row launch would hold them, but has no measurement at that
+    // length
     {
         int A, B;
         if (slot_form(p, A, B) && p->M <= 768) {

@@ -1,5 +1,5 @@
-// Grid stage of the FP64 nonlinear step on wave FFTs (n_phi = 128 P): per
-// radial level and theta row, the 18 inverse FFTs of the synthesised
+// Grid stage of the FP64 nonlinear step on wave FFTs (n_phi = 128 P, P = 2, 4, 8,
+// one wave per P): per radial level and theta row, the 18 inverse FFTs of the synthesised
 // components, the grid products of src/get_nl.f90 (curl advection :262-273,
 // Lorentz force :242-258 merged as src/rIter.f90:650-656, V s :320-325, V x B
 // :376-388, u_h . grad_h s), the Courant maxima (src/courant.f90:209-275) and

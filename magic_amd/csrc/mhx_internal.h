@@ -539,11 +539,11 @@ int ensure_fp64_tables(Plan *p);
 // the P, dP pair: a later axisymmetric call or table export then builds nothing
 int ensure_p_tables(Plan *p);
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff);
-// the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768
 // the FP64 step's grid stage on wave FFTs (mhx_gridwave.hip): n_phi = 256, 512, 1024
 bool grid_wave_supported(const Plan *p);
 int launch_grid_wave(const Plan *p, int nlev, const void *Fin, void *Fout, const double *rad,
                      double LFfac, void *dgrid, void *full_grids, hipStream_t s);
+// the split step's grid stage on theta-row tiles (mhx_grid.hip): n_phi = 768
 bool grid_tile_supported(const Plan *p);
 int launch_grid_tile(const Plan *p, int nlev, const void *Fin, void *Fout, const double *rad,
                      double LFfac, void *dgrid, void *full_grids, hipStream_t s);

@@ -1,8 +1,9 @@
 // phi FFTs between Fourier rows and theta-fastest grids (Fortran f(n_theta,
 // n_phi)) for n_phi = 64 P: one wave per pair of neighbouring theta rows of
-// one component, both real rows in one complex FFT of length n_phi (their
-// field's own north and south rows, so equal in size), 16-byte accesses of the
-// pair throughout.  Other lengths run the generic kernels of mhx_fft.hip.
+// one component, both real rows in one complex FFT of length n_phi (a colatitude's
+// north and south row, whose sums and differences are what the Legendre side takes
+// and gives: each row's rounding error is relative to the larger of the two), 16-byte
+// accesses of the pair throughout.  Other lengths run the generic kernels of mhx_fft.hip.
 //
 // Bound by HBM: n_theta n_phi 8 + n_theta n_m 16 bytes per component and
 // level.  All components of a call run in one launch, 8 theta rows per

@@ -6,8 +6,9 @@
                                           <copy_mib> <out.json> <command...>
 
 `stats` prints a markdown table of the kernel-trace summary.  `traffic`
-averages FETCH_SIZE and WRITE_SIZE (KiB per dispatch) per kernel and scales
-each by what the same counter reads for the device-to-device copy of
+averages FETCH_SIZE and WRITE_SIZE (KiB per dispatch) per kernel and grid over
+the dispatches within 5 % of the largest (the radial loop runs the step's grid
+stage without the du/dr grids, which moves less) and scales each by what the same counter reads for the device-to-device copy of
 <copy_mib> MiB that `bench.py --calib-copy-mib` runs in the same process
 (the largest copy dispatch), giving HBM bytes per launch; it writes them as
 JSON (read by bench.py for `roofline.traffic`) and prints a markdown table.
@@ -47,6 +48,10 @@ def per_kernel(path, counter):
     return acc
 
 
+def largest(vs):
+    return [v for v in vs if v >= 0.95 * max(vs)]
+
+
 def traffic(fetch_csv, write_csv, copy_mib, out_json, cmd):
     f = per_kernel(fetch_csv, "FETCH_SIZE")
     w = per_kernel(write_csv, "WRITE_SIZE")
@@ -59,7 +64,7 @@ def traffic(fetch_csv, write_csv, copy_mib, out_json, cmd):
     for (k, g), vs in f.items():
         if "mhx" not in k and not k.startswith("k_"):
             continue
-        wv = w.get((k, g), [0.0])
+        vs, wv = largest(vs), largest(w.get((k, g), [0.0]))
         fk = sum(vs) / len(vs)
         wk = sum(wv) / len(wv)
         name = k + " grid=%d" % g
