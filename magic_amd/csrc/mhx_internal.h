@@ -285,7 +285,8 @@ struct Plan {
 
     // device
     int *d_lstart = nullptr;
-    double *d_syn_P = nullptr, *d_syn_dP = nullptr;   // FP64 MFMA-tiled
+    double *d_syn_P = nullptr, *d_syn_dP = nullptr;   // FP64 MFMA-tiled (split and recurrence plans)
+    double *d_ax_P = nullptr, *d_ax_dP = nullptr;     // their m = 0 part (FP64 plans)
     double *d_ana_wP = nullptr, *d_ana_wdP = nullptr;
     size_t *d_syn_off = nullptr, *d_ana_off = nullptr;
     // the FP64 Legendre kernels' tables: P_lm for l <= l_max + 1, two K quads
@@ -530,10 +531,12 @@ int launch_rl_grid(const Plan *p, const RlGridArgs &a, hipStream_t s);
 // FP64 tables (mhx_tables.hip): table_layout fills the offsets, build_tables
 // also allocates and computes the tables; ensure_fp64_tables builds them on
 // first use where plan creation left them out (recurrence-table plans);
+// copy_tables copies P, dP to the host, from tables of its own where the plan has none;
 // split_rowscales_rec computes the split tables' row factors from the
 // recurrence, without FP64 tables
 int table_layout(Plan *p);
 int ensure_fp64_tables(Plan *p);
+int copy_tables(const Plan *p, std::vector<double> &P, std::vector<double> &dP);
 // the P-only tables of the FP64 Legendre kernels, built at plan creation or, for
 // recurrence-table plans, by the first call that runs those kernels, together with
 // the P, dP pair: a later axisymmetric call or table export then builds nothing

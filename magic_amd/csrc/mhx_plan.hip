@@ -491,18 +491,15 @@ int mhx_plan_create(int l_max, int m_max, int minc, int n_theta, int n_phi, int 
         mhx_plan_destroy(h);
         return fail(MHX_E_HIP, "hipStreamCreate failed");
     }
-    // every table a plan stores is built here, so that no call allocates one or waits
-    // for the device: P and dP serve the axisymmetric calls, the table export and the
-    // split tables.  (Left to the first axisymmetric call, an FP64 plan at l_max = 255
-    // took 1.60 ms instead of 1.84, and that call waited for every stream of the device
-    // and failed beside a capture or where memory had run short by then.)
-    // Recurrence-table plans (l_max > 255), whose kernels generate theirs, build them
-    // at the first FP64 call.
-    // The P-only tables of a split plan's FP64 calls take the memory of the analysis
-    // pair, which only the split tables are made from (a plan takes 3.6 ms so instead
-    // of 3.5 without them at l_max = 255, 13.1 instead of 12.4 at 511; freeing the pair
-    // and allocating again 5.2 and 14.5).
-    if ((rc = rec ? table_layout(p) : build_tables(p)) ||
+    // every table that a plan's calls read is built here, so that none of them allocates
+    // one or waits for the device: in an FP64 plan the P-only tables and, for the
+    // axisymmetric calls, the m = 0 part of P, dP; in a split plan P, dP, the split tables
+    // made from them, and the P-only tables of its FP64 calls in the memory of the analysis
+    // pair, which only the split tables are made from (a plan takes 3.6 ms so instead of 3.5
+    // without them at l_max = 255, 13.1 instead of 12.4 at 511; freeing the pair and
+    // allocating again 5.2 and 14.5).  Recurrence-table plans (l_max > 255), whose kernels
+    // generate theirs, build the FP64 tables at the first FP64 call.
+    if ((rc = rec || precision == MHX_PREC_FP64 ? table_layout(p) : build_tables(p)) ||
         (precision == MHX_PREC_SPLIT16 && (rc = build_split_tables(p))) ||
         (!rec && (rc = ensure_p_tables(p))) ||
         (rc = ensure_ws(p, std::max(1, max_levels)))) {
@@ -537,6 +534,8 @@ int mhx_plan_destroy(mhx_plan *h)
     free_dev(p->d_lstart);
     free_dev(p->d_syn_P);
     free_dev(p->d_syn_dP);
+    free_dev(p->d_ax_P);
+    free_dev(p->d_ax_dP);
     free_dev(p->d_ana_wP);
     free_dev(p->d_ana_wdP);
     free_dev(p->d_syn_off);
@@ -627,11 +626,8 @@ int mhx_plan_tables(const mhx_plan *h, double *theta_ord, double *gauss, double 
     if (theta_ord) std::memcpy(theta_ord, p->theta_ord.data(), sizeof(double) * p->nh);
     if (gauss) std::memcpy(gauss, p->gauss.data(), sizeof(double) * p->nh);
     if (plm || dplm) {
-        int rc;
-        if ((rc = ensure_fp64_tables(const_cast<Plan *>(p)))) return rc;
-        std::vector<double> sP(p->syn_size), sdP(p->syn_size);
-        MHX_HIP_CHECK(hipMemcpy(sP.data(), p->d_syn_P, p->syn_size * 8, hipMemcpyDeviceToHost));
-        MHX_HIP_CHECK(hipMemcpy(sdP.data(), p->d_syn_dP, p->syn_size * 8, hipMemcpyDeviceToHost));
+        std::vector<double> sP, sdP;
+        if (int rc = copy_tables(p, sP, sdP)) return rc;
         for (int mc = 0; mc < p->n_m; ++mc) {
             int m = mc * p->minc;
             for (int l = m; l <= p->l_max; ++l) {

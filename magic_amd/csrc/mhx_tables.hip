@@ -263,36 +263,43 @@ static PLayout p_layout(const Plan *p)
     return y;
 }
 
-// the tables are filled in memory of their own and given to the plan when all
-// of them are complete: a plan whose tables could not be built has none, and the
-// next call that needs them builds them
+// the P, dP pair of all orders, or of the first n_m of them; with wP, wdP (allocated
+// by the caller) the analysis pair too
+static int plm_tables(const Plan *p, int n_m, DevMem<double> &P, DevMem<double> &dP, double *wP = nullptr,
+                      double *wdP = nullptr)
+{
+    const size_t so = n_m < p->n_m ? p->syn_off[2 * n_m] : p->syn_size, ao = p->ana_size;
+    int rc;
+    if ((rc = P.alloc(so)) || (rc = dP.alloc(so))) return rc;
+    MHX_HIP_CHECK(hipMemset(P.p, 0, so * sizeof(double)));
+    MHX_HIP_CHECK(hipMemset(dP.p, 0, so * sizeof(double)));
+    if (wP) {
+        MHX_HIP_CHECK(hipMemset(wP, 0, ao * sizeof(double)));
+        MHX_HIP_CHECK(hipMemset(wdP, 0, ao * sizeof(double)));
+    }
+    const int n = n_m * p->nh;
+    k_plm_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, n_m, p->nh, p->nt16, p->nq4, p->d_theta, p->d_gauss,
+                                           p->d_syn_off, p->d_ana_off, P.p, dP.p, wP, wdP);
+    MHX_HIP_CHECK(hipGetLastError());
+    return MHX_OK;
+}
+
+// tables are filled in memory of their own and given to the plan when all of them
+// are complete: a plan whose tables could not be built has none, and the next call
+// that needs them builds them
 int build_tables(Plan *p)
 {
     int rc;
     if ((rc = table_layout(p))) return rc;
     if (p->d_syn_P) return MHX_OK;
-    const int nh = p->nh;
-    const size_t so = p->syn_size, ao = p->ana_size;
-    // the analysis pair feeds the split tables only, and its memory then holds the
-    // P-only tables (ensure_p_tables)
-    const bool ana = p->precision == MHX_PREC_SPLIT16 && !p->rec;
     DevMem<double> P, dP, wP, wdP;
-    if ((rc = P.alloc(so)) || (rc = dP.alloc(so))) return rc;
-    if (ana) {
+    if (p->precision == MHX_PREC_SPLIT16 && !p->rec) {
+        // the analysis pair feeds the split tables only, and its memory then holds the
+        // P-only tables (ensure_p_tables)
         const PLayout y = p_layout(p);
-        if ((rc = wP.alloc(std::max(ao, y.ns))) || (rc = wdP.alloc(std::max(ao, y.na)))) return rc;
+        if ((rc = wP.alloc(std::max(p->ana_size, y.ns))) || (rc = wdP.alloc(std::max(p->ana_size, y.na)))) return rc;
     }
-    MHX_HIP_CHECK(hipMemset(P.p, 0, so * sizeof(double)));
-    MHX_HIP_CHECK(hipMemset(dP.p, 0, so * sizeof(double)));
-    if (ana) {
-        MHX_HIP_CHECK(hipMemset(wP.p, 0, ao * sizeof(double)));
-        MHX_HIP_CHECK(hipMemset(wdP.p, 0, ao * sizeof(double)));
-    }
-    int n = p->n_m * nh;
-    k_plm_tables<<<(n + 127) / 128, 128>>>(p->l_max, p->minc, p->n_m, nh, p->nt16, p->nq4,
-                                           p->d_theta, p->d_gauss, p->d_syn_off, p->d_ana_off,
-                                           P.p, dP.p, wP.p, wdP.p);
-    MHX_HIP_CHECK(hipGetLastError());
+    if ((rc = plm_tables(p, p->n_m, P, dP, wP.p, wdP.p))) return rc;
     MHX_HIP_CHECK(hipDeviceSynchronize());
     p->d_syn_P = P.give();
     p->d_syn_dP = dP.give();
@@ -306,13 +313,16 @@ int ensure_p_tables(Plan *p)
     if (p->d_synx) return MHX_OK;
     // a recurrence-table plan's first FP64 call builds the P, dP pair too, which the
     // axisymmetric calls and the export read
-    if (int rc = ensure_fp64_tables(p)) return rc;
+    if (p->rec)
+        if (int rc = ensure_fp64_tables(p)) return rc;
     const int nq8 = (p->nh + 7) / 8;
     const PLayout y = p_layout(p);
     const size_t ns = y.ns, na = y.na;
     DevMem<size_t> soff, aoff;
-    DevMem<double> crec, anax, synx;
+    DevMem<double> crec, anax, synx, axP, axdP;
     int rc;
+    // of the pair an FP64 plan keeps m = 0, for the axisymmetric calls
+    if (!p->d_syn_P && (rc = plm_tables(p, 1, axP, axdP))) return rc;
     if ((rc = soff.alloc(y.so.size())) || (rc = aoff.alloc(y.ao.size())) || (rc = crec.alloc(y.nc))) return rc;
     if (p->d_ana_wP) {  // a split plan's analysis pair, read by its split tables' kernels only, gives its memory
         std::swap(synx.p, p->d_ana_wP);
@@ -337,12 +347,30 @@ int ensure_p_tables(Plan *p)
     p->d_synx_off = soff.give();
     p->d_anax_off = aoff.give();
     p->d_crec64 = crec.give();
+    p->d_ax_P = axP.give();
+    p->d_ax_dP = axdP.give();
     return MHX_OK;
 }
 
 int ensure_fp64_tables(Plan *p)
 {
     return p->d_syn_P ? MHX_OK : build_tables(p);
+}
+
+int copy_tables(const Plan *p, std::vector<double> &P, std::vector<double> &dP)
+{
+    DevMem<double> tP, tdP;
+    const double *sP = p->d_syn_P, *sdP = p->d_syn_dP;
+    if (!sP) {
+        if (int rc = plm_tables(p, p->n_m, tP, tdP)) return rc;
+        sP = tP.p;
+        sdP = tdP.p;
+    }
+    P.resize(p->syn_size);
+    dP.resize(p->syn_size);
+    MHX_HIP_CHECK(hipMemcpy(P.data(), sP, p->syn_size * sizeof(double), hipMemcpyDeviceToHost));
+    MHX_HIP_CHECK(hipMemcpy(dP.data(), sdP, p->syn_size * sizeof(double), hipMemcpyDeviceToHost));
+    return MHX_OK;
 }
 
 int split_rowscales_rec(Plan *p, float *syn_rs, float *ana_rs, const size_t *ana_soff)

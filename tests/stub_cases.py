@@ -109,6 +109,7 @@ def failed_first_call(st, precision, name):
             break
         failures += 1
         assert st.L.mhx_last_error()
+        before = len(st.log())
         assert p.call(name) == 0, st.L.mhx_last_error()
         log = st.log()
         if name == "scal_to_spat":
@@ -117,8 +118,11 @@ def failed_first_call(st, precision, name):
             check_filled(log, "k_crec64", [e for e in log if launched(e, "k_crec64")][-1][2:])
         elif name != "tables":
             check_filled(log, "k_plm_tables", [e for e in log if launched(e, "k_axi")][-1][2:])
-        else:
-            check_filled(log, "k_plm_tables", [e for e in log if launched(e, "k_plm_tables")][-1][2:4])
+        else:  # the export's own tables: allocated, written, copied and freed in the call
+            again = log[before:]
+            pair = [e for e in again if launched(e, "k_plm_tables")][0][2:4]
+            assert [e[1] for e in again if e[0] == "malloc"] == pair
+            assert sorted(e[1] for e in again if e[0] == "free") == sorted(pair)
         assert st.s.stub_live() == live, (n, st.s.stub_live(), live)
         p.close()
         assert st.s.stub_live() == 0
@@ -128,14 +132,16 @@ def failed_first_call(st, precision, name):
 
 def tables_at_creation(st, precision):
     """After its creation a plan's calls allocate, build and wait for nothing
-    beyond their own work."""
+    beyond their own work, and the table export leaves nothing behind."""
     p = st.plan(precision)
-    for name in ("axi_to_spat", "toraxi_to_spat", "tables", "scal_to_spat", "spat_to_qst"):
+    for name in ("axi_to_spat", "toraxi_to_spat", "scal_to_spat", "spat_to_qst"):
         st.s.stub_clear()
         assert p.call(name) == 0, st.L.mhx_last_error()
         log = st.log()
         assert not [e for e in log if e[0] in ("malloc", "free", "memset", "sync")], (name, log)
         assert not [e for e in log if launched(e, "tables")], (name, log)
+    live = st.s.stub_live()
+    assert p.call("tables") == 0 and st.s.stub_live() == live
     p.close()
 
 
