@@ -131,8 +131,8 @@ template <int KIND> constexpr int syn_np() { return KIND == SYN_QST ? 3 : (KIND 
 // loaded one step of 2 NP TPW products ahead.  Loads are unconditional at
 // clamped addresses, the values masked at their use.
 //
-// No unit is saturated: at l_max = 255 x 97 levels the matrix pipe is busy 43 % of
-// the cycles, the vector-memory data path 71 % (55 % waiting for the cache), and at
+// No unit is saturated: at l_max = 255 x 97 levels the matrix pipe is busy 42 % of
+// the cycles, the vector-memory data path 68 % (53 % waiting for the cache), and at
 // two waves per SIMD (144 accumulator registers) a chunk's loads, column forming and
 // products add up more than they overlap (waves wait 39 % of their time, and 43 % on
 // instructions in flight).  QST at that size: 0.65 ms with
@@ -381,7 +381,7 @@ constexpr int AE_ROW = 18;
 // order's tiles need more than one workgroup they overlap by one tile pair,
 // whose rows each workgroup's edge needs as neighbours.
 //
-// No unit is saturated: matrix pipe 43 % busy, data path 74 % (47 % waiting for the
+// No unit is saturated: matrix pipe 41 % busy, data path 71 % (45 % waiting for the
 // cache, for 3 n_theta n_m 16 bytes of F2 per level and component and the table), as in
 // the synthesis.  QST at l_max = 255 x 97 levels: 0.72 ms with five sums, 16-byte gathers
 // one per (theta, m) and 16-byte stores; 0.32 on wP alone with whole lines read and
