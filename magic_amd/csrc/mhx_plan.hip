@@ -125,11 +125,13 @@ int ensure_ws(Plan *p, int nlev)
     if ((rc = ensure_buf(p->ws_C, p->ws_C_bytes, (size_t)p->lm_max * 16 * 8))) return rc;
     if (p->d_lcut_n < nlev) {
         free_dev(p->d_lcut);
+        p->d_lcut_n = 0;
         MHX_HIP_CHECK(hipMalloc(&p->d_lcut, sizeof(int) * nlev));
         p->d_lcut_n = nlev;
     }
     if (p->d_rad_n < nlev) {
         free_dev(p->d_rad);
+        p->d_rad_n = 0;
         MHX_HIP_CHECK(hipMalloc(&p->d_rad, sizeof(double) * 3 * nlev));
         p->d_rad_n = nlev;
     }

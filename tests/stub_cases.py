@@ -55,10 +55,10 @@ class Handle:
                                                          self.host(2 * self.lm_max), self.l_max)}[name]()
 
     def step(self, nlev=2):
-        """one nonlinear step on device arrays"""
+        """one nonlinear step on device arrays (of four levels)"""
         def dev():
             p = ctypes.c_void_p()
-            assert self.stub.s.hipMalloc(ctypes.byref(p), ctypes.c_size_t(16 * nlev * self.lm_max)) == 0
+            assert self.stub.s.hipMalloc(ctypes.byref(p), ctypes.c_size_t(16 * 4 * self.lm_max)) == 0
             return p.value
         if not hasattr(self, "arrays"):
             self.arrays = (ctypes.c_void_p * 11)(*[dev() for _ in range(11)]), \
@@ -197,6 +197,26 @@ def graph_destroyed_first(st, precision):
     log = [e for e in st.log() if e[0] in ("destroy", "free")]
     assert log[0] == ["destroy", "exec"], log[:3]
     assert log.count(["destroy", "exec"]) == 1
+
+
+def failed_growth(st, precision):
+    """A step on more levels than the plan has room for, each of its
+    allocations failing in turn, then a step on the plan's own number of
+    levels: it finds every workspace it needs."""
+    for n in range(1, 200):
+        p = st.plan(precision, levels=2)
+        assert p.step(2) == 0, st.L.mhx_last_error()
+        st.s.stub_fail(n)
+        rc = p.step(4)
+        st.s.stub_fail(0)
+        if rc == 0:
+            break
+        assert p.step(2) == 0, (n, st.L.mhx_last_error())
+        st.s.stub_clear()
+        assert p.step(2) == 0 and p.step(2) == 0
+        assert "0" not in [e[1] for e in st.log() if e[0] == "memcpy"], n
+        p.close()
+    assert n > 6
 
 
 if __name__ == "__main__":

@@ -56,3 +56,8 @@ def test_lds_sizes_are_set_on_every_device(scenario):
 @pytest.mark.parametrize("precision", [FP64, SPLIT16, SPLIT16_REC])
 def test_captured_step_is_destroyed_before_what_it_uses(scenario, precision):
     scenario("graph_destroyed_first", precision)
+
+
+@pytest.mark.parametrize("precision", [FP64, SPLIT16, SPLIT16_REC])
+def test_step_after_a_failed_growth_of_the_workspaces(scenario, precision):
+    scenario("failed_growth", precision)
