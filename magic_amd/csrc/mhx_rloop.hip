@@ -467,8 +467,10 @@ int mhx_rloop(mhx_plan *h, const mhx_rloop_phys *ph, int nlev, const mhx_rloop_r
                 t[RT_OSIN * P->n_theta + row] = 1.0 / sn;
             }
         }
-        MHX_HIP_CHECK(hipMalloc(&B->th, t.size() * sizeof(double)));
-        MHX_HIP_CHECK(hipMemcpy(B->th, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+        DevMem<double> th;
+        if ((rc = th.alloc(t.size()))) return rc;
+        MHX_HIP_CHECK(hipMemcpy(th.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+        B->th = th.give();
     }
     // per-level factors: grid stage, lm assembly, Courant lengths
     {

@@ -1,7 +1,13 @@
 """Scenarios of the library's host code on the stand-in runtime of
 hip_stub.cpp, one per process: python stub_cases.py STUB LIBRARY SCENARIO."""
 import ctypes
+import os
 import sys
+
+import numpy as np
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+from magic_amd import sht  # noqa: E402
 
 FP64, SPLIT16, SPLIT16_REC = 0, 1, 2
 # a plan of each kind at its smallest: l_max, minc, n_theta, n_phi
@@ -16,6 +22,7 @@ class Stub:
         self.s.stub_bytes.restype = self.s.stub_live.restype = ctypes.c_size_t
         self.L = ctypes.CDLL(library)
         self.L.mhx_last_error.restype = ctypes.c_char_p
+        sht._lib = self.L
 
     def log(self):
         return [x.split() for x in self.s.stub_log().decode().splitlines()]
@@ -217,6 +224,37 @@ def failed_growth(st, precision):
         assert "0" not in [e[1] for e in st.log() if e[0] == "memcpy"], n
         p.close()
     assert n > 6
+
+
+def failed_rloop(st):
+    """Every way in which a first radial loop's resources can fail, then the
+    same call again: the theta factors it reads were copied to the device."""
+    for n in range(1, 300):
+        p = st.plan(FP64)
+        p._L = p.L
+        z = np.zeros((2, p.lm_max), dtype=np.complex128)
+        rad = dict({k: np.ones(2) for k in sht.RLOOP_RAD}, **{k: np.full(2, 5, dtype=np.int32) for k in sht.RLOOP_RAD_INT})
+        fields = {k: z for k in sht.RLOOP_IN}
+        outs = {k: z.copy() for k in sht.RLOOP_OUT}
+        phys = dict(l_conv=1, l_conv_nl=1, l_heat=1, l_heat_nl=1, l_mag=1, l_mag_LF=1, l_mag_nl=1)
+
+        def call():
+            sht.rloop(p, phys, 2, rad, fields, outs, np.zeros(2), np.zeros(2))
+        st.s.stub_fail(n)
+        try:
+            call()
+            break
+        except sht.MhxError:
+            st.s.stub_fail(0)
+        call()
+        size = str(5 * p.nt * 8)
+        log = st.log()
+        made = [i for i, e in enumerate(log) if e[0] == "malloc" and e[2] == size][-1]
+        assert ["memcpy", log[made][1], size] in log[made:], n
+        p.close()
+        assert st.s.stub_live() == 0, n
+        st.s.stub_clear()
+    assert n > 10
 
 
 if __name__ == "__main__":

@@ -61,3 +61,7 @@ def test_captured_step_is_destroyed_before_what_it_uses(scenario, precision):
 @pytest.mark.parametrize("precision", [FP64, SPLIT16, SPLIT16_REC])
 def test_step_after_a_failed_growth_of_the_workspaces(scenario, precision):
     scenario("failed_growth", precision)
+
+
+def test_radial_loop_after_a_failed_first_call(scenario):
+    scenario("failed_rloop")
